@@ -1111,21 +1111,20 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   if ((rc = sync_alive())) return rc;
   if ((rc = refresh_degen())) return rc;
 
-  HIPCHK(hipMemsetAsync(c_->s_err_, 0, (size_t)nq * sizeof(double), c_->stream), "memset");
-  // query prep per range; each range's slots run to the next range (the last
-  // to nq_pad), the slots past its queries flagged as padding
+  // query prep, every range in one launch: a range's slots run to the next
+  // range (the last's to nq_pad), the slots past its queries flagged as
+  // padding.  It also clears the error report and the fail counts.
+  QueryPrepArgs pq{dQ, ldq, nq_pad, (uint32_t)d_, dp, fp8 ? sh8_.rho_bits : sh_.rho_bits,
+                   c_->s_qb_, (QParams*)c_->s_qp_, (double*)c_->s_err_, nq,
+                   (uint32_t*)c_->s_fail_, nr, {}, {}, {}, {}};
   for (int i = 0; i < nr; i++) {
-    const uint32_t send = i + 1 < nr ? R[i + 1].soff : nq_pad;
-    const double* q = dQ + (size_t)R[i].qoff * ldq;
-    unsigned char* qb = (unsigned char*)c_->s_qb_ + (size_t)R[i].soff * dp * qbytes;
-    QParams* qp = (QParams*)c_->s_qp_ + R[i].soff;
-    if (fp8)
-      HIPCHK(launch_query_prep8(q, ldq, R[i].n, send - R[i].soff, (uint32_t)d_, dp, R[i].metric,
-                                sh8_.rho_bits, (uint8_t*)qb, qp, c_->stream), "k_query_prep8");
-    else
-      HIPCHK(launch_query_prep(q, ldq, R[i].n, send - R[i].soff, (uint32_t)d_, dp, R[i].metric,
-                               sh_.rho_bits, (uint16_t*)qb, qp, c_->stream), "k_query_prep");
+    pq.metric[i] = R[i].metric;
+    pq.qoff[i] = R[i].qoff;
+    pq.soff[i] = R[i].soff;
+    pq.n[i] = R[i].n;
   }
+  HIPCHK(fp8 ? launch_query_prep8(pq, c_->stream) : launch_query_prep(pq, c_->stream),
+         "k_query_prep");
   // per-row ordering-key arrays: BF16 L2 (nx, pen), dot (xn, pen), cosine
   // (inv, pen); FP8 L2 (nx, sx), dot (xn, sx), cosine (sx/‖x‖, pen)
   auto w0_of = [&](int m) {
@@ -1204,7 +1203,6 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   const uint32_t Lmax = L;  // shortlist block stride per slot
   // FP64 rerank of every range's shortlist; fail counts and the first-pass
   // error report come back together after one wait
-  HIPCHK(hipMemsetAsync(c_->s_fail_, 0, nr * sizeof(uint32_t), c_->stream), "memset");
   auto rerank_args = [&](int ri) {
     const LowpRange& rg = R[ri];
     const uint32_t* fl = (uint32_t*)c_->s_fail_ + nr + rg.soff;

@@ -160,9 +160,26 @@ hipError_t launch_quantize_rows(const Shadow& sh, const double* X, size_t ldx, c
                                 const double* xn, const uint32_t* slots, uint32_t first,
                                 uint32_t n, uint32_t d, hipStream_t s);
 hipError_t launch_kill_rows(const Shadow& sh, const uint32_t* slots, uint32_t n, hipStream_t s);
-hipError_t launch_query_prep(const double* Q, size_t ldq, uint32_t nq, uint32_t nq_pad,
-                             uint32_t d, size_t dp, int metric, const uint32_t* rho_bits,
-                             uint16_t* Qb, QParams* qp, hipStream_t s);
+// One call's query slots: up to three metric ranges, range i holding the
+// queries at rows qoff[i].. of Q in slots soff[i].. (n[i] of them; the slots
+// up to the next range's first, and past the last range's up to nslots, are
+// padding).
+struct QueryPrepArgs {
+  const double* Q;
+  size_t ldq;
+  uint32_t nslots, d;
+  size_t dp;
+  const uint32_t* rho_bits;
+  void* Qb;              // [nslots][dp] BF16 or e4m3 query rows
+  QParams* qp;           // [nslots]
+  double* err;           // [nerr] first-pass error report, zeroed here
+  uint32_t nerr;
+  uint32_t* fail_count;  // [nr] zeroed here
+  int nr;
+  int metric[3];
+  uint32_t qoff[3], soff[3], n[3];
+};
+hipError_t launch_query_prep(const QueryPrepArgs& a, hipStream_t s);
 // minonly: one entry per list, its smallest key (the sample pre-pass).
 hipError_t launch_scan_bf16(const LowpScanArgs& a, int metric, uint32_t nslices, bool minonly,
                             hipStream_t s);
@@ -186,9 +203,7 @@ hipError_t launch_quantize_rows8(const Shadow8& sh, const double* X, size_t ldx,
 hipError_t launch_kill_rows8(const Shadow8& sh, const uint32_t* slots, uint32_t n, hipStream_t s);
 // Q8: e4m3 queries [nq_pad][dp]; QParams as for BF16 with P / scale carrying
 // the query's power-of-two scale (see svdb_fp8.hip).
-hipError_t launch_query_prep8(const double* Q, size_t ldq, uint32_t nq, uint32_t nq_pad,
-                              uint32_t d, size_t dp, int metric, const uint32_t* rho_bits,
-                              uint8_t* Q8, QParams* qp, hipStream_t s);
+hipError_t launch_query_prep8(const QueryPrepArgs& a, hipStream_t s);
 // a.Xb / a.Qb point at e4m3 bytes; a.w0 / a.w1: L2 (nx, sx), dot (xn, sx),
 // cosine (inv, pen).
 hipError_t launch_scan_fp8(const LowpScanArgs& a, int metric, uint32_t nslices, bool minonly,

@@ -5,6 +5,8 @@
 
 #include <math.h>
 
+#include "svdb_prep.h"
+
 namespace svdb {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -210,46 +212,59 @@ hipError_t launch_kill_rows(const Shadow& sh, const uint32_t* slots, uint32_t n,
 
 // ------------------------------------------------------------- query prep
 //
-// One thread per query: FP64 ‖q‖ (the canonical chain), bf16 q̂ scaled by
-// -2 (Euclidean) or -1 (dot, cosine) — exact power-of-two scalings — and
-// the per-query bound constants.
+// Per query: FP64 ‖q‖ (the canonical chain), bf16 q̂ scaled by -2 (Euclidean)
+// or -1 (dot, cosine) — exact power-of-two scalings — and the per-query
+// bound constants.  The error sums are in no fixed order; (1 + 2^-40) covers
+// their rounding in any order.
 
-__global__ void k_query_prep(const double* __restrict__ Q, size_t ldq, uint32_t nq,
-                             uint32_t nq_pad, uint32_t d, size_t dp, int metric,
-                             const uint32_t* __restrict__ rho_bits, uint16_t* __restrict__ Qb,
-                             QParams* __restrict__ qp) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nq_pad) return;
-  uint16_t* qb = Qb + (size_t)i * dp;
+__global__ __launch_bounds__(64 * kPrepWaves) void k_query_prep(QueryPrepArgs a) {
+  extern __shared__ __attribute__((aligned(16))) double prep_rows[];
+  const int lane = threadIdx.x & 63;
+  if (blockIdx.x == 0 && threadIdx.x < (uint32_t)a.nr) a.fail_count[threadIdx.x] = 0u;
+  const uint32_t i = blockIdx.x * kPrepWaves + (threadIdx.x >> 6);
+  if (i >= a.nslots) return;
+  int metric;
+  const PrepSlot ps = prep_slot(a, i, metric);
+  const uint32_t d = a.d, cols = (d + 15) & ~15u;
+  uint32_t* qb = reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(a.Qb) + (size_t)i * a.dp);
+  QParams* qp = a.qp;
+  if (lane == 0 && i < a.nerr) a.err[i] = 0.0;
   QParams p{};
   p.metric = metric;
-  if (i >= nq) {
-    for (size_t c = 0; c < dp; c++) qb[c] = 0;
+  if (ps.range < 0) {
+    for (uint32_t c = 2 * lane; c < a.dp; c += 128) qb[c >> 1] = 0;
     p.flags = 1;
-    qp[i] = p;
+    if (lane == 0) qp[i] = p;
     return;
   }
-  const double* q = Q + (size_t)i * ldq;
+  double* row = prep_rows + (threadIdx.x >> 6) * cols;
+  double maxabs;
+  bool finite;
+  const double nq2 = prep_stage(a.Q + (size_t)ps.row * a.ldq, d, cols, row, lane, maxabs, finite);
   const double sc = metric == kL2 ? -2.0 : -1.0;
-  double nq2 = 0.0, esq = 0.0, hsq = 0.0, maxabs = 0.0;
-  bool finite = true;
-  for (uint32_t c = 0; c < d; c++) {
-    double v = q[c];
-    nq2 = fma(v, v, nq2);
-    finite = finite && isfinite(v);
-    maxabs = fmax(maxabs, fabs(v));
-    uint16_t b = bf16_of(v);
-    double h = bf16_val(b);
-    double e = h - v;
-    esq = fma(e, e, esq);
-    hsq = fma(h, h, hsq);
-    qb[c] = bf16_of(h * sc);
+  double esq = 0.0, hsq = 0.0;
+  for (uint32_t c = 2 * lane; c < a.dp; c += 128) {
+    uint32_t word = 0;
+    if (c < cols) {
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const double v = row[c + j];
+        const double h = bf16_val(bf16_of(v));
+        const double e = h - v;
+        esq = fma(e, e, esq);
+        hsq = fma(h, h, hsq);
+        word |= (uint32_t)bf16_of(h * sc) << (16 * j);
+      }
+    }
+    if (c + 1 >= d) word &= c < d ? 0xFFFFu : 0u;  // (0 · sc is -0)
+    qb[c >> 1] = word;
   }
-  for (size_t c = d; c < dp; c++) qb[c] = 0;
+  esq = wave_sum(esq);
+  hsq = wave_sum(hsq);
+  const double rho = (double)__uint_as_float(*a.rho_bits);
   const double qn = sqrt(nq2);
   const double lim = 1152921504606846976.0;  // 2^60
   const double up = 1.0 + 0x1p-40;
-  const double rho = (double)__uint_as_float(*rho_bits);
   const double gam = (double)(d + 32) * 0x1p-24;
   const double qh = sqrt(hsq) * up, eq = sqrt(esq) * up;
   const double qh1 = qh * (1.0 + rho) * (1.0 + gam) * up;  // >= |s| / ‖x‖
@@ -275,15 +290,14 @@ __global__ void k_query_prep(const double* __restrict__ Q, size_t ldq, uint32_t 
     p.scale = 1.0 / qn;
     p.off = -(c + 0x1p-23 * qh1 * 1.01 + delta * lim) / qn - (double)(d + 16) * 0x1p-52;
   }
-  qp[i] = p;
+  if (lane == 0) qp[i] = p;
 }
 
-hipError_t launch_query_prep(const double* Q, size_t ldq, uint32_t nq, uint32_t nq_pad,
-                             uint32_t d, size_t dp, int metric, const uint32_t* rho_bits,
-                             uint16_t* Qb, QParams* qp, hipStream_t s) {
-  if (nq_pad == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_query_prep, dim3((nq_pad + 127) / 128), dim3(128), 0, s, Q, ldq, nq, nq_pad,
-                     d, dp, metric, rho_bits, Qb, qp);
+hipError_t launch_query_prep(const QueryPrepArgs& a, hipStream_t s) {
+  if (a.nslots == 0) return hipSuccess;
+  const uint32_t cols = (a.d + 15) & ~15u;
+  hipLaunchKernelGGL(k_query_prep, dim3((a.nslots + kPrepWaves - 1) / kPrepWaves),
+                     dim3(64 * kPrepWaves), kPrepWaves * cols * sizeof(double), s, a);
   return hipGetLastError();
 }
 

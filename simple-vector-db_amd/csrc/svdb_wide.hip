@@ -23,6 +23,8 @@
 
 #include <math.h>
 
+#include "svdb_prep.h"
+
 namespace svdb {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -184,54 +186,60 @@ hipError_t launch_kill_rows8(const Shadow8& sh, const uint32_t* slots, uint32_t 
 
 // ------------------------------------------------------------- query prep
 //
-// One thread per query: FP64 ‖q‖ (the canonical chain), e4m3 codes of
-// q·sc / sq (sc = -2 Euclidean, -1 dot and cosine; sq its power-of-two
-// scale), ĥ = sq·e4m3(q·sc/sq)/sc, and the bound constants of the BF16 form
-// with ‖ĥ‖, ‖ĥ - q‖ and this shadow's ρ; then the power-of-two rescaling of
-// P and scale.
+// Per query: FP64 ‖q‖ (the canonical chain), e4m3 codes of q·sc / sq (sc = -2
+// Euclidean, -1 dot and cosine; sq its power-of-two scale),
+// ĥ = sq·e4m3(q·sc/sq)/sc, and the bound constants of the BF16 form with ‖ĥ‖,
+// ‖ĥ - q‖ and this shadow's ρ; then the power-of-two rescaling of P and scale.
 
-__global__ void k_query_prep8(const double* __restrict__ Q, size_t ldq, uint32_t nq,
-                              uint32_t nq_pad, uint32_t d, size_t dp, int metric,
-                              const uint32_t* __restrict__ rho_bits, uint8_t* __restrict__ Q8,
-                              QParams* __restrict__ qp) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nq_pad) return;
-  uint8_t* q8 = Q8 + (size_t)i * dp;
+__global__ __launch_bounds__(64 * kPrepWaves) void k_query_prep8(QueryPrepArgs a) {
+  extern __shared__ __attribute__((aligned(16))) double prep_rows8[];
+  const int lane = threadIdx.x & 63;
+  if (blockIdx.x == 0 && threadIdx.x < (uint32_t)a.nr) a.fail_count[threadIdx.x] = 0u;
+  const uint32_t i = blockIdx.x * kPrepWaves + (threadIdx.x >> 6);
+  if (i >= a.nslots) return;
+  int metric;
+  const PrepSlot ps = prep_slot(a, i, metric);
+  const uint32_t d = a.d, cols = (d + 15) & ~15u;
+  uint32_t* q8 = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(a.Qb) + (size_t)i * a.dp);
+  QParams* qp = a.qp;
+  if (lane == 0 && i < a.nerr) a.err[i] = 0.0;
   QParams p{};
   p.metric = metric;
-  if (i >= nq) {
-    for (size_t c = 0; c < dp; c++) q8[c] = 0;
+  if (ps.range < 0) {
+    for (uint32_t c = 4 * lane; c < a.dp; c += 256) q8[c >> 2] = 0;
     p.flags = 1;
-    qp[i] = p;
+    if (lane == 0) qp[i] = p;
     return;
   }
-  const double* q = Q + (size_t)i * ldq;
+  double* row = prep_rows8 + (threadIdx.x >> 6) * cols;
+  double maxabs;
+  bool finite;
+  const double nq2 = prep_stage(a.Q + (size_t)ps.row * a.ldq, d, cols, row, lane, maxabs, finite);
   const double sc = metric == kL2 ? -2.0 : -1.0;
-  double nq2 = 0.0, maxabs = 0.0;
-  bool finite = true;
-  for (uint32_t c = 0; c < d; c++) {
-    const double v = q[c];
-    nq2 = fma(v, v, nq2);
-    finite = finite && isfinite(v);
-    maxabs = fmax(maxabs, fabs(v));
-  }
   const double qn = sqrt(nq2);
   const double lim = 1152921504606846976.0;  // 2^60
   p.flags = (!finite || !(qn >= 1.0 / lim) || !(qn <= lim) || !(maxabs <= lim)) ? 1 : 0;
   const double sq = p.flags ? 1.0 : pow2_scale(maxabs * fabs(sc));
   double esq = 0.0, hsq = 0.0;
-  for (uint32_t c = 0; c < d; c++) {
-    const double v = q[c];
-    const uint32_t code = p.flags ? 0u : e4m3_of(v * sc / sq);
-    q8[c] = (uint8_t)code;
-    const double h = e4m3_val(code) * sq / sc;
-    const double e = h - v;
-    esq = fma(e, e, esq);
-    hsq = fma(h, h, hsq);
+  for (uint32_t c = 4 * lane; c < a.dp; c += 256) {
+    uint32_t word = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if (c + j >= d) continue;
+      const double v = row[c + j];
+      const uint32_t code = p.flags ? 0u : e4m3_of(v * sc / sq);
+      word |= code << (8 * j);
+      const double h = e4m3_val(code) * sq / sc;
+      const double e = h - v;
+      esq = fma(e, e, esq);
+      hsq = fma(h, h, hsq);
+    }
+    q8[c >> 2] = word;
   }
-  for (size_t c = d; c < dp; c++) q8[c] = 0;
+  esq = wave_sum(esq);
+  hsq = wave_sum(hsq);
   const double up = 1.0 + 0x1p-40;
-  const double rho = (double)__uint_as_float(*rho_bits);
+  const double rho = (double)__uint_as_float(*a.rho_bits);
   const double gam = (double)(d + 32) * 0x1p-24;
   const double qh = sqrt(hsq) * up, eq = sqrt(esq) * up;
   const double qh1 = qh * (1.0 + rho) * (1.0 + gam) * up;  // >= |s| / ‖x‖
@@ -257,15 +265,14 @@ __global__ void k_query_prep8(const double* __restrict__ Q, size_t ldq, uint32_t
     p.scale = 1.0 / qn;
     p.off = -(c + 0x1p-23 * qh1 * 1.01 + delta * lim) / qn - (double)(d + 16) * 0x1p-52;
   }
-  qp[i] = p;
+  if (lane == 0) qp[i] = p;
 }
 
-hipError_t launch_query_prep8(const double* Q, size_t ldq, uint32_t nq, uint32_t nq_pad,
-                              uint32_t d, size_t dp, int metric, const uint32_t* rho_bits,
-                              uint8_t* Q8, QParams* qp, hipStream_t s) {
-  if (nq_pad == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_query_prep8, dim3((nq_pad + 127) / 128), dim3(128), 0, s, Q, ldq, nq,
-                     nq_pad, d, dp, metric, rho_bits, Q8, qp);
+hipError_t launch_query_prep8(const QueryPrepArgs& a, hipStream_t s) {
+  if (a.nslots == 0) return hipSuccess;
+  const uint32_t cols = (a.d + 15) & ~15u;
+  hipLaunchKernelGGL(k_query_prep8, dim3((a.nslots + kPrepWaves - 1) / kPrepWaves),
+                     dim3(64 * kPrepWaves), kPrepWaves * cols * sizeof(double), s, a);
   return hipGetLastError();
 }
 
