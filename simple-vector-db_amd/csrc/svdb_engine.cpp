@@ -1361,7 +1361,7 @@ int Engine::lowp_complete() {
       // read again
       rw.carry = 1;
       prof_begin(SVDB_K_RERANK);
-      HIPCHK(launch_rerank(rw, metric, c_->stream), "k_rerank (widened)");
+      HIPCHK(launch_rerank_wide(rw, metric, c_->stream), "k_rerank (widened)");
       prof_end(SVDB_K_RERANK);
       HIPCHK(hipMemcpyAsync(c_->h_fail_, out_count, sizeof(uint32_t), hipMemcpyDeviceToHost, c_->stream),
              "copy");

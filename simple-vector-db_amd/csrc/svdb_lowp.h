@@ -210,7 +210,8 @@ hipError_t launch_scan_fp8(const LowpScanArgs& a, int metric, uint32_t nslices, 
                            hipStream_t s);
 
 hipError_t launch_shortlist(const ShortlistArgs& a, hipStream_t s);
-hipError_t launch_rerank(const RerankArgs& a, int metric, hipStream_t s);
+// a widening retry: a.carry set, a.L up to kMaxShort
+hipError_t launch_rerank_wide(const RerankArgs& a, int metric, hipStream_t s);
 // n ranges in as few launches as possible (kMaxLaunchRanges per launch; for
 // the shortlist, consecutive ranges that take the same kernel)
 constexpr int kMaxLaunchRanges = 4;

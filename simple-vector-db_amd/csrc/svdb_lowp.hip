@@ -633,13 +633,44 @@ hipError_t launch_kth_key(const float* key, uint32_t nq, uint32_t n, uint32_t L,
 
 // ------------------------------------------------------------- FP64 rerank
 //
-// One wavefront per query.  Lanes take the candidates 64 at a time (the
-// shortlist, then the degenerate rows) and compute their canonical FP64 rank
-// key with the sequential fma chain; the k best by (key, slot) are
-// selected; the query is certified when its k-th key is below the bound
-// beta*scale + off (minus the FP64 rounding slack of that expression and,
-// for Euclidean, of the keys themselves).  Certified queries get their ids
-// and scores written; the others are listed for the FP64 scan.
+// The candidates' canonical FP64 rank keys (the sequential fma chains), the k
+// best by (key, slot), and the certificate: the k-th key is below the bound
+// beta*scale + off (minus the FP64 rounding slack of that expression and, for
+// Euclidean, of the keys themselves).  Certified queries get their ids and
+// scores written; the others are listed for the next stage.  The first stage
+// (shortlists up to 256, k_rerank) takes a block per query, the widening
+// retries (1,024 and 4,096, k_rerank1) a wavefront.
+
+// FP64 lower bound on the ordering value of a row whose first-pass key is at
+// least `bo` (the rounding slack of the key's conversion included).
+__device__ __forceinline__ double lowp_lower(float bo, const QParams& qp, int metric, uint32_t d) {
+  if (bo == INFINITY) return INFINITY;
+  const double bs = (double)bo * qp.scale;
+  double bR = bs + qp.off;
+  bR -= 0x1p-40 * (fabs(bs) + fabs(qp.off));
+  if (metric == kL2 && bR > 0.0) bR *= 1.0 - (double)(d + 4) * 0x1p-52;
+  return bR;
+}
+
+// |first-pass estimate - score| / |score| of a result whose first-pass key
+// is O (finite), for the error report; 0 where it has no value.
+__device__ __forceinline__ double lowp_rel_err(float O, double sc, uint32_t slot,
+                                               const QParams& qp, int metric,
+                                               const RerankArgs& a) {
+  if (!(sc == sc) || sc == 0.0) return 0.0;
+  double est;
+  if (metric == kL2) {
+    // (FP8 keys are the BF16-form key / sq; scale = sq there, 1 for BF16)
+    const double xn = a.st.xn[slot];
+    const double sp = ((double)O - (double)qp.P * (double)a.w0[slot]) * qp.scale;
+    est = sqrt(fmax(qp.nq2 + xn * xn + sp, 0.0));
+  } else if (metric == kDot) {
+    est = -((double)O - (double)qp.P * (double)a.w0[slot]) * qp.scale;
+  } else {
+    est = -(double)O / qp.qn;
+  }
+  return fabs(est - sc) / fabs(sc);
+}
 
 // Candidate rows reach the lanes through LDS: per round of 64 candidates
 // the wave copies kRC columns of all 64 rows at a time (lane l fetches
@@ -662,15 +693,8 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a, uint32_t blk, d
   const uint32_t ndeg = min(*a.degen_count, (uint32_t)kDegenCap);
   const int kk = (int)a.k;
 
-  // FP64 lower bound on the ordering value of a row whose first-pass key is
-  // at least `bo` (the rounding slack of the key's conversion included)
   auto lower = [&](float bo) __attribute__((always_inline)) -> double {
-    if (bo == INFINITY) return INFINITY;
-    const double bs = (double)bo * qp.scale;
-    double bR = bs + qp.off;
-    bR -= 0x1p-40 * (fabs(bs) + fabs(qp.off));
-    if (METRIC == kL2 && bR > 0.0) bR *= 1.0 - (double)(a.d + 4) * 0x1p-52;
-    return bR;
+    return lowp_lower(bo, qp, METRIC, a.d);
   };
   // a flagged query's keys carry no bound: no pruning
   const bool prune = !qp.flags;
@@ -872,22 +896,7 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a, uint32_t blk, d
                  ? (uint64_t)a.st.rank_base[slot >> 6] +
                        (uint64_t)__popcll(a.st.alive[slot >> 6] & ((1ull << (slot & 63)) - 1ull))
                  : slot;
-        // first-pass estimate of this score, for the error report
-        const float O = O2[p];
-        if (O != INFINITY && sc == sc && sc != 0.0) {
-          const double xn = a.st.xn[slot];
-          double est;
-          if (METRIC == kL2) {
-            // (FP8 keys are the BF16-form key / sq; scale = sq there, 1 for BF16)
-            const double sp = ((double)O - (double)qp.P * (double)a.w0[slot]) * qp.scale;
-            est = sqrt(fmax(qp.nq2 + xn * xn + sp, 0.0));
-          } else if (METRIC == kDot) {
-            est = -((double)O - (double)qp.P * (double)a.w0[slot]) * qp.scale;
-          } else {
-            est = -(double)O / qp.qn;
-          }
-          err = fmax(err, fabs(est - sc) / fabs(sc));
-        }
+        if (O2[p] != INFINITY) err = fmax(err, lowp_rel_err(O2[p], sc, slot, qp, METRIC, a));
       }
       a.ids[(size_t)q * a.ostride + e] = id;
       a.scores[(size_t)q * a.ostride + e] = sc;
@@ -897,33 +906,308 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a, uint32_t blk, d
   if (lane == 0) a.max_rel_err[q] = err;
 }
 
-// one wavefront per shortlist row; each range its own metric
-__global__ __launch_bounds__(256) void k_rerank(RangeBatch<RerankArgs> b) {
+// The widening retries: one wavefront per shortlist row, one metric, held to
+// 128 VGPRs for 4 wavefronts per SIMD (the row gather is latency-bound; a few
+// spilled dwords cost less than the lost occupancy: measured 12-20 % faster
+// than the same code at 3 per SIMD)
+template <int METRIC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_rerank1(
+    RerankArgs a) {
   __shared__ double stage[4][64 * (kRC + 1)];
   __shared__ uint32_t queue[4][128];
-  const int i = range_of(b, blockIdx.x);
-  const uint32_t blk = blockIdx.x - b.first[i];
-  double* stg = stage[threadIdx.x >> 6];
-  uint32_t* qu = queue[threadIdx.x >> 6];
-  switch (b.metric[i]) {
-    case kL2: rerank_body<kL2>(b.r[i], blk, stg, qu); break;
-    case kCos: rerank_body<kCos>(b.r[i], blk, stg, qu); break;
-    default: rerank_body<kDot>(b.r[i], blk, stg, qu); break;
+  rerank_body<METRIC>(a, blockIdx.x, stage[threadIdx.x >> 6], queue[threadIdx.x >> 6]);
+}
+
+hipError_t launch_rerank_wide(const RerankArgs& a, int metric, hipStream_t s) {
+  if (a.nq == 0) return hipSuccess;
+  if (!a.carry || !a.lk) return hipErrorInvalidValue;
+  const dim3 grid((a.nq + 3) / 4);
+  switch (metric) {
+    case kL2: hipLaunchKernelGGL(k_rerank1<kL2>, grid, dim3(256), 0, s, a); break;
+    case kCos: hipLaunchKernelGGL(k_rerank1<kCos>, grid, dim3(256), 0, s, a); break;
+    case kDot: hipLaunchKernelGGL(k_rerank1<kDot>, grid, dim3(256), 0, s, a); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+// First-stage rerank (L <= kRrMaxL): one block of 4 wavefronts per query.
+// The candidates — shortlist and degenerate rows — are ordered by first-pass
+// key; the first `m1` are scored, their k-th FP64 key bounds which of the
+// others can still enter the top k (a prefix of the order, since the lower
+// bound grows with the key), those are scored too, and every scored row takes
+// its place by counting the keys before it.  All the orderings are counts over
+// LDS, which costs no more per query at k = 100 than at k = 10, where sorted
+// insertions, one at a time through a wavefront, had taken most of the time.
+//
+// A wavefront scores 16 rows at a time, 64 columns per step: each load
+// instruction reads 512 contiguous bytes of one row, and the next step's
+// loads are in flight during this step's chains (lane l: row l%16; LDS rows
+// are 65 doubles apart, so the 16 chains read distinct banks).  64 columns
+// per step rather than 16 because the time of a small batch is the number of
+// dependent memory round trips; large ones are bound by the row gather.
+// Kernel time against a wavefront per query with sorted insertions: 1 query
+// of 128 columns, L = 64 30 → 13.5 µs; 101 queries of 200 columns, k = 100,
+// L = 256 208 → 37; 32 queries of 1,536 columns, L = 64 209 → 45; 16,384
+// queries of 128 columns, L = 64 299 → 218 (1.07 GB if every row were read);
+// 4,096 queries of 768 columns, k = 100, L = 128 541 → 490 (3.2 GB).
+constexpr int kRrMaxL = 256;
+constexpr int kRrCand = kRrMaxL + kDegenCap;
+constexpr int kRrRows = 16, kRrCols = 64;
+// Queries from which reading fewer rows beats fewer rounds (16,384 queries,
+// L = 64, k = 10: 218 µs in two rounds, 312 in one before the orderings were
+// vectorized; 1 query: 13.5 µs in one).
+constexpr int kRrBulk = 1024;
+
+struct RrShared {
+  double stage[4][kRrRows + 1][kRrCols + 1];  // the last row: the query
+  uint64_t k64[kRrCand];
+  float okey[kRrCand];
+  uint32_t oslot[kRrCand];
+  uint32_t count;  // candidates that need a score, or may
+  uint64_t tau;    // the k-th FP64 key
+  float kmax;
+  float errw[4], kmaxw[4];
+  int n2;
+};
+static_assert(sizeof(RrShared) <= 160 * 1024 / 4, "four blocks per CU");
+
+// FP64 rank keys of the ordered candidates c0 .. c0+15 below n (one
+// wavefront).
+template <bool L2M>
+__device__ __forceinline__ void rr_score(const RerankArgs& a, const QParams& qp, int metric,
+                                         const double* __restrict__ qv, RrShared& sm, int wave,
+                                         int lane, uint32_t c0, uint32_t n) {
+  double(*stg)[kRrCols + 1] = sm.stage[wave];
+  const double* src[kRrRows];
+#pragma unroll
+  for (int u = 0; u < kRrRows; u++)
+    src[u] = a.st.X + (size_t)uni32(sm.oslot[min(c0 + u, n - 1)]) * a.st.ldx;
+  double v[kRrRows], qe = 0.0;
+  auto fetch = [&](uint32_t col) __attribute__((always_inline)) {
+    const uint32_t e = col + lane;
+    const bool in = e < a.d;
+    qe = in ? qv[e] : 0.0;
+#pragma unroll
+    for (int u = 0; u < kRrRows; u++) v[u] = in ? src[u][e] : 0.0;
+  };
+  double acc = 0.0;
+  const double* my = stg[lane & 15];
+  const double* qr = stg[kRrRows];
+  fetch(0);
+  for (uint32_t col = 0; col < a.d; col += kRrCols) {
+#pragma unroll
+    for (int u = 0; u < kRrRows; u++) stg[u][lane] = v[u];
+    stg[kRrRows][lane] = qe;
+    __builtin_amdgcn_wave_barrier();
+    if (col + kRrCols < a.d) fetch(col + kRrCols);
+    __builtin_amdgcn_sched_barrier(0);
+    // (columns past d are zero in both operands: they leave the chain as it
+    // is, up to the sign of a zero, which ranking and scores fold)
+    const uint32_t ne = min((uint32_t)kRrCols, (a.d - col + 7) & ~7u);
+    for (uint32_t t0 = 0; t0 < ne; t0 += 8) {
+      double x[8], q[8];
+#pragma unroll
+      for (int t = 0; t < 8; t++) {
+        x[t] = my[t0 + t];
+        q[t] = qr[t0 + t];
+      }
+#pragma unroll
+      for (int t = 0; t < 8; t++) {
+        if (L2M) {
+          const double tt = x[t] - q[t];
+          acc = fma(tt, tt, acc);
+        } else {
+          acc = fma(q[t], x[t], acc);
+        }
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  const uint32_t c = c0 + lane;
+  if (lane < kRrRows && c < n) {
+    double r = acc;
+    if (metric == kDot) r = -acc;
+    else if (metric == kCos) r = -(acc / (qp.qn * a.st.xn[sm.oslot[c]]));
+    sm.k64[c] = rank_bits64(r);
   }
 }
 
-// ranges of one metric: that metric's code only, held to 128 VGPRs for 4
-// wavefronts per SIMD (the row gather is latency-bound; a few spilled
-// dwords cost less than the lost occupancy: measured 12-20 % faster than
-// the same code at 3 per SIMD)
-template <int METRIC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_rerank1(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_rerank(
     RangeBatch<RerankArgs> b) {
-  __shared__ double stage[4][64 * (kRC + 1)];
-  __shared__ uint32_t queue[4][128];
-  const int i = range_of(b, blockIdx.x);
-  rerank_body<METRIC>(b.r[i], blockIdx.x - b.first[i], stage[threadIdx.x >> 6],
-                      queue[threadIdx.x >> 6]);
+  __shared__ RrShared sm;
+  // the candidates before they are ordered: in the stage, not yet in use
+  // (their keys as order-preserving bits, all ones for the unusable ones)
+  uint32_t* ckey = reinterpret_cast<uint32_t*>(&sm.stage[0][0][0]);
+  uint32_t* cslot = reinterpret_cast<uint32_t*>(&sm.stage[1][0][0]);
+  const int ri = range_of(b, blockIdx.x);
+  const RerankArgs& a = b.r[ri];
+  const int metric = b.metric[ri];
+  const uint32_t q = blockIdx.x - b.first[ri];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const QParams qp = a.qp[q];
+  const double* __restrict__ qv = a.Q + (size_t)q * a.ldq;
+  const uint32_t ndeg_all = *a.degen_count;
+  const uint32_t ndeg = min(ndeg_all, (uint32_t)kDegenCap);
+  const uint32_t nc = a.L + ndeg, kk = a.k;
+  auto lower = [&](float bo) -> double { return lowp_lower(bo, qp, metric, a.d); };
+
+  // candidates: (slot, key), the unusable ones keyed +inf; degenerate rows
+  // first in the order, unless the shortlist holds them too
+  float kmax = -INFINITY;
+  for (uint32_t j = tid; j < nc; j += 256) {
+    uint32_t slot;
+    float key = -INFINITY;
+    if (j < a.L) {
+      slot = a.short_slot[(size_t)q * a.L + j];
+      key = a.short_key[(size_t)q * a.L + j];
+      kmax = fmaxf(kmax, key);
+    } else {
+      slot = a.degen[j - a.L];
+    }
+    const bool ok = slot < a.st.nrows && ((a.st.alive[slot >> 6] >> (slot & 63)) & 1ull);
+    cslot[j] = slot;
+    ckey[j] = ok ? rank_bits32(key) : ~0u;
+  }
+  if (tid < 3) ckey[nc + tid] = ~0u;
+  if (tid == 0) {
+    sm.count = 0;
+    sm.tau = ~0ull;
+    sm.n2 = 0;
+  }
+  for (int o = 32; o >= 1; o >>= 1) kmax = fmaxf(kmax, __shfl_xor(kmax, o));
+  if (lane == 0) sm.kmaxw[wave] = kmax;
+  __syncthreads();
+  for (uint32_t j = a.L + tid; j < nc; j += 256) {
+    const uint32_t slot = cslot[j];
+    bool dup = false;
+    for (uint32_t t = 0; t < a.L; t++) dup |= cslot[t] == slot;
+    if (dup) ckey[j] = ~0u;
+  }
+  __syncthreads();
+  // order by (key, position), unusable ones out
+  for (uint32_t j = tid; j < nc; j += 256) {
+    const uint32_t kb = ckey[j];
+    if (kb == ~0u) continue;
+    uint32_t pos = 0;
+    for (uint32_t t = 0; t < nc; t += 4) {
+      const uint4 o = *reinterpret_cast<const uint4*>(ckey + t);
+      pos += (o.x < kb) | ((o.x == kb) & (t < j));
+      pos += (o.y < kb) | ((o.y == kb) & (t + 1 < j));
+      pos += (o.z < kb) | ((o.z == kb) & (t + 2 < j));
+      pos += (o.w < kb) | ((o.w == kb) & (t + 3 < j));
+    }
+    sm.oslot[pos] = cslot[j];
+    sm.okey[pos] = __uint_as_float((kb >> 31) ? (kb & 0x7FFFFFFFu) : ~kb);
+    atomicAdd(&sm.count, 1u);
+  }
+  __syncthreads();
+  const uint32_t n = sm.count;
+  // First round.  A large batch is bound by the rows it reads: no more than
+  // the k (and the degenerate rows) are read before their k-th key can bound
+  // the rest.  A small one is bound by latency: the four wavefronts read 64
+  // rows at once.
+  uint32_t m1 = (kk + ndeg + kRrRows - 1) & ~(uint32_t)(kRrRows - 1);
+  if (a.nq < (uint32_t)kRrBulk) m1 = max(m1, 4u * kRrRows);
+  m1 = min(m1, n);
+  auto score = [&](uint32_t c0, uint32_t end) {
+    for (uint32_t c = c0 + kRrRows * wave; c < end; c += 4 * kRrRows) {
+      if (metric == kL2) rr_score<true>(a, qp, metric, qv, sm, wave, lane, c, end);
+      else rr_score<false>(a, qp, metric, qv, sm, wave, lane, c, end);
+    }
+  };
+  // entry j's rank among the first m scored rows, by (key, slot)
+  auto rank_of = [&](uint32_t j, uint32_t m) {
+    const uint64_t K = sm.k64[j];
+    const uint32_t S = sm.oslot[j];
+    uint32_t r = 0;
+    for (uint32_t t = 0; t < m; t++) r += lt2(sm.k64[t], sm.oslot[t], K, S);
+    return r;
+  };
+  score(0, m1);
+  __syncthreads();
+  uint32_t ns = m1;  // rows scored
+  if (n > m1) {
+    for (uint32_t j = tid; j < m1; j += 256)
+      if (rank_of(j, m1) + 1 == kk) sm.tau = sm.k64[j];
+    __syncthreads();
+    // A row whose lower bound exceeds the k-th value cannot be in the top k
+    // (a flagged query's keys carry no bound; a NaN bound keeps its row).
+    const double thr = !qp.flags && sm.tau != ~0ull ? rank_val64(sm.tau) : INFINITY;
+    int mine = 0;
+    for (uint32_t j = m1 + tid; j < n; j += 256) mine = !(lower(sm.okey[j]) > thr) ? (int)j + 1 : mine;
+    if (mine) atomicMax(&sm.n2, mine);
+    __syncthreads();
+    ns = max(m1, (uint32_t)sm.n2);
+    if (tid == 0) sm.tau = ~0ull;
+    score(m1, ns);
+    __syncthreads();
+  }
+  uint32_t rk[2] = {~0u, ~0u};
+#pragma unroll
+  for (int p = 0; p < 2; p++) {
+    const uint32_t j = tid + 256 * p;
+    if (j < ns) {
+      rk[p] = rank_of(j, ns);
+      if (rk[p] + 1 == kk) sm.tau = sm.k64[j];
+    }
+  }
+  __syncthreads();
+
+  // certification (more degenerate rows than the list holds: nothing can be
+  // certified)
+  const double tau = sm.tau == ~0ull ? INFINITY : rank_val64(sm.tau);
+  const bool cert =
+      !qp.flags && ndeg_all <= (uint32_t)kDegenCap && tau < lower(a.beta[q]);
+  if (!cert) {
+    if (a.lk) {
+#pragma unroll
+      for (int p = 0; p < 2; p++)
+        if (rk[p] < kk) {
+          a.lk[(size_t)q * kk + rk[p]] = sm.k64[tid + 256 * p];
+          a.ls[(size_t)q * kk + rk[p]] = sm.oslot[tid + 256 * p];
+        }
+      for (uint32_t e = ns + tid; e < kk; e += 256) {
+        a.lk[(size_t)q * kk + e] = ~0ull;
+        a.ls[(size_t)q * kk + e] = ~0u;
+      }
+    }
+    if (tid == 0) {
+      if (a.lk)
+        a.kmax[q] = fmaxf(fmaxf(sm.kmaxw[0], sm.kmaxw[1]), fmaxf(sm.kmaxw[2], sm.kmaxw[3]));
+      a.fail_list[atomicAdd(a.fail_count, 1u)] = q;
+    }
+    return;
+  }
+  double err = 0.0;
+#pragma unroll
+  for (int p = 0; p < 2; p++) {
+    if (rk[p] >= kk) continue;
+    const uint32_t j = tid + 256 * p, slot = sm.oslot[j];
+    const double v = rank_val64(sm.k64[j]);
+    double sc = __longlong_as_double(0x7FF8000000000000ll);
+    if (v == v) sc = metric == kL2 ? sqrt(v) : (v == 0.0 ? 0.0 : -v);
+    const uint64_t id =
+        a.st.has_deletes
+            ? (uint64_t)a.st.rank_base[slot >> 6] +
+                  (uint64_t)__popcll(a.st.alive[slot >> 6] & ((1ull << (slot & 63)) - 1ull))
+            : slot;
+    const float O = sm.okey[j];
+    if (O > -INFINITY && O < INFINITY)
+      err = fmax(err, lowp_rel_err(O, sc, slot, qp, metric, a));
+    a.ids[(size_t)q * a.ostride + rk[p]] = id;
+    a.scores[(size_t)q * a.ostride + rk[p]] = sc;
+  }
+  for (uint32_t e = ns + tid; e < kk; e += 256) {
+    a.ids[(size_t)q * a.ostride + e] = ~0ull;
+    a.scores[(size_t)q * a.ostride + e] = __longlong_as_double(0x7FF8000000000000ll);
+  }
+  for (int off = 32; off >= 1; off >>= 1) err = fmax(err, __shfl_xor(err, off));
+  if (lane == 0) sm.stage[wave][0][0] = err;
+  __syncthreads();
+  if (tid == 0)
+    a.max_rel_err[q] = fmax(fmax(sm.stage[0][0][0], sm.stage[1][0][0]),
+                            fmax(sm.stage[2][0][0], sm.stage[3][0][0]));
 }
 
 hipError_t launch_rerank_ranges(const RerankArgs* a, const int* metric, int n, hipStream_t s) {
@@ -931,30 +1215,22 @@ hipError_t launch_rerank_ranges(const RerankArgs* a, const int* metric, int n, h
     RangeBatch<RerankArgs> b{};
     uint32_t blocks = 0;
     b.n = 0;
-    bool one = true;
     for (int r = r0; r < n && b.n < kMaxLaunchRanges; r++) {
       if (metric[r] != kL2 && metric[r] != kCos && metric[r] != kDot) return hipErrorInvalidValue;
+      if (a[r].L > (uint32_t)kRrMaxL || a[r].carry || a[r].qidx) return hipErrorInvalidValue;
       b.r[b.n] = a[r];
       b.metric[b.n] = metric[r];
       b.first[b.n] = blocks;
-      blocks += (a[r].nq + 3) / 4;
-      one &= metric[r] == metric[r0];
+      blocks += a[r].nq;
       b.n++;
     }
     b.first[b.n] = blocks;
     if (blocks == 0) continue;
-    if (!one) hipLaunchKernelGGL(k_rerank, dim3(blocks), dim3(256), 0, s, b);
-    else if (metric[r0] == kL2) hipLaunchKernelGGL(k_rerank1<kL2>, dim3(blocks), dim3(256), 0, s, b);
-    else if (metric[r0] == kCos) hipLaunchKernelGGL(k_rerank1<kCos>, dim3(blocks), dim3(256), 0, s, b);
-    else hipLaunchKernelGGL(k_rerank1<kDot>, dim3(blocks), dim3(256), 0, s, b);
+    hipLaunchKernelGGL(k_rerank, dim3(blocks), dim3(256), 0, s, b);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
-}
-
-hipError_t launch_rerank(const RerankArgs& a, int metric, hipStream_t s) {
-  return launch_rerank_ranges(&a, &metric, 1, s);
 }
 
 // ------------------------------------------------------------- fallback plumbing

@@ -37,3 +37,34 @@ def test_query_prep_widths(precision, d):
         for metric in ("l2", "cos", "dot"):
             check(db, X, Q[:nq], 7, metric, precision)
     db.close()
+
+
+@pytest.mark.parametrize("n,d,nq,k,short", [
+    (1, 5, 3, 4, None),       # fewer rows than k
+    (40, 64, 2, 40, None),    # k is every row
+    (700, 65, 1, 1, 256),     # a shortlist far wider than k: the second round
+    (700, 63, 5, 128, 256),
+    (900, 16, 4, 17, 17),     # the shortlist is k
+    (900, 129, 1030, 10, 64), # a bulk batch: k rows, then what their k-th leaves
+    (900, 8, 1024, 128, None),
+])
+def test_rerank_shapes(n, d, nq, k, short):
+    """Row counts, widths, k and shortlist widths around the first-stage
+    rerank's rounds (16 rows, 64 columns, 1,024 queries), over a store with
+    duplicated rows (ties by id) and with degenerate rows, which enter every
+    query's candidates, also when they are its answer."""
+    rng = np.random.default_rng(n + d)
+    X = rng.integers(-3, 4, size=(n, d)).astype(np.float64)
+    if n > 4:
+        X[n // 2:] = X[:n - n // 2]
+        X[1] = 0.0
+        X[n - 1] = 0.0
+        X[2] = 1e30
+    Q = rng.integers(-3, 4, size=(nq, d)) + 0.125 * rng.standard_normal((nq, d))
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    if short:
+        db.set_shortlist(short)
+    for metric in ("l2", "cos", "dot"):
+        check(db, X, Q, k, metric, "bf16")
+    db.close()
