@@ -952,7 +952,7 @@ uint32_t Engine::lowp_width(int kk, bool fp8, size_t shortlist) {
 
 int Engine::run_lowp(const double* dQ, size_t ldq, uint32_t nq, int metric, int k,
                      uint64_t* dids, double* dscores, uint32_t ostride, bool fp8) {
-  LowpRange r{metric, 0, nq, k, 0, 0, 0, 0, 0};
+  LowpRange r{metric, 0, nq, k, 0, 0, 0, 0, 0, 0};
   return run_lowp_ranges(dQ, ldq, &r, 1, k, dids, dscores, ostride, fp8);
 }
 
@@ -1001,21 +1001,66 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   const uint32_t nrows_pad = (uint32_t)round_up(nphys_, kLowpTile);
   const uint32_t groups = nq_pad / qpb;
   const uint32_t tiles = nrows_pad / kLowpTile;
+  // Sample pre-pass: the same scan over ns_pre evenly spaced runs of tp
+  // tiles (at most 1/16 of the store, a quarter of one below 1,024 tiles),
+  // each lane keeping only the smallest key of its rows.  The lanes' rows are
+  // disjoint, so the j-th smallest of those minima is the ordering key of a
+  // real row with j-1 others at or below it, and about j / f rows of the store
+  // lie below it (f: the sampled fraction).  The main scan's lists start from
+  // it: they then skip nearly every row from the first tile on, and take a
+  // few hundred rows per query in all.
+  // BF16: j = 3·L·f, so that about three times the shortlist passes, and at
+  // least k + 16, so that at least that many do however the rows are placed.
+  // (j = L let about L / f rows pass: 1M × 128, 16 times the shortlist.)
+  // FP8 keeps j = L: its widening retries look for up to kMaxShort candidates
+  // in the lists, and its error band needs them.
+  uint32_t ns_pre = tiles >= 16 * kPrepassSlices       ? kPrepassSlices
+                    : tiles >= 16 * kPrepassSlices / 4 ? kPrepassSlices / 4
+                    : tiles >= 128                     ? 32
+                                                       : 16;
+  // BF16: twice the sample for shortlists past 64 (their threshold sits
+  // further out, and a sparser sample leaves more rows below it to insert)
+  // and for batches of up to 4096 queries (the scan's saving outweighs the
+  // larger pre-pass there; at 16,384 queries and L = 64 they break even).
+  // Not FP8: a list the threshold leaves short bounds β by the threshold,
+  // and FP8's wider error band then certifies fewer queries (measured on
+  // 5M x 768 cosine: 861 instead of 4,293 of 12,288 before the BF16 pass).
+  const uint32_t tpmax =
+      (!fp8 && (L > 64 || nq <= 4096)) ? 2 * kPrepassMaxTiles : kPrepassMaxTiles;
+  const uint32_t tp =
+      std::max<uint32_t>(1, std::min<uint32_t>(tpmax, tiles / (16 * ns_pre)));
+  const double frac = (double)ns_pre * tp / tiles;
+  auto thr_rank = [&](int kk) {
+    const uint32_t w = width(kk);
+    return fp8 ? w
+               : std::min<uint32_t>(
+                     w, std::max<uint32_t>((uint32_t)std::ceil(3.0 * w * frac), kk + 16));
+  };
+  const bool pre =
+      prepass_ && tiles >= 4 * ns_pre && ns_pre * kLowpLanesPerQuery >= thr_rank(k);
+  const uint32_t NL_pre = ns_pre * kLowpLanesPerQuery;
   // Row slices for a scan of grp query blocks wanting kk neighbours: at
-  // least 8 (each query then has >= 32 candidate lists, so the lists' own
-  // bound sits well past the shortlist's), more when there are few query
-  // blocks, each at least 4 tiles long.  One block per CU fits at a time,
-  // so the grid is kept at or just under two rounds of the 256 CUs (a few
-  // blocks past a round cost a whole round).
+  // least 8, more when there are few query blocks, each at least 4 tiles
+  // long.  One block per CU fits at a time, so the grid is kept at or just
+  // under two rounds of the 256 CUs (a few blocks past a round cost a whole
+  // round).  With a threshold, enough that the rows it lets pass fill a list
+  // to half on average (a full list's bound becomes its largest key, which
+  // may then lie below the shortlist's); without one, past k = 32 at least
+  // 512 lists per query and for FP8 2,048, which keep the lists' own bound
+  // (the smallest 8th entry) clear of the k-th neighbour and of the retries'
+  // 4,096th candidate.
   auto slicing = [&](uint32_t grp, int kk, LowpRange& r) {
     uint32_t ns = std::max<uint32_t>(8, (512 / grp) & ~7u);
-    // Past k = 32 the lists' own bound (the smallest 8th entry) must stay
-    // well beyond the k-th neighbour: at least 512 lists per query.
-    if (kk > 32) ns = std::max<uint32_t>(ns, 128);
-    // FP8: the widening retries take up to kMaxShort candidates from these
-    // lists; 2048 lists per query keep their own bound (the smallest 8th
-    // entry) clear of the 4096th candidate.
-    if (fp8) ns = std::max<uint32_t>(ns, 512);
+    // rows below the threshold: a lane's smallest of m rows lies below it with
+    // probability 1 - (1 - p)^m = j / (number of lanes), p the share of rows
+    const double m = tp * (double)kLowpTile / kLowpLanesPerQuery;
+    r.pass = pre ? (uint32_t)(nrows_pad * -std::expm1(std::log1p(-std::min(0.99, (double)thr_rank(kk) / NL_pre)) / m))
+                 : 0;
+    if (pre) ns = std::max<uint32_t>(ns, r.pass / (kLowpLC / 2 * kLowpLanesPerQuery));
+    else if (fp8) ns = std::max<uint32_t>(ns, 512);
+    else if (kk > 32) ns = std::max<uint32_t>(ns, 128);
+    // (a query's lists stay within 128 KiB: 960 lists of 17 words)
+    ns = std::min<uint32_t>(ns, pre ? 240 : 512);
     ns = std::max<uint32_t>(1, std::min<uint32_t>(ns, std::max<uint32_t>(1, tiles / 4)));
     r.rps = (uint32_t)((tiles + ns - 1) / ns) * kLowpTile;
     ns = (nrows_pad + r.rps - 1) / r.rps;
@@ -1042,7 +1087,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     else
       sgs.push_back({i, i + 1, mixed_scan ? kMixed : R[i].metric, R[i].soff, 0});
   }
-  size_t cand_end = 0;  // candidate-list entries, all groups
+  size_t nlists = 0;  // candidate lists, all groups
   for (auto& g : sgs) {
     const LowpRange& last = R[g.r1 - 1];
     g.n = last.soff + last.n - g.soff;
@@ -1055,38 +1100,22 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
       R[i].ns = sl.ns;
       R[i].rps = sl.rps;
       R[i].NL = sl.NL;
-      R[i].coff = cand_end + (size_t)(R[i].soff - g.soff) * sl.NL * kLowpLP;
+      R[i].pass = sl.pass;
+      R[i].coff = nlists + (size_t)(R[i].soff - g.soff) * sl.NL;
     }
-    cand_end += (size_t)(send - g.soff) * sl.NL * kLowpLP;
+    nlists += (size_t)(send - g.soff) * sl.NL;
   }
-  // Sample pre-pass: the same scan over ns_pre evenly spaced runs of tp
-  // tiles (at most 1/16 of the store), each lane keeping only the smallest
-  // key of its rows.  The lanes' rows are disjoint, so the L-th smallest of
-  // those minima is the ordering key of a real row with L-1 others at or
-  // below it: the global L-th key lies at or below it, and the main scan's
-  // lists start from it.  They then skip nearly every row from the first
-  // tile on, where otherwise a short slice spends most of its subtiles
-  // filling its lists (the insertion path costs several times the MFMAs).
-  const uint32_t ns_pre = tiles >= 16 * kPrepassSlices ? kPrepassSlices : kPrepassSlices / 4;
-  const bool pre = prepass_ && tiles >= 16 * ns_pre && ns_pre * kLowpLanesPerQuery >= L;
-  // BF16: twice the sample for shortlists past 64 (their threshold sits
-  // further out, and a sparser sample leaves more rows below it to insert)
-  // and for batches of up to 4096 queries (the scan's saving outweighs the
-  // larger pre-pass there; at 16,384 queries and L = 64 they break even).
-  // Not FP8: a list the threshold leaves short bounds β by the threshold,
-  // and FP8's wider error band then certifies fewer queries (measured on
-  // 5M x 768 cosine: 861 instead of 4,293 of 12,288 before the BF16 pass).
-  const uint32_t tpmax =
-      (!fp8 && (L > 64 || nq <= 4096)) ? 2 * kPrepassMaxTiles : kPrepassMaxTiles;
-  const uint32_t tp = pre ? std::min<uint32_t>(tpmax, tiles / (16 * ns_pre)) : 0;
-  const uint32_t NL_pre = ns_pre * kLowpLanesPerQuery;
-  const size_t ncand = std::max(cand_end, pre ? (size_t)nq * NL_pre : (size_t)0);
   // query rows: nq_pad slots plus one block, since a launch over one range
   // (at slot offset soff) reads whole blocks of rows from soff on
   if ((rc = scratch(&c_->s_qb_, &c_->s_qb_n_, ((size_t)nq_pad + qpb) * dp * qbytes))) return rc;
   if ((rc = scratch(&c_->s_qp_, &c_->s_qp_n_, (size_t)nq_pad * sizeof(QParams)))) return rc;
-  if ((rc = scratch(&c_->s_ck_, &c_->s_ck_n_, ncand * sizeof(float)))) return rc;
-  if ((rc = scratch(&c_->s_cs_, &c_->s_cs_n_, ncand * sizeof(uint32_t)))) return rc;
+  // list headers (before them, in the same place, the pre-pass's keys) and
+  // entries
+  if ((rc = scratch(&c_->s_ck_, &c_->s_ck_n_,
+                    std::max(nlists * sizeof(uint2),
+                             pre ? (size_t)nq * NL_pre * sizeof(float) : (size_t)0))))
+    return rc;
+  if ((rc = scratch(&c_->s_cs_, &c_->s_cs_n_, nlists * kLowpLC * sizeof(uint2)))) return rc;
   if ((rc = scratch(&c_->s_sk_, &c_->s_sk_n_, (size_t)nq * L * sizeof(float)))) return rc;
   if ((rc = scratch(&c_->s_ss_, &c_->s_ss_n_, (size_t)nq * L * sizeof(uint32_t)))) return rc;
   if ((rc = scratch(&c_->s_beta_, &c_->s_beta_n_, (size_t)nq * sizeof(float)))) return rc;
@@ -1141,7 +1170,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // the fields every launch shares; each sets its own rows, queries and lists
   LowpScanArgs sa{fp8 ? (const uint16_t*)sh8_.X8 : sh_.Xb, dp, nullptr, nullptr, nullptr,
                   nullptr, (const uint16_t*)c_->s_qb_, (const QParams*)c_->s_qp_, nq, 0, 0,
-                  nrows_pad, 0, (float*)c_->s_ck_, (uint32_t*)c_->s_cs_, nullptr, 0};
+                  nrows_pad, 0, (float*)c_->s_ck_, (uint2*)c_->s_ck_, (uint2*)c_->s_cs_, nullptr, 0};
   if (pre) {
     prof_begin(SVDB_K_PREPASS);
     for (int i = 0; i < nr; i++) {
@@ -1160,7 +1189,8 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
       // thresholds in c_->s_beta_, read by the main scan before the shortlist
       // below overwrites them (padding slots' values are never used)
       HIPCHK(launch_kth_key((const float*)c_->s_ck_ + (size_t)R[i].soff * NL_pre, R[i].n, NL_pre,
-                            width(R[i].k), (float*)c_->s_beta_ + R[i].soff, c_->stream), "k_kth_key");
+                            thr_rank(R[i].k), (float*)c_->s_beta_ + R[i].soff, c_->stream),
+             "k_kth_key");
     }
     prof_end(SVDB_K_PREPASS);
     sa.tau0 = (const float*)c_->s_beta_;
@@ -1181,8 +1211,8 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     ma.nq = g.n;
     ma.rows_per_slice = ma.slice_stride = r.rps;
     ma.NL = r.NL;
-    ma.cand_key = (float*)c_->s_ck_ + r.coff;
-    ma.cand_slot = (uint32_t*)c_->s_cs_ + r.coff;
+    ma.hdr = (uint2*)c_->s_ck_ + r.coff;
+    ma.ent = (uint2*)c_->s_cs_ + r.coff * kLowpLC;
     if (ma.tau0) ma.tau0 += g.soff;
     HIPCHK(scan(ma, g.metric, r.ns, false), "first-pass scan");
   }
@@ -1192,8 +1222,8 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // every range's shortlist, in as few launches as the kernels allow
   std::vector<ShortlistArgs> sls(nr);
   for (int i = 0; i < nr; i++)
-    sls[i] = ShortlistArgs{(const float*)c_->s_ck_ + R[i].coff, (const uint32_t*)c_->s_cs_ + R[i].coff,
-                           R[i].n, R[i].NL, width(R[i].k),
+    sls[i] = ShortlistArgs{(const uint2*)c_->s_ck_ + R[i].coff,
+                           (const uint2*)c_->s_cs_ + R[i].coff * kLowpLC, R[i].n, R[i].NL, width(R[i].k),
                            (uint32_t*)c_->s_ss_ + (size_t)R[i].soff * L,
                            (float*)c_->s_sk_ + (size_t)R[i].soff * L, (float*)c_->s_beta_ + R[i].soff};
   prof_begin(SVDB_K_SHORTLIST);
@@ -1315,18 +1345,22 @@ int Engine::lowp_complete() {
     const double* rQ = dQ + (size_t)rg.qoff * ldq;
     uint64_t* rids = dids + (size_t)rg.qoff * ostride;
     double* rsc = dscores + (size_t)rg.qoff * ostride;
-    const float* rck = (const float*)c_->s_ck_ + rg.coff;
-    const uint32_t* rcs = (const uint32_t*)c_->s_cs_ + rg.coff;
+    const uint2* rhdr = (const uint2*)c_->s_ck_ + rg.coff;
+    const uint2* rent = (const uint2*)c_->s_cs_ + rg.coff * kLowpLC;
     const RerankArgs ra = rerank_args(ri);
     uint32_t* fail_list = ra.fail_list;  // may be redirected to a widening retry's list
     uint32_t nf = nf1;
     // Widening retries: queries not certified at L are shortlisted again at
-    // 1024, then 4096, from the same candidate lists (when they hold at
-    // least twice that many entries) and reranked; only those still
+    // 1024, then 4096, from the same candidate lists (when they hold more
+    // than the stage before took: with a threshold about rg.pass entries,
+    // without one up to kLowpLP a list) and reranked; only those still
     // uncertified go on.
+    uint32_t Lprev = L;
     for (int wi = 0; wi < 2; wi++) {
       const uint32_t Lw = wi == 0 ? 1024u : (uint32_t)kMaxShort;
-      if (nf == 0 || Lw <= L || (size_t)NL * kLowpLP < 2 * (size_t)Lw) continue;
+      if (nf == 0 || Lw <= L) continue;
+      if (rg.pass ? 2 * rg.pass < 3 * Lprev : (size_t)NL * kLowpLP < 2 * (size_t)Lw) continue;
+      Lprev = Lw;
       // A retry that has lately certified almost none of its queries for
       // this precision and metric is skipped (its queries go on to the next
       // stage), except every 16th time, which keeps the estimate current.
@@ -1343,7 +1377,7 @@ int Engine::lowp_complete() {
           (uint32_t*)c_->s_fail2_ + (fail_list == (uint32_t*)c_->s_fail2_ + 1 ? nf + 1 : 0);
       uint32_t* out_list = out_count + 1;
       HIPCHK(hipMemsetAsync(out_count, 0, sizeof(uint32_t), c_->stream), "memset");
-      ShortlistArgs sw{rck, rcs, nf, NL, Lw, (uint32_t*)c_->s_ss2_, (float*)c_->s_sk2_,
+      ShortlistArgs sw{rhdr, rent, nf, NL, Lw, (uint32_t*)c_->s_ss2_, (float*)c_->s_sk2_,
                        (float*)c_->s_beta2_, fail_list};
       prof_begin(SVDB_K_SHORTLIST);
       HIPCHK(launch_shortlist(sw, c_->stream), "k_shortlist (widened)");
@@ -1844,7 +1878,7 @@ int Engine::search_begin_locked(SearchCtx& c, const double* Q, size_t nq, size_t
         if (metric[i] == m) sel.push_back(i);
       if (sel.size() > first)
         R[nr++] = LowpRange{m, (uint32_t)first, (uint32_t)(sel.size() - first), (int)kmax_all,
-                            0, 0, 0, 0, 0};
+                            0, 0, 0, 0, 0, 0};
     }
     const size_t n = sel.size();
     if ((rc = scratch(&c.s_q_, &c.s_q_n_, n * D * sizeof(double)))) return rc;

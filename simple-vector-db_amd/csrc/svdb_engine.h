@@ -160,6 +160,7 @@ class Engine {
     // first-pass row slicing of this range's scan and where its candidate
     // lists start (set by run_lowp_ranges)
     uint32_t ns, rps, NL;
+    uint32_t pass;         // rows its threshold lets into the lists, about (0: no threshold)
     size_t coff;
   };
   static uint32_t lowp_width(int kk, bool fp8, size_t shortlist);

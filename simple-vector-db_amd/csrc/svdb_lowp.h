@@ -31,7 +31,8 @@ constexpr int kLowpWaves = 8;                      // wavefronts per block
 constexpr int kLowpQF = 4;                         // 16-query fragments per wavefront
 constexpr int kLowpQPB = kLowpWaves * kLowpQF * 16;  // queries per block (512)
 constexpr int kLowpTile = 128;                     // rows per LDS tile
-constexpr int kLowpLP = 8;                         // entries per per-lane list
+constexpr int kLowpLP = 8;                         // entries of a list kept in registers
+constexpr int kLowpLC = 16;                        // entries of a candidate list in memory
 constexpr int kLowpLanesPerQuery = 4;              // lists per query per slice
 constexpr int kDegenCap = 64;                      // degenerate rows kept in the list
 constexpr int kMaxShort = 4096;                    // widest shortlist (the widening retries)
@@ -97,20 +98,19 @@ struct LowpScanArgs {
   uint32_t slice_stride;    // rows from one slice's start to the next's (>= rows_per_slice)
   uint32_t nrows_pad;       // rows readable in Xb / aux (multiple of kLowpTile)
   uint32_t NL;              // lists per query = slices * 4
-  float* cand_key;          // [nq][NL][LP]
-  uint32_t* cand_slot;
+  float* cand_key;          // [nq][NL] sample pre-pass: each list's smallest key
+  uint2* hdr;               // [nq][NL] {entries, fp32 bound on the rows left out}
+  uint2* ent;               // [nq][NL][kLowpLC] {fp32 ordering key, slot}
   // Optional per-query starting threshold: query q's lists only take keys
-  // below tau0[q * tau0_stride].  It must be the ordering key of an actual
-  // row that has at least L-1 rows keyed at or below it (e.g. the L-th key
-  // of a shortlist over a sample of the rows), so the global top-L lies
-  // below it; a list left short then reports the threshold as its bound.
+  // below tau0[q * tau0_stride], the ordering key of an actual row (so that a
+  // list which leaves nothing else out has it as its bound).
   const float* tau0;
   uint32_t tau0_stride;
 };
 
 struct ShortlistArgs {
-  const float* cand_key;
-  const uint32_t* cand_slot;
+  const uint2* hdr;
+  const uint2* ent;
   uint32_t nq, NL, L;
   uint32_t* short_slot;     // [nq][L]  (UINT32_MAX when fewer)
   float* short_key;         // [nq][L]

@@ -303,214 +303,216 @@ hipError_t launch_query_prep(const QueryPrepArgs& a, hipStream_t s) {
 
 // ------------------------------------------------------------- shortlist
 //
-// One wavefront per query: merge the query's NL candidate lists (8 entries
-// each) into the L best by (ordering key, slot), and the bound
-// beta = min(8th entry of every list, L-th merged key): no row outside the
-// shortlist has a smaller ordering key.
+// One block per query: the L smallest ordering keys of the query's NL candidate
+// lists (svdb_cand.h), unordered (the rerank orders them), and the bound
+// beta = min(every list's bound, L-th key): no row outside the shortlist has
+// a smaller ordering key.  The headers are read first, all together; then four
+// threads take a list, four entries each, and each thread has four such loads
+// in flight, so the time goes with neither the lists' number nor their length
+// but with both.  The entries are packed into LDS as order-preserving bits and the L-th smallest is found by
+// counting them into 256 bins of the range that still holds it, until a bin is
+// one key wide (2 or 3 counts for keys of one magnitude).  More entries than
+// the LDS holds (the widening retries over full lists) are read again from the
+// lists instead. 
+// Against a wavefront per query with a sorted list (L <= 64) and radix passes
+// over every list slot (wider): 1 query over 1M rows 108 → 9 µs, 16,384 over
+// 2M rows 310 → 66, 1,400 queries at L = 256 over 1M rows 137 → 95, 4,096 FP8
+// queries at L = 128 270 → 87, at 1,024 310 → 87.
+// LDS capacity: the lists of a 64-wide shortlist hold some 400 entries (FP8
+// 1,600), wider ones' up to about 3,500; 4,096 for all had 4 blocks per CU
+// where 2,048 has 8 (16,384 queries, L = 64: 106 against 66 µs; 4,096 FP8
+// queries, L = 128: 87 against 524, most of them read again).
+constexpr uint32_t kSelLists = 2048;
 
-template <int KPL>
-__device__ __forceinline__ void shortlist_body(const ShortlistArgs& a, uint32_t blk) {
-  const int lane = threadIdx.x & 63;
-  const uint32_t i = blk * 4 + (threadIdx.x >> 6);
-  if (i >= a.nq) return;
-  const uint32_t q = a.qidx ? a.qidx[i] : i;  // candidate lists of query q -> output row i
-  const uint32_t n = a.NL * kLowpLP;
-  const size_t base = (size_t)q * n;
-  WL<KPL> L;
-  L.init();
-  const int kk = (int)a.L;
-  uint64_t tk = ~0ull;
-  uint32_t ts = ~0u;
-  float lane_min = INFINITY;
-  // Entries are read kSlU batches of 64 at a time, so the loads of a batch
-  // group are in flight together (most entries fail the ballot and cost
-  // only their load).
-  constexpr int kSlU = 8;
-  for (uint32_t c0 = 0; c0 < n; c0 += 64 * kSlU) {
-    float key[kSlU];
-    uint32_t slot[kSlU];
-#pragma unroll
-    for (int u = 0; u < kSlU; u++) {
-      const uint32_t c = c0 + u * 64 + lane;
-      key[u] = INFINITY;
-      slot[u] = ~0u;
-      if (c < n) {
-        key[u] = a.cand_key[base + c];
-        slot[u] = a.cand_slot[base + c];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kSlU; u++) {
-      const uint32_t c = c0 + u * 64 + lane;
-      if (c < n && (c % kLowpLP) == kLowpLP - 1) lane_min = fminf(lane_min, key[u]);
-      const uint64_t K = slot[u] == ~0u ? ~0ull : (uint64_t)rank_bits32(key[u]);
-      uint64_t m = __ballot(slot[u] != ~0u && lt2(K, slot[u], tk, ts));
-      while (m) {
-        int src = __ffsll((long long)m) - 1;
-        m &= m - 1;
-        L.insert(uni64(__shfl(K, src)), uni32(__shfl(slot[u], src)), kk, lane);
-        // lanes that no longer beat the (moved) kk-th entry drop out
-        L.at(kk - 1, tk, ts);
-        m &= __ballot(lt2(K, slot[u], tk, ts));
-      }
-      L.at(kk - 1, tk, ts);
-    }
-  }
-  // min over lanes of the lists' 8th entries
-  for (int off = 32; off >= 1; off >>= 1) lane_min = fminf(lane_min, __shfl_xor(lane_min, off));
-  float oL = INFINITY;
-  if (ts != ~0u) {
-    const uint32_t u = (uint32_t)tk;
-    oL = __uint_as_float((u >> 31) ? (u & 0x7FFFFFFFu) : ~u);
-  }
-#pragma unroll
-  for (int p = 0; p < KPL; p++) {
-    const int e = p * 64 + lane;
-    if (e < kk) {
-      const uint32_t u = (uint32_t)L.k[p];
-      a.short_slot[(size_t)i * a.L + e] = L.s[p];
-      a.short_key[(size_t)i * a.L + e] =
-          L.s[p] == ~0u ? INFINITY : __uint_as_float((u >> 31) ? (u & 0x7FFFFFFFu) : ~u);
-    }
-  }
-  if (lane == 0) a.beta[i] = fminf(lane_min, oL);
-}
-
-// Wide shortlists (L > 256): one 256-thread block per query.  The query's
-// n <= 256*kSelPT candidate keys sit in registers as order-preserving
-// uint32 (empty entries: all ones); four 8-bit histogram passes in LDS find
-// the L-th smallest key K*; every entry below K* and enough entries equal to
-// it are written out, unordered (the rerank does not need an order).  A row
-// left out has a key >= K* or >= its list's 8th entry, so
-// beta = min(8th entry of every list, K*) as in the sorted form.
-constexpr int kSelPT = 64;
-
+template <int T, uint32_t CAP>
 struct SelShared {
+  uint32_t key[CAP], slot[CAP];
+  uint8_t cnt[kSelLists];
   uint32_t hist[256];
-  uint32_t prefix, mask, rank, nvalid, lt, eq;
-  float min[4];
+  uint32_t n, lo, hi, rank, lt, eq;
+  uint32_t wlo[T / 64], whi[T / 64];
+  float wmin[T / 64];
 };
 
-__device__ __forceinline__ void shortlist_sel_body(const ShortlistArgs& a, uint32_t blk,
-                                                   SelShared& sm) {
-  uint32_t* hist = sm.hist;
-  uint32_t &s_prefix = sm.prefix, &s_mask = sm.mask, &s_rank = sm.rank, &s_nvalid = sm.nvalid,
-           &s_lt = sm.lt, &s_eq = sm.eq;
-  float* s_min = sm.min;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t i = blk;
-  const uint32_t q = a.qidx ? a.qidx[i] : i;
-  const uint32_t n = a.NL * kLowpLP;
-  const size_t base = (size_t)q * n;
-  uint32_t u[kSelPT];
-  float lmin = INFINITY;
-  uint32_t nv = 0;
+__device__ __forceinline__ float rank_float32(uint32_t u) {
+  return __uint_as_float((u >> 31) ? (u & 0x7FFFFFFFu) : ~u);
+}
+
+// This lane's first place of `m` in a block-wide counter: the wavefront's
+// lanes are counted together and reserved with one atomic.
+__device__ __forceinline__ uint32_t wave_reserve(uint32_t* counter, uint32_t m, int lane) {
+  uint32_t inc = m;
 #pragma unroll
-  for (int t = 0; t < kSelPT; t++) {
-    const uint32_t c = t * 256 + tid;
-    u[t] = 0xFFFFFFFFu;
-    if (c < n) {
-      const float key = a.cand_key[base + c];
-      if ((c % kLowpLP) == kLowpLP - 1) lmin = fminf(lmin, key);
-      if (a.cand_slot[base + c] != ~0u) {
-        u[t] = rank_bits32(key);
-        nv++;
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t v = __shfl_up(inc, off);
+    if (lane >= off) inc += v;
+  }
+  uint32_t base = 0;
+  if (lane == 63 && inc) base = atomicAdd(counter, inc);
+  return __shfl(base, 63) + inc - m;
+}
+
+template <int T, uint32_t CAP>
+__device__ __forceinline__ void shortlist_body(const ShortlistArgs& a, uint32_t i,
+                                               SelShared<T, CAP>& sm) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t q = a.qidx ? a.qidx[i] : i;  // candidate lists of query q -> output row i
+  const uint2* __restrict__ hdr = a.hdr + (size_t)q * a.NL;
+  const uint2* __restrict__ ent = a.ent + (size_t)q * a.NL * kLowpLC;
+  if (tid == 0) {
+    sm.n = 0;
+    sm.lt = 0;
+    sm.eq = 0;
+  }
+  __syncthreads();
+  // every entry below the LDS capacity, their number, range and the bounds
+  float bmin = INFINITY;
+  uint32_t lo = ~0u, hi = 0u;
+  for (uint32_t l = tid; l < a.NL; l += T) {
+    const uint2 h = hdr[l];
+    sm.cnt[l] = (uint8_t)h.x;
+    bmin = fminf(bmin, __uint_as_float(h.y));
+  }
+  __syncthreads();
+  constexpr int U = 4;
+  const uint32_t quads = a.NL * (kLowpLC / 4);
+  for (uint32_t t0 = 0; t0 < quads; t0 += U * T) {
+    uint32_t m[U], sum = 0;
+    uint4 v[U][2];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t t = t0 + u * T + tid, e0 = (t & 3) * 4;
+      const uint32_t c = t < quads ? sm.cnt[t >> 2] : 0u;
+      m[u] = c > e0 ? min(4u, c - e0) : 0u;
+      sum += m[u];
+      if (m[u]) {
+        const uint4* src = reinterpret_cast<const uint4*>(ent + (size_t)t * 4);
+        v[u][0] = src[0];
+        v[u][1] = src[1];
       }
+    }
+    uint32_t pos = wave_reserve(&sm.n, sum, lane);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t ks[4] = {v[u][0].x, v[u][0].z, v[u][1].x, v[u][1].z};
+      const uint32_t ss[4] = {v[u][0].y, v[u][0].w, v[u][1].y, v[u][1].w};
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        if ((uint32_t)j < m[u]) {
+          const uint32_t kb = rank_bits32(__uint_as_float(ks[j]));
+          lo = min(lo, kb);
+          hi = max(hi, kb);
+          if (pos < CAP) {
+            sm.key[pos] = kb;
+            sm.slot[pos] = ss[j];
+          }
+          pos++;
+        }
     }
   }
   for (int off = 32; off >= 1; off >>= 1) {
-    lmin = fminf(lmin, __shfl_xor(lmin, off));
-    nv += __shfl_xor(nv, off);
+    bmin = fminf(bmin, __shfl_xor(bmin, off));
+    lo = min(lo, (uint32_t)__shfl_xor((int)lo, off));
+    hi = max(hi, (uint32_t)__shfl_xor((int)hi, off));
   }
-  if (tid == 0) {
-    s_prefix = 0;
-    s_mask = 0;
-    s_rank = a.L;
-    s_nvalid = 0;
-    s_lt = 0;
-    s_eq = 0;
-  }
-  __syncthreads();
   if (lane == 0) {
-    s_min[wave] = lmin;
-    atomicAdd(&s_nvalid, nv);
+    sm.wmin[wave] = bmin;
+    sm.wlo[wave] = lo;
+    sm.whi[wave] = hi;
   }
   __syncthreads();
-  const uint32_t nvalid = s_nvalid;
-  lmin = fminf(fminf(s_min[0], s_min[1]), fminf(s_min[2], s_min[3]));
-  uint32_t kstar = 0xFFFFFFFFu;  // fewer than L valid entries: take them all
-  if (nvalid >= a.L) {
-    for (int pass = 0; pass < 4; pass++) {
-      const int shift = 24 - 8 * pass;
-      hist[tid] = 0;
+  const uint32_t n = sm.n;
+  if (tid == 0) {
+    for (int w = 1; w < T / 64; w++) {
+      lo = min(lo, sm.wlo[w]);
+      hi = max(hi, sm.whi[w]);
+      bmin = fminf(bmin, sm.wmin[w]);
+    }
+    sm.lo = lo;
+    sm.hi = hi;
+    sm.rank = a.L;
+  }
+  // f(key bits, slot) for every entry
+  auto each = [&](auto&& f) __attribute__((always_inline)) {
+    if (n <= CAP) {
+      for (uint32_t c = tid; c < n; c += T) f(sm.key[c], sm.slot[c]);
+      return;
+    }
+    for (uint32_t l = tid; l < a.NL; l += T) {
+      const uint32_t m = sm.cnt[l];
+      for (uint32_t e = 0; e < m; e++) {
+        const uint2 v = ent[(size_t)l * kLowpLC + e];
+        f(rank_bits32(__uint_as_float(v.x)), v.y);
+      }
+    }
+  };
+  __syncthreads();
+  if (n > a.L) {
+    for (;;) {
+      // the L-th smallest key is the sm.rank-th of those in [l, h]
+      const uint32_t l = sm.lo, h = sm.hi;
+      if (l == h) break;
+      const uint32_t w = h - l;
+      const int shift = max(0, 24 - __clz((int)w));
+      for (int b = tid; b < 256; b += T) sm.hist[b] = 0;
       __syncthreads();
-      const uint32_t prefix = s_prefix, mask = s_mask;
-#pragma unroll
-      for (int t = 0; t < kSelPT; t++)
-        if (u[t] != 0xFFFFFFFFu && (u[t] & mask) == prefix)
-          atomicAdd(&hist[(u[t] >> shift) & 255u], 1u);
+      each([&](uint32_t k, uint32_t) {
+        if (k >= l && k <= h) atomicAdd(&sm.hist[(k - l) >> shift], 1u);
+      });
       __syncthreads();
       if (wave == 0) {
-        // lane l holds bins 4l..4l+3; an inclusive scan over lanes finds
+        // lane b holds bins 4b..4b+3; an inclusive scan over lanes finds
         // the bin where the running count reaches the target rank
-        const uint32_t h0 = hist[4 * lane], h1 = hist[4 * lane + 1], h2 = hist[4 * lane + 2],
-                       h3 = hist[4 * lane + 3];
-        const uint32_t sum = h0 + h1 + h2 + h3;
+        const uint32_t hs[4] = {sm.hist[4 * lane], sm.hist[4 * lane + 1], sm.hist[4 * lane + 2],
+                                sm.hist[4 * lane + 3]};
+        const uint32_t sum = hs[0] + hs[1] + hs[2] + hs[3];
         uint32_t inc = sum;
         for (int off = 1; off < 64; off <<= 1) {
           const uint32_t v = __shfl_up(inc, off);
           if (lane >= off) inc += v;
         }
-        const uint32_t exc = inc - sum, rank = s_rank;
+        const uint32_t exc = inc - sum, rank = sm.rank;
         if (exc < rank && rank <= inc) {
           uint32_t cum = exc, bin = 4 * lane;
-          const uint32_t hs[4] = {h0, h1, h2, h3};
-          for (int b = 0; b < 4; b++) {
-            if (cum + hs[b] >= rank) {
-              bin = 4 * lane + b;
-              break;
+#pragma unroll
+          for (int b = 0; b < 3; b++)
+            if (bin == 4u * lane + b && cum + hs[b] < rank) {
+              cum += hs[b];
+              bin++;
             }
-            cum += hs[b];
-          }
-          s_rank = rank - cum;
-          s_prefix = prefix | (bin << shift);
-          s_mask = mask | (255u << shift);
+          sm.rank = rank - cum;
+          sm.lo = l + (bin << shift);
+          sm.hi = min(h, l + (bin << shift) + ((1u << shift) - 1u));
         }
       }
       __syncthreads();
     }
-    kstar = s_prefix;
   }
-  // entries below K*: all of them; equal to K*: the first s_rank that come
-  const uint32_t need_eq = nvalid >= a.L ? s_rank : 0u;
-  const uint32_t n_lt = nvalid >= a.L ? a.L - need_eq : 0u;
-#pragma unroll
-  for (int t = 0; t < kSelPT; t++) {
-    if (u[t] == 0xFFFFFFFFu) continue;
+  // entries below the L-th key: all of them; equal to it: the first that
+  // come, as many as are needed
+  const bool all = n <= a.L;
+  const uint32_t kstar = all ? ~0u : sm.lo;
+  const uint32_t need_eq = all ? 0u : sm.rank;
+  const uint32_t n_lt = all ? 0u : a.L - need_eq;
+  each([&](uint32_t k, uint32_t slot) {
     uint32_t pos = ~0u;
-    if (nvalid < a.L || u[t] < kstar) {
-      pos = atomicAdd(&s_lt, 1u);
-    } else if (u[t] == kstar) {
-      const uint32_t e = atomicAdd(&s_eq, 1u);
+    if (all || k < kstar) {
+      pos = atomicAdd(&sm.lt, 1u);
+    } else if (k == kstar) {
+      const uint32_t e = atomicAdd(&sm.eq, 1u);
       if (e < need_eq) pos = n_lt + e;
     }
     if (pos != ~0u) {
-      const uint32_t c = t * 256 + tid;
-      a.short_slot[(size_t)i * a.L + pos] = a.cand_slot[base + c];
-      a.short_key[(size_t)i * a.L + pos] = a.cand_key[base + c];
+      a.short_slot[(size_t)i * a.L + pos] = slot;
+      a.short_key[(size_t)i * a.L + pos] = rank_float32(k);
     }
-  }
-  __syncthreads();
-  // unused tail (fewer than L valid entries)
-  for (uint32_t e = (nvalid < a.L ? nvalid : a.L) + tid; e < a.L; e += 256) {
+  });
+  // unused tail (fewer than L entries)
+  for (uint32_t e = n + tid; e < a.L; e += T) {
     a.short_slot[(size_t)i * a.L + e] = ~0u;
     a.short_key[(size_t)i * a.L + e] = INFINITY;
   }
-  if (tid == 0) {
-    const float oL =
-        nvalid >= a.L ? __uint_as_float((kstar >> 31) ? (kstar & 0x7FFFFFFFu) : ~kstar) : INFINITY;
-    a.beta[i] = fminf(lmin, oL);
-  }
+  if (tid == 0) a.beta[i] = n >= a.L ? fminf(bmin, rank_float32(all ? hi : kstar)) : bmin;
 }
 
 // Several ranges' shortlists (or reranks) in one launch: range r takes
@@ -531,53 +533,39 @@ __device__ __forceinline__ int range_of(const RangeBatch<A>& b, uint32_t blk) {
   return i;
 }
 
-template <int KPL>
-__global__ __launch_bounds__(256) void k_shortlist(RangeBatch<ShortlistArgs> b) {
+template <int T, uint32_t CAP>
+__global__ __launch_bounds__(T) void k_shortlist(RangeBatch<ShortlistArgs> b) {
+  __shared__ SelShared<T, CAP> sm;
   const int i = range_of(b, blockIdx.x);
-  shortlist_body<KPL>(b.r[i], blockIdx.x - b.first[i]);
+  shortlist_body<T, CAP>(b.r[i], blockIdx.x - b.first[i], sm);
 }
 
-__global__ __launch_bounds__(256) void k_shortlist_sel(RangeBatch<ShortlistArgs> b) {
-  __shared__ SelShared sm;
-  const int i = range_of(b, blockIdx.x);
-  shortlist_sel_body(b.r[i], blockIdx.x - b.first[i], sm);
-}
-
-// Up to 64 wide: one wavefront per query keeps a sorted list (few
-// insertions past the first 64).  Wider: the block-per-query select, whose
-// cost does not grow with L (a 256-wide sorted list in one wavefront takes
-// hundreds of serial insertions per query); the sorted 256-wide form
-// remains for candidate sets too large for its registers.
-static int shortlist_variant(const ShortlistArgs& a) {
-  const bool sel_fits = (size_t)a.NL * kLowpLP <= 256u * kSelPT;
-  if (a.L == 0 || a.L > (uint32_t)kMaxShort) return -1;
-  if (a.L <= 64) return 1;
-  if (sel_fits) return 0;
-  if (a.L <= 256) return 4;
-  return -1;
-}
-
+// Up to 256 queries (one block per CU or fewer) a block takes 1,024 threads, so
+// that the headers of the many lists such batches have are read in a few
+// rounds; beyond, 256 threads, and 8 queries a CU at once.
 hipError_t launch_shortlist_ranges(const ShortlistArgs* a, int n, hipStream_t s) {
-  for (int r0 = 0; r0 < n;) {
-    // one launch per run of ranges that take the same kernel
+  for (int r0 = 0; r0 < n; r0 += kMaxLaunchRanges) {
     RangeBatch<ShortlistArgs> b{};
-    const int v = shortlist_variant(a[r0]);
-    if (v < 0) return hipErrorInvalidValue;
     uint32_t blocks = 0;
+    bool narrow = true;
     b.n = 0;
-    int r = r0;
-    for (; r < n && b.n < kMaxLaunchRanges && shortlist_variant(a[r]) == v; r++) {
+    for (int r = r0; r < n && b.n < kMaxLaunchRanges; r++) {
+      if (a[r].L == 0 || a[r].L > (uint32_t)kMaxShort || a[r].NL > kSelLists)
+        return hipErrorInvalidValue;
+      narrow &= a[r].L <= 64;
       b.r[b.n] = a[r];
       b.first[b.n] = blocks;
-      blocks += v == 0 ? a[r].nq : (a[r].nq + 3) / 4;
+      blocks += a[r].nq;
       b.n++;
     }
     b.first[b.n] = blocks;
-    r0 = r;
     if (blocks == 0) continue;
-    if (v == 1) hipLaunchKernelGGL(k_shortlist<1>, dim3(blocks), dim3(256), 0, s, b);
-    else if (v == 4) hipLaunchKernelGGL(k_shortlist<4>, dim3(blocks), dim3(256), 0, s, b);
-    else hipLaunchKernelGGL(k_shortlist_sel, dim3(blocks), dim3(256), 0, s, b);
+    if (blocks <= 256)
+      hipLaunchKernelGGL((k_shortlist<1024, 4096>), dim3(blocks), dim3(1024), 0, s, b);
+    else if (narrow)
+      hipLaunchKernelGGL((k_shortlist<256, 2048>), dim3(blocks), dim3(256), 0, s, b);
+    else
+      hipLaunchKernelGGL((k_shortlist<256, 4096>), dim3(blocks), dim3(256), 0, s, b);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

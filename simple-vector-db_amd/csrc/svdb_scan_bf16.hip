@@ -10,11 +10,11 @@
 // 16-row A-operand reads hit distinct banks.  Per 16-row subtile a lane
 // gets 4 scores per fragment — rows 4*(lane/16)+r, query lane%16 — and its
 // fp32 ordering key is one FMA of the score and a per-row value.  Keys below
-// the lane's current 8th best enter the lane's private sorted list (an
-// insertion into 8 registers); each list is one candidate list of its
-// query and its 8th entry bounds every row the lane left out.  Subtiles are
+// the lane's bound for the query enter the lane's private candidate list
+// (svdb_cand.h).  Subtiles are
 // software-pipelined: subtile s+1's MFMAs are issued before subtile s's
 // epilogue, whose per-row values were read into registers beforehand.
+#include "svdb_cand.h"
 #include "svdb_lowp.h"
 
 #include <math.h>
@@ -70,15 +70,16 @@ __device__ __forceinline__ void issue_tile(const LowpScanArgs& a, unsigned char*
   }
 }
 
-// MINONLY: each lane keeps only the smallest key of its rows (one list
-// entry, cand_key[q * NL + list]); the sample pre-pass uses it to bound the
-// L-th key cheaply.
+// FORM kFormMin: each lane keeps only the smallest key of its rows
+// (cand_key[q * NL + list]); the sample pre-pass uses it to find a threshold
+// cheaply.  kFormAppend needs a.tau0.
 // METRIC kMixed: each wavefront's queries share one metric (QParams.metric
 // of its first slot; the engine aligns metric ranges to wavefronts), read at
 // run time; the tile then carries all four per-row arrays.
-template <int METRIC, int KS, int QF, bool MINONLY>
+template <int METRIC, int KS, int QF, int FORM>
 __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
   constexpr bool MIXED = METRIC == kMixed;
+  constexpr bool MINONLY = FORM == kFormMin, SORTED = FORM == kFormSorted;
   constexpr int NAUX = MIXED ? 4 : (METRIC == kCos ? 2 : 1);
   using G = TileGeom<KS, NAUX < 2 ? 2 : NAUX>;
   __shared__ __attribute__((aligned(16))) unsigned char buf0[G::BUF_B];
@@ -110,8 +111,9 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
 
   bf16x8 B[QF][KS];
   float P[QF], tau[QF];
-  float lk[QF][LP];
-  uint32_t ls[QF][LP];
+  float lk[SORTED ? QF : 1][LP];     // kFormSorted
+  uint32_t ls[SORTED ? QF : 1][LP];
+  uint32_t cnt[QF];                  // kFormAppend
 #pragma unroll
   for (int f = 0; f < QF; f++) {
     const uint32_t q = qbase + f * 16 + ql;  // < nq_pad (Qb is padded)
@@ -132,10 +134,13 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
       }
     }
     tau[f] = MINONLY ? INFINITY : t0;
+    cnt[f] = 0;
+    if constexpr (SORTED) {
 #pragma unroll
-    for (int j = 0; j < LP; j++) {
-      lk[f][j] = t0;
-      ls[f][j] = ~0u;
+      for (int j = 0; j < LP; j++) {
+        lk[f][j] = t0;
+        ls[f][j] = ~0u;
+      }
     }
   }
 
@@ -157,8 +162,9 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
     return MIXED ? fmaf(wcos ? acc[f][r] : P[f], wv[r], wcos ? pv[r] : acc[f][r])
                  : (COS ? fmaf(acc[f][r], wv[r], pv[r]) : fmaf(P[f], wv[r], acc[f][r]));
   };
+  const uint32_t list = slice * kLowpLanesPerQuery + rg;
   // One test per subtile for all fragments: in the common case no key
-  // beats its list's 8th entry and the insertion code is skipped with a
+  // is below its list's bound and the insertion code is skipped with a
   // single branch; the rare insertion path recomputes the keys.
   auto need_of = [&](const f32x4 (&acc)[QF], const float (&wv)[4], const float (&pv)[4]) {
     bool need = false;
@@ -188,24 +194,29 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
       for (int r = 0; r < 4; r++) k4[r] = key(acc, f, r, wv, pv);
       const float mn = fminf(fminf(k4[0], k4[1]), fminf(k4[2], k4[3]));
       if (mn < tau[f]) {
+        if constexpr (!SORTED) {
+          cand_append4(a.ent + cand_list(a, qbase + f * 16 + ql, list) * kLowpLC, cnt[f], tau[f],
+                       k4, srow);
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          if (k4[r] < lk[f][LP - 1]) {
-            lk[f][LP - 1] = k4[r];
-            ls[f][LP - 1] = srow + r;
+          for (int r = 0; r < 4; r++) {
+            if (k4[r] < lk[f][LP - 1]) {
+              lk[f][LP - 1] = k4[r];
+              ls[f][LP - 1] = srow + r;
 #pragma unroll
-            for (int j = LP - 1; j > 0; j--) {
-              const bool sw = lk[f][j] < lk[f][j - 1];
-              const float tk = sw ? lk[f][j - 1] : lk[f][j];
-              const uint32_t tsl = sw ? ls[f][j - 1] : ls[f][j];
-              lk[f][j - 1] = sw ? lk[f][j] : lk[f][j - 1];
-              ls[f][j - 1] = sw ? ls[f][j] : ls[f][j - 1];
-              lk[f][j] = tk;
-              ls[f][j] = tsl;
+              for (int j = LP - 1; j > 0; j--) {
+                const bool sw = lk[f][j] < lk[f][j - 1];
+                const float tk = sw ? lk[f][j - 1] : lk[f][j];
+                const uint32_t tsl = sw ? ls[f][j - 1] : ls[f][j];
+                lk[f][j - 1] = sw ? lk[f][j] : lk[f][j - 1];
+                ls[f][j - 1] = sw ? ls[f][j] : ls[f][j - 1];
+                lk[f][j] = tk;
+                ls[f][j] = tsl;
+              }
             }
           }
+          tau[f] = lk[f][LP - 1];
         }
-        tau[f] = lk[f][LP - 1];
       }
     }
   };
@@ -296,6 +307,7 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
           }
 #pragma unroll
           for (int f = 0; f < QF; f++) pacc[f] = acc[f];
+          if (sub == kLowpTile / 16 - 1) settle_mfma(pacc[QF - 1]);
           pw = w;
           ppen = pen;
           prow = trow + rl;
@@ -326,6 +338,9 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
 #pragma unroll
             for (int f = 0; f < QF; f++)
               acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[ks], B[f][ks], acc[f], 0, 0, 0);
+            // (the previous subtile's test stays behind the first MFMAs:
+            // settle_mfma)
+            if (!LATE && ks == 0) __builtin_amdgcn_sched_barrier(0);
             if (LATE && ks == 0) {
               __builtin_amdgcn_sched_barrier(0);
               w = *reinterpret_cast<const float4*>(aux + warr * kLowpTile + rl);
@@ -345,6 +360,7 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
           }
 #pragma unroll
           for (int f = 0; f < QF; f++) pacc[f] = acc[f];
+          if (sub == kLowpTile / 16 - 1) settle_mfma(pacc[QF - 1]);
           pw = w;
           ppen = pen;
           prow = trow + rl;
@@ -356,21 +372,13 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
   }
   epilogue(pacc, pw, ppen, prow);
 
-  const uint32_t list = slice * kLowpLanesPerQuery + rg;
 #pragma unroll
   for (int f = 0; f < QF; f++) {
     const uint32_t q = qbase + f * 16 + ql;
     if (q >= a.nq) continue;
-    if constexpr (MINONLY) {
-      a.cand_key[(size_t)q * a.NL + list] = tau[f];
-      continue;
-    }
-    const size_t o = ((size_t)q * a.NL + list) * LP;
-#pragma unroll
-    for (int j = 0; j < LP; j++) {
-      a.cand_key[o + j] = lk[f][j];
-      a.cand_slot[o + j] = ls[f][j];
-    }
+    if constexpr (MINONLY) a.cand_key[cand_list(a, q, list)] = tau[f];
+    else if constexpr (SORTED) cand_store_sorted(a, cand_list(a, q, list), lk[f], ls[f]);
+    else a.hdr[cand_list(a, q, list)] = make_uint2(cnt[f], __float_as_uint(tau[f]));
   }
 }
 
@@ -382,9 +390,10 @@ static hipError_t scan_bf16_t(const LowpScanArgs& a, uint32_t nslices, bool mino
   if constexpr (METRIC == kMixed) {
     if (minonly) return hipErrorInvalidValue;
   }
-  auto fn = k_scan_bf16<METRIC, KS, QF, false>;
+  auto fn = a.tau0 ? k_scan_bf16<METRIC, KS, QF, kFormAppend>
+                   : k_scan_bf16<METRIC, KS, QF, kFormSorted>;
   if constexpr (METRIC != kMixed)
-    if (minonly) fn = k_scan_bf16<METRIC, KS, QF, true>;
+    if (minonly) fn = k_scan_bf16<METRIC, KS, QF, kFormMin>;
   constexpr size_t shm = 0;  // both tile buffers are static LDS
   const uint32_t qpb = kLowpWaves * QF * 16;
   // nslices is a multiple of 8 (one set of slices per XCD); 1-D grid.

@@ -10,7 +10,7 @@
 //
 // Scan (k_scan_wide): queries held as B operands, row tiles streamed
 // direct-to-LDS into two static buffers, XCD owning whole slices, per-lane
-// 8-entry sorted lists, a branch-free per-fragment test among the next
+// candidate lists (svdb_cand.h), a branch-free per-fragment test among the next
 // subtile's MFMAs and one rare wave-uniform insertion branch, with
 // v_mfma_scale_f32_16x16x128_f8f6f4 (unit E8M0 scales): lane l supplies
 // row (or query) l%16, bytes k = 32·(l/16) .. +31 of each 128-byte K step;
@@ -19,6 +19,7 @@
 //   cosine:         O = fma(acc·sq, sx/‖x‖, pen)
 // Both equal the BF16-form key divided by sq (Euclidean, dot) or equal it
 // (cosine) exactly; QParams.scale carries sq back.
+#include "svdb_cand.h"
 #include "svdb_lowp.h"
 
 #include <math.h>
@@ -334,13 +335,14 @@ __device__ __forceinline__ void issue_tile8(const LowpScanArgs& a, unsigned char
 // each 32-element half; one-FMA keys as in k_scan_bf16); else FP8.
 // NW = 4 (one wavefront per SIMD) leaves each wavefront 512 registers, for
 // the 192-register query fragment of a 1536-wide BF16 row.
-template <int METRIC, int KS, int QF, bool MINONLY, bool BF, int NW>
+template <int METRIC, int KS, int QF, int FORM, bool BF, int NW>
 __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
   using G = Geom8<KS, NW>;
   __shared__ __attribute__((aligned(16))) unsigned char buf0[G::BUF_B];
   __shared__ __attribute__((aligned(16))) unsigned char buf1[G::BUF_B];
   constexpr int LP = kLowpLP;
   constexpr bool COS = METRIC == kCos;
+  constexpr bool MINONLY = FORM == kFormMin, SORTED = FORM == kFormSorted;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -360,8 +362,9 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
   // pieces at 128·ks + 16·rg and 128·ks + 64 + 16·rg
   i32x8 B[QF][KS];
   float P[QF], tau[QF];
-  float lk[QF][LP];
-  uint32_t ls[QF][LP];
+  float lk[SORTED ? QF : 1][LP];     // kFormSorted
+  uint32_t ls[SORTED ? QF : 1][LP];
+  uint32_t cnt[QF];                  // kFormAppend
 #pragma unroll
   for (int f = 0; f < QF; f++) {
     const uint32_t q = qbase + f * 16 + ql;  // < nq_pad (Q8 is padded)
@@ -387,12 +390,16 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
       }
     }
     tau[f] = MINONLY ? INFINITY : t0;
+    cnt[f] = 0;
+    if constexpr (SORTED) {
 #pragma unroll
-    for (int j = 0; j < LP; j++) {
-      lk[f][j] = t0;
-      ls[f][j] = ~0u;
+      for (int j = 0; j < LP; j++) {
+        lk[f][j] = t0;
+        ls[f][j] = ~0u;
+      }
     }
   }
+  const uint32_t list = slice * kLowpLanesPerQuery + rg;
 
   auto key = [&](const f32x4 (&acc)[QF], int f, int r, const float4& w0, const float4& w1) {
     const float v0 = r == 0 ? w0.x : r == 1 ? w0.y : r == 2 ? w0.z : w0.w;
@@ -400,8 +407,8 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
     return BF ? (COS ? fmaf(acc[f][r], v0, v1) : fmaf(P[f], v0, acc[f][r]))
               : (COS ? fmaf(acc[f][r] * P[f], v0, v1) : fmaf(P[f], v0, acc[f][r] * v1));
   };
-  // Fragment f's common-case test: does any of its four keys beat the
-  // list's last entry?  Branch-free VALU work, issued among the next
+  // Fragment f's common-case test: is any of its four keys below the
+  // list's bound?  Branch-free VALU work, issued among the next
   // subtile's MFMAs (the minimum-only pre-pass folds its keys here).
   auto need_of = [&](const f32x4 (&acc)[QF], int f, const float4& w0, const float4& w1) {
     const float mn = fminf(fminf(key(acc, f, 0, w0, w1), key(acc, f, 1, w0, w1)),
@@ -422,24 +429,29 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
       for (int r = 0; r < 4; r++) k4[r] = key(acc, f, r, w0, w1);
       const float mn = fminf(fminf(k4[0], k4[1]), fminf(k4[2], k4[3]));
       if (mn < tau[f]) {
+        if constexpr (!SORTED) {
+          cand_append4(a.ent + cand_list(a, qbase + f * 16 + ql, list) * kLowpLC, cnt[f], tau[f],
+                       k4, srow);
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          if (k4[r] < lk[f][LP - 1]) {
-            lk[f][LP - 1] = k4[r];
-            ls[f][LP - 1] = srow + r;
+          for (int r = 0; r < 4; r++) {
+            if (k4[r] < lk[f][LP - 1]) {
+              lk[f][LP - 1] = k4[r];
+              ls[f][LP - 1] = srow + r;
 #pragma unroll
-            for (int j = LP - 1; j > 0; j--) {
-              const bool sw = lk[f][j] < lk[f][j - 1];
-              const float tk = sw ? lk[f][j - 1] : lk[f][j];
-              const uint32_t tsl = sw ? ls[f][j - 1] : ls[f][j];
-              lk[f][j - 1] = sw ? lk[f][j] : lk[f][j - 1];
-              ls[f][j - 1] = sw ? ls[f][j] : ls[f][j - 1];
-              lk[f][j] = tk;
-              ls[f][j] = tsl;
+              for (int j = LP - 1; j > 0; j--) {
+                const bool sw = lk[f][j] < lk[f][j - 1];
+                const float tk = sw ? lk[f][j - 1] : lk[f][j];
+                const uint32_t tsl = sw ? ls[f][j - 1] : ls[f][j];
+                lk[f][j - 1] = sw ? lk[f][j] : lk[f][j - 1];
+                ls[f][j - 1] = sw ? ls[f][j] : ls[f][j - 1];
+                lk[f][j] = tk;
+                ls[f][j] = tsl;
+              }
             }
           }
+          tau[f] = lk[f][LP - 1];
         }
-        tau[f] = lk[f][LP - 1];
       }
     }
   };
@@ -503,8 +515,9 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
         f32x4 acc[QF];
 #pragma unroll
         for (int f = 0; f < QF; f++) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // The previous subtile's test, one fragment per K step (the rest at
-        // the last step): VALU work in the same basic block as this
+        // The previous subtile's test, one fragment per K step from the second
+        // on (settle_mfma says why not the first; the rest at the last step):
+        // VALU work in the same basic block as this
         // subtile's MFMAs, issued between them — with one wavefront per
         // SIMD nothing else would fill the matrix core meanwhile.  One
         // wave-uniform, unlikely branch after the last step takes the rare
@@ -530,7 +543,7 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
           }
 #pragma unroll
           for (int f = 0; f < QF; f++)
-            if (f == ks || (ks == KS - 1 && f > ks)) need |= need_of(pacc, f, pw0, pw1);
+            if (f + 1 == ks || (ks == KS - 1 && f + 1 > ks)) need |= need_of(pacc, f, pw0, pw1);
           const int nx = sub * KS + ks + 2;
           if (nx < NSUB * KS) Ab[ks & 1] = loadA((nx / KS) * 16 + ql, nx % KS);
           // one MFMA, then up to four VALU instructions, and so on
@@ -546,6 +559,7 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
         const int rl = sub * 16 + rg * 4;
 #pragma unroll
         for (int f = 0; f < QF; f++) pacc[f] = acc[f];
+        if (sub == NSUB - 1) settle_mfma(pacc[QF - 1]);
         pw0 = *reinterpret_cast<const float4*>(aux + rl);
         pw1 = *reinterpret_cast<const float4*>(aux + G::TR + rl);
         prow = trow + rl;
@@ -555,29 +569,22 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
     }
   }
   if (active) epilogue(pacc, pw0, pw1, prow);
-  const uint32_t list = slice * kLowpLanesPerQuery + rg;
 #pragma unroll
   for (int f = 0; f < QF; f++) {
     const uint32_t q = qbase + f * 16 + ql;
     if (q >= a.nq) continue;
-    if constexpr (MINONLY) {
-      a.cand_key[(size_t)q * a.NL + list] = tau[f];
-      continue;
-    }
-    const size_t o = ((size_t)q * a.NL + list) * LP;
-#pragma unroll
-    for (int j = 0; j < LP; j++) {
-      a.cand_key[o + j] = lk[f][j];
-      a.cand_slot[o + j] = ls[f][j];
-    }
+    if constexpr (MINONLY) a.cand_key[cand_list(a, q, list)] = tau[f];
+    else if constexpr (SORTED) cand_store_sorted(a, cand_list(a, q, list), lk[f], ls[f]);
+    else a.hdr[cand_list(a, q, list)] = make_uint2(cnt[f], __float_as_uint(tau[f]));
   }
 }
 
 template <int METRIC, int KS, int QF, bool BF = false, int NW = kLowpWaves>
 static hipError_t scan_fp8_t(const LowpScanArgs& a, uint32_t nslices, bool minonly,
                              hipStream_t s) {
-  auto fn = minonly ? k_scan_wide<METRIC, KS, QF, true, BF, NW>
-                    : k_scan_wide<METRIC, KS, QF, false, BF, NW>;
+  auto fn = minonly  ? k_scan_wide<METRIC, KS, QF, kFormMin, BF, NW>
+            : a.tau0 ? k_scan_wide<METRIC, KS, QF, kFormAppend, BF, NW>
+                     : k_scan_wide<METRIC, KS, QF, kFormSorted, BF, NW>;
   const uint32_t qpb = NW * QF * 16;
   // nslices is a multiple of 8 (one set of slices per XCD); rows per slice
   // and the slice stride are multiples of the 128-row slot granularity.

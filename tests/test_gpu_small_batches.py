@@ -68,3 +68,33 @@ def test_rerank_shapes(n, d, nq, k, short):
     for metric in ("l2", "cos", "dot"):
         check(db, X, Q, k, metric, "bf16")
     db.close()
+
+
+@pytest.mark.parametrize("d,nq", [(30, 70), (64, 5), (128, 600), (129, 130), (256, 300),
+                                  (500, 40), (768, 130), (1536, 70)])
+def test_thresholded_lists(d, nq):
+    """Row and query counts over which the first pass starts from a sample's
+    threshold, every padded width, ragged last tile; k on both sides of the
+    wider shortlist.  A third of the rows are one cluster stored in a row, so
+    that the lists of the slices it lies in fill up."""
+    rng = np.random.default_rng(d)
+    n = 20_011
+    X = rng.standard_normal((n, d))
+    X[5000:5000 + n // 3] = X[0] + 0.05 * rng.standard_normal((n // 3, d))
+    Q = np.vstack([X[0] + 0.05 * rng.standard_normal((nq // 2, d)),
+                   rng.standard_normal((nq - nq // 2, d))])
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    for metric in ("l2", "cos", "dot"):
+        for k in (10, 40):
+            check(db, X, Q, k, metric, "bf16")
+    if d <= 256:
+        ids, sc = db.search(Q, 10, [("l2", "cos", "dot")[i % 3] for i in range(nq)], "bf16")
+        for j, metric in enumerate(("l2", "cos", "dot")):
+            rid, rsc = O.topk(X, Q[j::3], 10, metric)
+            assert np.array_equal(ids[j::3], rid) and np.array_equal(sc[j::3], rsc), metric
+    if d >= 500:
+        db.enable_shadow("fp8")
+        for metric in ("l2", "cos", "dot"):
+            check(db, X, Q, 10, metric, "fp8")
+    db.close()
