@@ -886,54 +886,86 @@ uint32_t Engine::exact_slices(uint32_t nq, int kmax, size_t max_entries) const {
   return (uint32_t)nslices;
 }
 
+// The partial lists of an exact scan within max_entries: on the matrix cores
+// from scan_f64_lists, on the VALU nslices · kWavesPerBlock sorted lists of
+// kmax entries.  ok = false when exact_slices refuses the size (in either
+// form, so that what is accepted does not depend on the path).
+Engine::ExactPlan Engine::exact_plan(int metric, uint32_t nq, uint32_t D, int kmax,
+                                     size_t max_entries) const {
+  ExactPlan p{};
+  p.nslices = exact_slices(nq, kmax, max_entries);
+  p.ok = nphys_ == 0 || p.nslices != 0;
+  StoreView sv{X_, ld_, xn_, alive_, rank_, (uint32_t)nphys_, has_deletes_ ? 1 : 0,
+               D == d_ ? nx2_ : nullptr};
+  p.mfma = scan_f64_uses_mfma(metric, D, sv);
+  if (p.mfma) {
+    // (64 entries are left for the arrays' alignment)
+    const F64Lists l = scan_f64_lists((uint32_t)nphys_, nq, kmax, max_entries - 64);
+    p.P = l.P;
+    p.stride = l.cap;
+  } else {
+    p.P = p.nslices * kWavesPerBlock;
+    p.stride = (uint32_t)kmax;
+  }
+  p.entries = (size_t)nq * p.P * p.stride;
+  return p;
+}
+
 int Engine::run_exact(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, const int* dk,
                       int metric, int kmax, uint64_t* dids, double* dscores, uint32_t ostride) {
   int rc;
   if (nq == 0) return SVDB_OK;
   // partial lists stay under 2^25 entries (~400 MB)
-  const uint32_t nslices = exact_slices(nq, kmax, std::max<size_t>((size_t)1 << 25,
-                                                                    (size_t)nq * 32 * kmax));
-  const size_t nlist = (size_t)nq * nslices * kWavesPerBlock * kmax;
-  if ((rc = scratch(&c_->s_pk_, &c_->s_pk_n_, std::max<size_t>(nlist, 1) * sizeof(uint64_t)))) return rc;
-  if ((rc = scratch(&c_->s_ps_, &c_->s_ps_n_, std::max<size_t>(nlist, 1) * sizeof(uint32_t)))) return rc;
-  if ((rc = scratch(&c_->s_qn_, &c_->s_qn_n_, (size_t)nq * 3 * sizeof(double)))) return rc;
-  return run_exact_with(dQ, ldq, nq, D, dk, metric, kmax, dids, dscores, ostride, nslices,
+  const ExactPlan p = exact_plan(metric, nq, D, kmax,
+                                 std::max<size_t>((size_t)1 << 25, (size_t)nq * 32 * kmax));
+  const size_t n = std::max<size_t>(p.entries, 1);
+  if ((rc = scratch(&c_->s_pk_, &c_->s_pk_n_, n * sizeof(uint64_t)))) return rc;
+  if ((rc = scratch(&c_->s_ps_, &c_->s_ps_n_, n * sizeof(uint32_t)))) return rc;
+  if ((rc = scratch(&c_->s_qn_, &c_->s_qn_n_, exact_aux_bytes(nq, p)))) return rc;
+  return run_exact_with(dQ, ldq, nq, D, dk, metric, kmax, dids, dscores, ostride, p,
                         (uint64_t*)c_->s_pk_, (uint32_t*)c_->s_ps_, (double*)c_->s_qn_);
 }
 
-// The exact scan and merge into caller-provided scratch: partial lists
-// pk / ps of nq × nslices × kWavesPerBlock × kmax entries, and 3·nq
-// doubles at qn: the query norms, their squares as fma chains, and the
-// per-query global bounds of the scan (ScanF64Args.qq, .gtk).  Allocates
-// nothing.
+// Bytes at run_exact_with's qn: per query the norm, its square and the scan's
+// global bound, then (matrix cores) a count per partial list.
+size_t Engine::exact_aux_bytes(uint32_t nq, const ExactPlan& p) {
+  return (size_t)nq * 3 * sizeof(double) + (p.mfma ? (size_t)nq * p.P * sizeof(uint32_t) : 0);
+}
+
+// The exact scan and merge into caller-provided scratch: the plan's partial
+// lists pk / ps and exact_aux_bytes at qn.  Allocates nothing.
 int Engine::run_exact_with(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, const int* dk,
                            int metric, int kmax, uint64_t* dids, double* dscores,
-                           uint32_t ostride, uint32_t nslices, uint64_t* pk, uint32_t* ps,
+                           uint32_t ostride, const ExactPlan& p, uint64_t* pk, uint32_t* ps,
                            double* qn) {
   int rc;
   if (nq == 0) return SVDB_OK;
   // the squared row norms cover every column: usable when the scan does
   StoreView sv{X_, ld_, xn_, alive_, rank_, (uint32_t)nphys_, has_deletes_ ? 1 : 0,
                D == d_ ? nx2_ : nullptr};
-  const uint32_t rps = nslices ? (uint32_t)((nphys_ + nslices - 1) / nslices) : 0;
-  const uint32_t P = scan_f64_lists(metric, D, sv, kmax, nq, nslices);
-  const bool mfma = scan_f64_uses_mfma(metric, D, sv, kmax, nq);
+  const uint32_t rps = p.nslices ? (uint32_t)((nphys_ + p.nslices - 1) / p.nslices) : 0;
   double* qq = qn + nq;
   uint64_t* gtk = reinterpret_cast<uint64_t*>(qn + 2 * (size_t)nq);
+  uint32_t* cnt = reinterpret_cast<uint32_t*>(gtk + nq);
   if ((rc = sync_alive())) return rc;
-  if (metric == kCos || (metric == kL2 && mfma))
+  if (metric == kCos || (metric == kL2 && p.mfma))
     HIPCHK(launch_query_norms(dQ, ldq, nq, D, qn, metric == kL2 ? qq : nullptr, c_->stream),
            "k_query_norms");
-  if (nslices) {
-    HIPCHK(launch_fill_i32(reinterpret_cast<int*>(gtk), 2 * nq, -1, c_->stream), "k_fill_i32");
-    ScanF64Args a{sv, dQ, ldq, qn, dk, nq, D, rps, P, (uint32_t)kmax, pk, ps, gtk, qq};
+  if (p.P) {
+    if (!p.mfma)
+      HIPCHK(launch_fill_i32(reinterpret_cast<int*>(gtk), 2 * nq, -1, c_->stream), "k_fill_i32");
+    ScanF64Args a{sv, dQ, ldq, qn, dk, nq, D, rps, p.P, p.stride, pk, ps, gtk, qq, cnt, rps};
     prof_begin(SVDB_K_SCAN_FP64);
-    HIPCHK(launch_scan_f64(a, metric, kmax, nslices, c_->stream), "k_scan_f64");
+    HIPCHK(p.mfma ? launch_scan_f64_mfma(a, metric, kmax, c_->stream)
+                  : launch_scan_f64(a, kmax, p.nslices, c_->stream),
+           "k_scan_f64");
     prof_end(SVDB_K_SCAN_FP64);
   }
-  MergeArgs m{sv, dk, nq, P, (uint32_t)kmax, pk, ps, ostride, dids, dscores};
+  MergeArgs m{sv, dk, nq, p.P, p.stride, pk, ps, ostride, dids, dscores};
   prof_begin(SVDB_K_MERGE);
-  HIPCHK(launch_merge(m, metric, kmax, c_->stream), "k_merge");
+  HIPCHK(p.mfma ? launch_select_f64(m, cnt, gtk, metric, c_->stream)
+                : launch_merge(m, kmax, c_->stream),
+         "k_merge");
   prof_end(SVDB_K_MERGE);
   return SVDB_OK;
 }
@@ -1578,8 +1610,8 @@ int Engine::search_device_noalloc(const double* dQ, size_t nq, size_t ldq, size_
     return SVDB_EINVAL;
   }
   if (nq == 0) return SVDB_OK;
-  // scratch: k per query | query norms, squared norms, global bounds |
-  // partial keys | partial slots
+  // scratch: k per query | query norms, squared norms, global bounds, entries
+  // per list | partial keys | partial slots
   char* base = static_cast<char*>(scratch);
   const size_t kb = round_up(nq * sizeof(int), 256), qb = round_up(nq * 3 * sizeof(double), 256);
   if (nq > kMaxBatch || kb + qb >= bytes) {
@@ -1587,16 +1619,16 @@ int Engine::search_device_noalloc(const double* dQ, size_t nq, size_t ldq, size_
     return SVDB_EINVAL;
   }
   const size_t entries = (bytes - kb - qb - 256) / (sizeof(uint64_t) + sizeof(uint32_t));
-  const uint32_t nslices = exact_slices((uint32_t)nq, (int)k, entries);
-  if (nphys_ > 0 && nslices == 0) {
+  const ExactPlan p = exact_plan(metric, (uint32_t)nq, (uint32_t)d_, (int)k, entries);
+  if (!p.ok) {
     set_error_static(SVDB_EINVAL, "queries x k too large for the allocation-free scratch");
     return SVDB_EINVAL;
   }
-  const size_t nlist = (size_t)nq * nslices * kWavesPerBlock * k;
+  const size_t aux = round_up(exact_aux_bytes((uint32_t)nq, p), 256);
   int* dk = reinterpret_cast<int*>(base);
   double* qn = reinterpret_cast<double*>(base + kb);
-  uint64_t* pk = reinterpret_cast<uint64_t*>(base + kb + qb);
-  uint32_t* ps = reinterpret_cast<uint32_t*>(base + kb + qb + round_up(nlist * 8, 256));
+  uint64_t* pk = reinterpret_cast<uint64_t*>(base + kb + aux);
+  uint32_t* ps = reinterpret_cast<uint32_t*>(base + kb + aux + round_up(p.entries * 8, 256));
   if (launch_fill_i32(dk, (uint32_t)nq, (int)k, c_->stream) != hipSuccess) {
     set_error_static(SVDB_EDEVICE, "k fill failed");
     return SVDB_EDEVICE;
@@ -1604,7 +1636,7 @@ int Engine::search_device_noalloc(const double* dQ, size_t nq, size_t ldq, size_
   const bool prof = prof_;
   prof_ = false;  // the profiling slots create events
   int rc = run_exact_with(dQ, ldq, (uint32_t)nq, (uint32_t)d_, dk, metric, (int)k, dids, dscores,
-                          (uint32_t)k, nslices, pk, ps, qn);
+                          (uint32_t)k, p, pk, ps, qn);
   prof_ = prof;
   if (rc) return rc;
   if (hipStreamSynchronize(c_->stream) != hipSuccess) {

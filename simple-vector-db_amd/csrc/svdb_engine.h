@@ -148,9 +148,17 @@ class Engine {
   void* host_stage(void** buf, size_t* have, size_t bytes);
   int run_exact(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, const int* dk, int metric,
                 int kmax, uint64_t* dids, double* dscores, uint32_t ostride);
+  struct ExactPlan {
+    bool ok, mfma;
+    uint32_t nslices;    // row slices (VALU)
+    uint32_t P, stride;  // partial lists per query, entries per list
+    size_t entries;      // nq * P * stride
+  };
+  ExactPlan exact_plan(int metric, uint32_t nq, uint32_t D, int kmax, size_t max_entries) const;
+  static size_t exact_aux_bytes(uint32_t nq, const ExactPlan& p);
   int run_exact_with(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, const int* dk,
                      int metric, int kmax, uint64_t* dids, double* dscores, uint32_t ostride,
-                     uint32_t nslices, uint64_t* pk, uint32_t* ps, double* qn);
+                     const ExactPlan& p, uint64_t* pk, uint32_t* ps, double* qn);
   uint32_t exact_slices(uint32_t nq, int kmax, size_t max_entries) const;
   struct LowpRange {
     int metric;

@@ -42,11 +42,13 @@ struct ScanF64Args {
   uint64_t* part_key;       // [nq][P][kstride]
   uint32_t* part_slot;
   // Per query, the smallest k-th rank key any partial list has reached so
-  // far (all ones before the scan; the matrix-core scan lowers it with
-  // atomic min and skips every row whose key is above it), or null.
+  // far (all ones before the scan, lowered with atomic min): rows whose key is
+  // above it are skipped.
   uint64_t* gtk;
   const double* qq;         // per-query Σ fma(q_i,q_i,·) (Euclidean on the
                             // matrix cores), or null
+  uint32_t* part_cnt;       // [nq][P] entries per list (matrix-core scan)
+  uint32_t slice_stride;    // rows from one slice's start to the next's (ditto)
 };
 
 struct MergeArgs {
@@ -72,16 +74,27 @@ hipError_t launch_row_norms(const double* X, size_t ldx, const uint32_t* slots, 
 hipError_t launch_query_norms(const double* Q, size_t ldq, uint32_t nq, uint32_t D, double* qn,
                               double* qq,
                               hipStream_t s);
-// Whether the FP64 scan of this metric, width and row layout runs on the
-// matrix cores, and how many partial lists per query it then writes for
-// nslices row slices (the value ScanF64Args.P and MergeArgs.P must hold).
-// (kmax: the largest k of the batch, ScanF64Args.kstride; nq its queries)
-bool scan_f64_uses_mfma(int metric, uint32_t D, const StoreView& st, int kmax, uint32_t nq);
-uint32_t scan_f64_lists(int metric, uint32_t D, const StoreView& st, int kmax, uint32_t nq,
-                        uint32_t nslices);
-hipError_t launch_scan_f64(const ScanF64Args& a, int metric, int kmax, uint32_t nslices,
-                           hipStream_t s);
-hipError_t launch_merge(const MergeArgs& a, int metric, int kmax, hipStream_t s);
+// ---- the Euclidean scan of a column prefix, on the VALU, and its merge ----
+// nslices row slices (a multiple of 8), a.P = nslices * kWavesPerBlock lists
+// of a.kstride >= kmax entries.
+hipError_t launch_scan_f64(const ScanF64Args& a, int kmax, uint32_t nslices, hipStream_t s);
+hipError_t launch_merge(const MergeArgs& a, int kmax, hipStream_t s);
+
+// ---- the FP64 scan on the matrix cores (svdb_scan_f64.hip) ----
+// Whether it serves this metric, width and row layout: every column compared.
+bool scan_f64_uses_mfma(int metric, uint32_t D, const StoreView& st);
+// Its partial lists per query and entries per list (P · cap · nq entries, at
+// most max_entries; P = 0 for an empty store).
+struct F64Lists {
+  uint32_t P, cap;
+};
+F64Lists scan_f64_lists(uint32_t nrows, uint32_t nq, int kmax, size_t max_entries);
+// a.P and a.kstride from scan_f64_lists; a.gtk, a.part_cnt set (gtk written).
+hipError_t launch_scan_f64_mfma(const ScanF64Args& a, int metric, int kmax, hipStream_t s);
+// The k best of a query's unsorted lists (m.kstride entries apart,
+// cnt[q][list] of them) with keys at most gtk[q].
+hipError_t launch_select_f64(const MergeArgs& m, const uint32_t* cnt, const uint64_t* gtk,
+                             int metric, hipStream_t s);
 
 // The nearest live row to one query over the first D columns (canonical
 // Euclidean key, lowest slot on ties) in one launch: each block reduces its

@@ -147,3 +147,56 @@ def test_matrix_core_cosine_underflowing_quotients():
         check(db, X, Q, k, "cos", what="underflow")
         check(db, X, Q, k, "dot", what="underflow")
     db.close()
+
+
+@pytest.mark.parametrize("D", [1, 3, 4, 5, 31, 33, 63, 65, 100, 127, 129, 200])
+def test_ragged_widths(D):
+    """Widths that are no whole stage or k-step, either side of the forms'
+    limits (64 and 128 columns), over the edge values."""
+    X, Q = ragged_store(D)
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    say(f"ragged D={D}")
+    for metric in ("l2", "cos", "dot"):
+        for k in (1, 10, 128):
+            check(db, X, Q, k, metric, what=f"D={D}")
+    db.close()
+
+
+def ragged_store(D):
+    rng = np.random.default_rng(D)
+    X = rng.standard_normal((3000, D))
+    X[100:140] = X[0:40]
+    X[200:220] *= 1e155
+    X[300:320] *= 1e-160
+    X[400, D - 1] = np.nan
+    X[401, 0] = np.inf
+    X[402, D - 1] = -np.inf
+    X[403] = 0.0
+    Q = rng.standard_normal((67, D))
+    Q[1] = X[0]
+    Q[3] = 0.0
+    Q[4, D - 1] = np.nan
+    return X, Q
+
+
+@pytest.mark.parametrize("n,nq,k", [(20_000, 70, 100), (70_001, 5, 10), (70_001, 1100, 3),
+                                    (33_000, 300, 128)])
+def test_sampled_bounds_and_ties(n, nq, k):
+    """Stores large enough for the sample's bound.  Half the rows are copies of
+    one row, a query's nearest: far more rows than a list, the selection's LDS
+    or its counting step hold, all equal, the lowest ids first; and rows sorted
+    by distance, so that one slice holds every answer."""
+    rng = np.random.default_rng(n)
+    D = 24
+    X = rng.standard_normal((n, D))
+    X[n // 4:n // 4 + n // 2] = X[7]
+    X[-5000:] = X[7] + np.linspace(0.0, 2.0, 5000)[:, None] * rng.standard_normal((1, D))
+    Q = np.vstack([X[7] + 0.01 * rng.standard_normal((nq - nq // 3, D)),
+                   rng.standard_normal((nq // 3, D))])
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    for metric in ("l2", "cos", "dot"):
+        say(f"ties {n} rows {nq} queries k={k} {metric}")
+        check(db, X, Q, k, metric, what="ties")
+    db.close()
