@@ -1046,10 +1046,9 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // (j = L let about L / f rows pass: 1M × 128, 16 times the shortlist.)
   // FP8 keeps j = L: its widening retries look for up to kMaxShort candidates
   // in the lists, and its error band needs them.
-  uint32_t ns_pre = tiles >= 16 * kPrepassSlices       ? kPrepassSlices
-                    : tiles >= 16 * kPrepassSlices / 4 ? kPrepassSlices / 4
-                    : tiles >= 128                     ? 32
-                                                       : 16;
+  // At least twice j minima: a rank near their number is the largest of them,
+  // no threshold at all (58k × 768 FP8, L = 128 of 128 minima: 3.3 ms for 2,816
+  // queries, 1.9 without a threshold).
   // BF16: twice the sample for shortlists past 64 (their threshold sits
   // further out, and a sparser sample leaves more rows below it to insert)
   // and for batches of up to 4096 queries (the scan's saving outweighs the
@@ -1059,17 +1058,24 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // 5M x 768 cosine: 861 instead of 4,293 of 12,288 before the BF16 pass).
   const uint32_t tpmax =
       (!fp8 && (L > 64 || nq <= 4096)) ? 2 * kPrepassMaxTiles : kPrepassMaxTiles;
-  const uint32_t tp =
-      std::max<uint32_t>(1, std::min<uint32_t>(tpmax, tiles / (16 * ns_pre)));
-  const double frac = (double)ns_pre * tp / tiles;
+  uint32_t ns_pre = tiles >= 16 * kPrepassSlices       ? kPrepassSlices
+                    : tiles >= 16 * kPrepassSlices / 4 ? kPrepassSlices / 4
+                                                       : 16;
+  uint32_t tp;
+  double frac;
   auto thr_rank = [&](int kk) {
     const uint32_t w = width(kk);
     return fp8 ? w
                : std::min<uint32_t>(
                      w, std::max<uint32_t>((uint32_t)std::ceil(3.0 * w * frac), kk + 16));
   };
-  const bool pre =
-      prepass_ && tiles >= 4 * ns_pre && ns_pre * kLowpLanesPerQuery >= thr_rank(k);
+  auto enough = [&] { return ns_pre * kLowpLanesPerQuery >= 2 * thr_rank(k); };
+  for (;; ns_pre *= 2) {
+    tp = std::max<uint32_t>(1, std::min<uint32_t>(tpmax, tiles / (16 * ns_pre)));
+    frac = (double)ns_pre * tp / std::max<uint32_t>(1, tiles);
+    if (enough() || ns_pre >= kPrepassSlices || tiles < 8 * ns_pre) break;
+  }
+  const bool pre = prepass_ && tiles >= 4 * ns_pre && enough();
   const uint32_t NL_pre = ns_pre * kLowpLanesPerQuery;
   // Row slices for a scan of grp query blocks wanting kk neighbours: at
   // least 8, more when there are few query blocks, each at least 4 tiles
@@ -1387,11 +1393,28 @@ int Engine::lowp_complete() {
     // than the stage before took: with a threshold about rg.pass entries,
     // without one up to kLowpLP a list) and reranked; only those still
     // uncertified go on.
+    // An FP8 retry gathers some 3/4 of its candidates' FP64 rows at about 6 TB/s
+    // (a wavefront per query: at least a round trip per 64 rows and 16 columns),
+    // the BF16 pass scans every row at about 500 TF/s, its rows read once at 5
+    // TB/s, and costs some 0.4 ms more: on small stores it is the cheaper one, and it
+    // certifies more (51k × 1,536, 114 queries, k = 10: 13.7 ms with both
+    // retries, 5.6 ms with the 4,096-wide one mostly skipped, 0.6 ms by this
+    // rule).
+    const bool bf16_ok = lowp_ && (sh_.dp <= 256 || bf16_wide_dp_supported(sh_.dp));
+    auto second_pass_cheaper = [&](uint32_t n, uint32_t Lw) {
+      if (!fp8 || !bf16_ok) return false;
+      const double rows = std::min<double>(Lw, (double)nphys_);
+      const double retry = std::max(n * rows * 0.75 * 8.0 * d_ / 6e12,
+                                    rows / 64 * ((d_ + 15) / 16) * 0.8e-6);
+      const double scan = (double)nphys_ * sh_.dp * 2.0;
+      return std::max(scan * n / 5e14, scan / 5e12) + 4e-4 < retry;
+    };
     uint32_t Lprev = L;
     for (int wi = 0; wi < 2; wi++) {
       const uint32_t Lw = wi == 0 ? 1024u : (uint32_t)kMaxShort;
       if (nf == 0 || Lw <= L) continue;
       if (rg.pass ? 2 * rg.pass < 3 * Lprev : (size_t)NL * kLowpLP < 2 * (size_t)Lw) continue;
+      if (second_pass_cheaper(nf, Lw)) break;
       Lprev = Lw;
       // A retry that has lately certified almost none of its queries for
       // this precision and metric is skipped (its queries go on to the next
@@ -1455,7 +1478,6 @@ int Engine::lowp_complete() {
     // Second chance for FP8: queries its stages leave uncertified go through
     // the BF16 first pass when the store has a BF16 shadow (a bound about
     // 16x tighter); that pass rescans in FP64 only what it cannot certify.
-    const bool bf16_ok = lowp_ && (sh_.dp <= 256 || bf16_wide_dp_supported(sh_.dp));
     if (fp8 && bf16_ok) {
       if ((rc = scratch(&c_->s_cidx_, &c_->s_cidx_n_, (size_t)nf * sizeof(uint32_t)))) return rc;
       if ((rc = scratch(&c_->s_cq_, &c_->s_cq_n_, (size_t)nf * d_ * sizeof(double)))) return rc;
