@@ -41,44 +41,73 @@ __device__ __forceinline__ size_t cand_list(const LowpScanArgs& a, uint32_t q, u
   return (size_t)q * a.NL + list;
 }
 
-// The four rows of a lane's accumulator, at least one keyed below tau: those
-// below it enter the list at `e` holding `cnt` entries.  Straight-line stores
-// (a lane seldom has more than one, but its wavefront's lanes have theirs at
-// different rows); a list that is or has become full takes the loop.
-__device__ __forceinline__ void cand_append4(uint2* __restrict__ e, uint32_t& cnt, float& tau,
-                                             float (&k4)[4], uint32_t srow) {
-#pragma unroll
-  for (int r = 0; r < 4; r++)
-    if (k4[r] < tau && cnt < (uint32_t)kLowpLC) {
-      e[cnt++] = make_uint2(__float_as_uint(k4[r]), srow + r);
-      k4[r] = INFINITY;
-    }
-  if (__builtin_expect(cnt < (uint32_t)kLowpLC, 1)) return;
-  for (int r = 0; r < 4;) {
-    float m1 = -INFINITY, m2 = -INFINITY;  // the largest two keys held
-    uint32_t at = 0;
+// A lane's last entry waits here for the start of the next tile (or for the
+// lane's next entry): a tile ends with a wait for its successor's loads, which
+// counts stores too, and one issued late in the tile would hold up the block
+// (2M × 128, 16,384 cosine queries: 7.5 ms with stores at once, 6.9 deferred).
+// Entries count from the block's first list: its lists stay below 2^32 entries.
+struct CandPending {
+  uint32_t at = ~0u;  // entry index (~0: none)
+  uint32_t key, slot;
+};
+
+__device__ __forceinline__ void cand_flush(uint2* ent, CandPending& p) {
+  if (p.at != ~0u) ent[p.at] = make_uint2(p.key, p.slot);
+  p.at = ~0u;
+}
+
+// The four rows of a lane's accumulator: those keyed below tau enter list
+// `list` holding `cnt` entries, the smallest first.  A wavefront seldom has
+// more than one such row, so a pass takes each lane's smallest and the loop
+// ends with the wavefront's last.  A test and a store for each of the four
+// rows spent the time in branches over nothing, and sixteen copies of that code
+// made a kernel of 74 KB, past the 64 KB instruction cache (1M × 256, 8,192
+// queries: 5.1 ms, so 3.9).  Called by a whole wavefront; `ent` is the entries
+// of the block's first list.
+__device__ __forceinline__ void cand_append4(uint2* ent, CandPending& p, uint32_t list,
+                                             uint32_t& cnt, float& tau, float (&k4)[4],
+                                             uint32_t srow) {
+  const uint32_t e0 = list * kLowpLC;
+  do {
+    const float k = fminf(fminf(k4[0], k4[1]), fminf(k4[2], k4[3]));
+    if (k < tau) {
+      const uint32_t r = k4[0] == k ? 0 : k4[1] == k ? 1 : k4[2] == k ? 2 : 3;
+      const uint32_t at = cnt;
+      if (at < (uint32_t)kLowpLC) {
+        cand_flush(ent, p);
+        p.at = e0 + at;
+        p.key = __float_as_uint(k);
+        p.slot = srow + r;
+        cnt = at + 1;
+      }
+      if (__builtin_expect(cnt == (uint32_t)kLowpLC, 0)) {
+        // full: from here on tau is the largest key held, whose place a
+        // smaller one takes
+        cand_flush(ent, p);
+        uint2* e = ent + e0;
+        float m1 = -INFINITY, m2 = -INFINITY;  // the largest two keys held
+        uint32_t big = 0;
 #pragma unroll 2
-    for (int i = 0; i < kLowpLC; i += 2) {
-      const uint4 v = *reinterpret_cast<const uint4*>(e + i);
-      const float x = __uint_as_float(v.x), y = __uint_as_float(v.z);
-      m2 = fmaxf(m2, fminf(m1, x));
-      at = x > m1 ? i : at;
-      m1 = fmaxf(m1, x);
-      m2 = fmaxf(m2, fminf(m1, y));
-      at = y > m1 ? i + 1 : at;
-      m1 = fmaxf(m1, y);
+        for (int i = 0; i < kLowpLC; i += 2) {
+          const uint4 v = *reinterpret_cast<const uint4*>(e + i);
+          const float x = __uint_as_float(v.x), y = __uint_as_float(v.z);
+          m2 = fmaxf(m2, fminf(m1, x));
+          big = x > m1 ? i : big;
+          m1 = fmaxf(m1, x);
+          m2 = fmaxf(m2, fminf(m1, y));
+          big = y > m1 ? i + 1 : big;
+          m1 = fmaxf(m1, y);
+        }
+        tau = m1;
+        if (at == (uint32_t)kLowpLC) {
+          e[big] = make_uint2(__float_as_uint(k), srow + r);
+          tau = fmaxf(m2, k);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) k4[i] = r == (uint32_t)i ? INFINITY : k4[i];
     }
-    tau = m1;
-    // the next row keyed below the largest entry takes its place
-    for (; r < 4; r++) {
-      const float k = r == 0 ? k4[0] : r == 1 ? k4[1] : r == 2 ? k4[2] : k4[3];
-      if (!(k < tau)) continue;
-      e[at] = make_uint2(__float_as_uint(k), srow + r);
-      tau = fmaxf(m2, k);
-      r++;
-      break;
-    }
-  }
+  } while (__ballot(fminf(fminf(k4[0], k4[1]), fminf(k4[2], k4[3])) < tau));
 }
 
 // A sorted register list (unused entries: slot ~0) to its place.

@@ -350,7 +350,7 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
   const uint32_t qpb = NW * QF * 16;
   const uint32_t nqb = (a.nq + qpb - 1) / qpb;
   const uint32_t xcd = blockIdx.x % 8, local = blockIdx.x / 8;
-  const uint32_t qbase = (local % nqb) * qpb + wave * QF * 16;
+  const uint32_t qblock = (local % nqb) * qpb, qbase = qblock + wave * QF * 16;
   const uint32_t slice = (local / nqb) * 8 + xcd;
   const uint32_t r0 = slice * a.slice_stride;
   const uint32_t r1 = min(r0 + a.rows_per_slice, a.nrows_pad);
@@ -365,6 +365,8 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
   float lk[SORTED ? QF : 1][LP];     // kFormSorted
   uint32_t ls[SORTED ? QF : 1][LP];
   uint32_t cnt[QF];                  // kFormAppend
+  CandPending pend;
+  uint2* const ent = a.ent + cand_list(a, qblock, 0) * kLowpLC;
 #pragma unroll
   for (int f = 0; f < QF; f++) {
     const uint32_t q = qbase + f * 16 + ql;  // < nq_pad (Q8 is padded)
@@ -428,30 +430,29 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; r++) k4[r] = key(acc, f, r, w0, w1);
       const float mn = fminf(fminf(k4[0], k4[1]), fminf(k4[2], k4[3]));
-      if (mn < tau[f]) {
-        if constexpr (!SORTED) {
-          cand_append4(a.ent + cand_list(a, qbase + f * 16 + ql, list) * kLowpLC, cnt[f], tau[f],
-                       k4, srow);
-        } else {
+      if constexpr (!SORTED) {
+        if (__ballot(mn < tau[f]))
+          cand_append4(ent, pend, (uint32_t)cand_list(a, qbase - qblock + f * 16 + ql, list), cnt[f],
+                       tau[f], k4, srow);
+      } else if (mn < tau[f]) {
 #pragma unroll
-          for (int r = 0; r < 4; r++) {
-            if (k4[r] < lk[f][LP - 1]) {
-              lk[f][LP - 1] = k4[r];
-              ls[f][LP - 1] = srow + r;
+        for (int r = 0; r < 4; r++) {
+          if (k4[r] < lk[f][LP - 1]) {
+            lk[f][LP - 1] = k4[r];
+            ls[f][LP - 1] = srow + r;
 #pragma unroll
-              for (int j = LP - 1; j > 0; j--) {
-                const bool sw = lk[f][j] < lk[f][j - 1];
-                const float tk = sw ? lk[f][j - 1] : lk[f][j];
-                const uint32_t tsl = sw ? ls[f][j - 1] : ls[f][j];
-                lk[f][j - 1] = sw ? lk[f][j] : lk[f][j - 1];
-                ls[f][j - 1] = sw ? ls[f][j] : ls[f][j - 1];
-                lk[f][j] = tk;
-                ls[f][j] = tsl;
-              }
+            for (int j = LP - 1; j > 0; j--) {
+              const bool sw = lk[f][j] < lk[f][j - 1];
+              const float tk = sw ? lk[f][j - 1] : lk[f][j];
+              const uint32_t tsl = sw ? ls[f][j - 1] : ls[f][j];
+              lk[f][j - 1] = sw ? lk[f][j] : lk[f][j - 1];
+              ls[f][j - 1] = sw ? ls[f][j] : ls[f][j - 1];
+              lk[f][j] = tk;
+              ls[f][j] = tsl;
             }
           }
-          tau[f] = lk[f][LP - 1];
         }
+        tau[f] = lk[f][LP - 1];
       }
     }
   };
@@ -487,6 +488,7 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
       if (t >= ntiles) break;
       const unsigned char* cur = h ? buf1 : buf0;
       if (t + 1 < ntiles) issue_tile8<KS, NW>(a, h ? buf0 : buf1, r0 + (t + 1) * G::TR, wave, lane);
+      if constexpr (FORM == kFormAppend) cand_flush(ent, pend);
       const uint32_t trow = r0 + t * G::TR;
       const float* aux = reinterpret_cast<const float*>(cur + G::TILE_B);
       // A operand of K step ks: bytes 128·ks + 32·rg .. +31 of row arow
@@ -569,6 +571,7 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
     }
   }
   if (active) epilogue(pacc, pw0, pw1, prow);
+  if constexpr (FORM == kFormAppend) cand_flush(ent, pend);
 #pragma unroll
   for (int f = 0; f < QF; f++) {
     const uint32_t q = qbase + f * 16 + ql;

@@ -98,3 +98,25 @@ def test_thresholded_lists(d, nq):
         for metric in ("l2", "cos", "dot"):
             check(db, X, Q, 10, metric, "fp8")
     db.close()
+
+
+@pytest.mark.parametrize("d,nq,k", [(20, 11_777, 2), (256, 5_800, 10)])
+def test_slices_past_two_rounds(d, nq, k):
+    """Query counts whose blocks leave a last round of the GPU part empty at
+    the fewest slices, so that the scan takes more of them; ids and scores as
+    the exhaustive FP64 search has them.  A third of the rows are one cluster
+    stored in a row."""
+    rng = np.random.default_rng(d)
+    n = 100_003
+    X = rng.standard_normal((n, d))
+    X[5000:5000 + n // 3] = X[0] + 0.05 * rng.standard_normal((n // 3, d))
+    Q = np.vstack([X[0] + 0.05 * rng.standard_normal((nq // 8, d)),
+                   rng.standard_normal((nq - nq // 8, d))])
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    for metric in ("l2", "cos", "dot"):
+        ids, sc = db.search(Q, k, metric, "bf16")
+        rid, rsc = db.search(Q, k, metric, "fp64")
+        assert np.array_equal(ids, rid), f"{d} {nq} {metric}: ids differ"
+        assert np.array_equal(sc.view(np.uint64), rsc.view(np.uint64)), f"{d} {nq} {metric}"
+    db.close()
