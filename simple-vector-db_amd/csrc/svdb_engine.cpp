@@ -93,7 +93,6 @@ struct RefCtx {
   hipStream_t stream = nullptr;
   double* buf = nullptr;
   size_t cap = 0;  // doubles
-  uint32_t* slots = nullptr;
   float* out = nullptr;
   uint64_t* host = nullptr;  // pinned: the one-launch form's (result, seq)
   uint64_t seq = 0;
@@ -106,10 +105,7 @@ int pair_ref32_host(const double* a_in, const double* b_in, size_t n, int metric
   std::lock_guard<std::mutex> g(g_ref.mu);
   if (!g_ref.stream) {
     HIPCHK(hipStreamCreateWithFlags(&g_ref.stream, hipStreamNonBlocking), "stream");
-    HIPCHK(hipMalloc(&g_ref.slots, 2 * sizeof(uint32_t)), "hipMalloc");
     HIPCHK(hipMalloc(&g_ref.out, sizeof(float)), "hipMalloc");
-    uint32_t s[2] = {0, 1};
-    HIPCHK(hipMemcpy(g_ref.slots, s, sizeof(s), hipMemcpyHostToDevice), "copy");
     HIPCHK(hipHostMalloc((void**)&g_ref.host, 64), "hipHostMalloc");
     g_ref.host[0] = g_ref.host[1] = 0;
   }
@@ -154,8 +150,8 @@ int pair_ref32_host(const double* a_in, const double* b_in, size_t n, int metric
     HIPCHK(hipMemcpyAsync(g_ref.buf, a_in, n * sizeof(double), hipMemcpyHostToDevice, g_ref.stream), "copy");
     HIPCHK(hipMemcpyAsync(g_ref.buf + ld, b_in, n * sizeof(double), hipMemcpyHostToDevice, g_ref.stream), "copy");
   }
-  HIPCHK(launch_pair_ref32(g_ref.buf, ld, g_ref.slots, g_ref.slots + 1, 1, (uint32_t)n, metric,
-                           g_ref.out, g_ref.stream), "k_pair_ref32");
+  HIPCHK(launch_pair_ref32(g_ref.buf, g_ref.buf + ld, (uint32_t)n, metric, g_ref.out,
+                           g_ref.stream), "k_pair_ref32");
   HIPCHK(hipMemcpyAsync(out, g_ref.out, sizeof(float), hipMemcpyDeviceToHost, g_ref.stream), "copy");
   HIPCHK(hipStreamSynchronize(g_ref.stream), "sync");
   return SVDB_OK;

@@ -121,8 +121,9 @@ hipError_t launch_mfma_loop(int kind, uint32_t blocks, int iters, float* out, hi
 double mfma_loop_flop(int kind, uint32_t blocks, int iters);
 hipError_t launch_pair_f64(const double* X, size_t ldx, const uint32_t* sa, const uint32_t* sb,
                            uint32_t np, uint32_t D, int metric, double* out, hipStream_t s);
-hipError_t launch_pair_ref32(const double* M, size_t ld, const uint32_t* sa, const uint32_t* sb,
-                             uint32_t np, uint32_t n, int metric, float* out, hipStream_t s);
+// The reference's float metric of one pair of n-element device rows.
+hipError_t launch_pair_ref32(const double* A, const double* B, uint32_t n, int metric, float* out,
+                             hipStream_t s);
 // One pair of at most kRef32ArgsMax elements each, carried in the kernel
 // arguments (a then b in ab), the reference's float metric written to
 // host memory: out[0] the float's bits, then out[1] = seq.

@@ -625,52 +625,82 @@ hipError_t launch_pair_f64(const double* X, size_t ldx, const uint32_t* sa, cons
   return hipGetLastError();
 }
 
-// The reference's own float arithmetic (vector_database.c:301-352), one
-// thread per pair, so the legacy float-returning metrics are bit-identical
-// to the reference: FP64 products added into float accumulators
-// (acc = (float)((double)acc + a*b)); Euclidean squares the float-rounded
-// difference in float; sqrt and the cosine division in double.
-// The reference's float metric of one pair (vector_database.c:301-352):
-// float accumulators, each step widened to double and rounded back, as its
-// C compiles.
-__device__ float ref32_metric(const double* __restrict__ A, const double* __restrict__ B,
-                              uint32_t n, int metric) {
-  if (metric == kCos) {
-    float dp = 0.0f, na = 0.0f, nb = 0.0f;
-    for (uint32_t i = 0; i < n; i++) {
-      dp = (float)((double)dp + A[i] * B[i]);
-      na = (float)((double)na + A[i] * A[i]);
-      nb = (float)((double)nb + B[i] * B[i]);
-    }
-    return (float)((double)dp / (sqrt((double)na) * sqrt((double)nb)));
-  }
-  if (metric == kL2) {
-    float sum = 0.0f;
-    for (uint32_t i = 0; i < n; i++) {
-      float diff = (float)(A[i] - B[i]);
-      float sq = diff * diff;
-      sum = sum + sq;
-    }
-    return (float)sqrt((double)sum);
-  }
+// The reference's float metrics (vector_database.c:301-352), bit-identical to
+// it: FP64 products added into float accumulators (acc = (float)((double)acc +
+// a*b)); Euclidean squares the float-rounded difference in float; sqrt and the
+// cosine division in double.  One wavefront: every product first, a column per
+// lane, into LDS, then the serial chains (cosine: its three in lanes 0..2, one
+// instruction stream).  Bound by those chains, some 24 cycles a column, with the
+// elements read beforehand: a single thread that also read them and multiplied
+// took 14.2 µs at 128 columns, 4.5 so.
+constexpr uint32_t kRefCols = 256;
+
+__device__ __forceinline__ float ref32_wave(const double* __restrict__ A,
+                                            const double* __restrict__ B, uint32_t n, int metric,
+                                            double (&P)[3][kRefCols]) {
+  const uint32_t lane = threadIdx.x;
+  const double* mine = P[lane < 3 && metric == kCos ? lane : 0];
   float acc = 0.0f;
-  for (uint32_t i = 0; i < n; i++) acc = (float)((double)acc + A[i] * B[i]);
-  return acc;
+  for (uint32_t c0 = 0; c0 < n; c0 += kRefCols) {
+    const uint32_t m = min(kRefCols, n - c0);
+    for (uint32_t i = lane; i < m; i += 64) {
+      const double u = A[c0 + i], v = B[c0 + i];
+      if (metric == kL2) {
+        const float diff = (float)(u - v);
+        P[0][i] = (double)(diff * diff);
+      } else {
+        P[0][i] = u * v;
+        if (metric == kCos) {
+          P[1][i] = u * u;
+          P[2][i] = v * v;
+        }
+      }
+    }
+    __syncthreads();
+    uint32_t i = 0;
+    if (metric == kL2) {
+      for (; i + 8 <= m; i += 8) {
+        float t[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) t[j] = (float)mine[i + j];
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc = acc + t[j];
+      }
+      for (; i < m; i++) acc = acc + (float)mine[i];
+    } else {
+      for (; i + 8 <= m; i += 8) {
+        double t[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) t[j] = mine[i + j];
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc = (float)((double)acc + t[j]);
+      }
+      for (; i < m; i++) acc = (float)((double)acc + mine[i]);
+    }
+    __syncthreads();
+  }
+  if (metric == kCos) {
+    const float na = __shfl(acc, 1), nb = __shfl(acc, 2);
+    return (float)((double)acc / (sqrt((double)na) * sqrt((double)nb)));
+  }
+  return metric == kL2 ? (float)sqrt((double)acc) : acc;
 }
 
-__global__ void k_pair_ref32(const double* __restrict__ M, size_t ld,
-                             const uint32_t* __restrict__ sa, const uint32_t* __restrict__ sb,
-                             uint32_t np, uint32_t n, int metric, float* __restrict__ out) {
-  uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np) return;
-  out[p] = ref32_metric(M + (size_t)sa[p] * ld, M + (size_t)sb[p] * ld, n, metric);
+// One pair of device rows.
+__global__ __launch_bounds__(64) void k_pair_ref32(const double* __restrict__ A,
+                                                   const double* __restrict__ B, uint32_t n,
+                                                   int metric, float* __restrict__ out) {
+  __shared__ double P[3][kRefCols];
+  const float r = ref32_wave(A, B, n, metric, P);
+  if (threadIdx.x == 0) out[0] = r;
 }
 
 // One pair from the kernel arguments (the drop-in per-call functions): the
 // result, then seq once it is visible, into host memory the caller polls.
-__global__ void k_pair_ref32_args(const PairRef32Args a) {
+__global__ __launch_bounds__(64) void k_pair_ref32_args(const PairRef32Args a) {
+  __shared__ double P[3][kRefCols];
+  const float r = ref32_wave(a.ab, a.ab + a.n, a.n, a.metric, P);
   if (threadIdx.x != 0) return;
-  const float r = ref32_metric(a.ab, a.ab + a.n, a.n, a.metric);
   a.out[0] = (uint64_t)__float_as_uint(r);
   __threadfence_system();
   __hip_atomic_store(a.out + 1, a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -682,11 +712,9 @@ hipError_t launch_pair_ref32_args(const PairRef32Args& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_pair_ref32(const double* M, size_t ld, const uint32_t* sa, const uint32_t* sb,
-                             uint32_t np, uint32_t n, int metric, float* out, hipStream_t s) {
-  if (np == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_pair_ref32, dim3((np + 255) / 256), dim3(256), 0, s, M, ld, sa, sb, np, n,
-                     metric, out);
+hipError_t launch_pair_ref32(const double* A, const double* B, uint32_t n, int metric, float* out,
+                             hipStream_t s) {
+  hipLaunchKernelGGL(k_pair_ref32, dim3(1), dim3(64), 0, s, A, B, n, metric, out);
   return hipGetLastError();
 }
 
