@@ -191,8 +191,7 @@ Engine::~Engine() {
   if (near_host_) (void)hipHostFree(near_host_);
   for (auto& c : ctx_) {
     if (c.stream) (void)hipStreamSynchronize(c.stream);
-    void* cb[] = {c.s_q_, c.s_qn_, c.s_k_, c.s_pk_, c.s_ps_, c.s_ids_, c.s_sc_, c.s_pair_,
-                  c.s_pout_, c.s_qb_, c.s_qp_, c.s_ck_, c.s_cs_, c.s_sk_, c.s_ss_, c.s_beta_,
+    void* cb[] = {c.s_q_, c.s_qn_, c.s_k_, c.s_pk_, c.s_ps_, c.s_ids_, c.s_sc_, c.s_qb_, c.s_qp_, c.s_ck_, c.s_cs_, c.s_sk_, c.s_ss_, c.s_beta_,
                   c.s_fail_, c.s_err_, c.s_lk_, c.s_ls_, c.s_km_, c.s_fq_, c.s_fid_, c.s_fsc_, c.s_fk_, c.s_sk2_, c.s_ss2_,
                   c.s_beta2_, c.s_fail2_, c.s_cidx_, c.s_cq_, c.s_cid_, c.s_csc_};
     for (void* p : cb)
@@ -212,6 +211,7 @@ Engine::~Engine() {
     if (p) (void)hipFree(p);
   if (h_stage_) (void)hipHostFree(h_stage_);
   for (auto& e : ev_pool_) (void)hipEventDestroy(e);
+  for (auto& e : pair_ev_) (void)hipEventDestroy(e);
   (void)hipStreamDestroy(stream_);
 }
 
@@ -2087,24 +2087,74 @@ int Engine::pairs_f64(const size_t* a, const size_t* b, size_t np, int metric, d
   }
   if (np == 0) return SVDB_OK;
   fault_point();
-  std::vector<uint32_t> hs(2 * np);
-  for (size_t p = 0; p < np; p++) {
-    if (a[p] >= nalive_ || b[p] >= nalive_) {
-      set_error(SVDB_EINVAL, "index out of range");
-      return SVDB_EINVAL;
-    }
-    hs[p] = select_slot(a[p]);
-    hs[np + p] = select_slot(b[p]);
+  // In blocks of up to kPairBlock pairs through pinned memory that the kernel
+  // reads and writes: a chunk's pairs are turned into slots while the GPU
+  // works on the chunks before it, and the block's results go to the caller
+  // once every index has proved good (past one block, all are looked at
+  // first), again beside the later chunks' work.
+  constexpr size_t kPairBlock = (size_t)1 << 20, kPairChunk = (size_t)1 << 17;
+  auto bad_index = [&]() -> int {
+    set_error(SVDB_EINVAL, "index out of range");
+    return SVDB_EINVAL;
+  };
+  if (np > kPairBlock) {
+    bool bad = false;
+    for (size_t p = 0; p < np; p++) bad |= a[p] >= nalive_ || b[p] >= nalive_;
+    if (bad) return bad_index();
   }
-  int rc;
-  if ((rc = scratch(&c_->s_pair_, &c_->s_pair_n_, 2 * np * sizeof(uint32_t)))) return rc;
-  if ((rc = scratch(&c_->s_pout_, &c_->s_pout_n_, np * sizeof(double)))) return rc;
-  HIPCHK(hipMemcpyAsync(c_->s_pair_, hs.data(), 2 * np * sizeof(uint32_t), hipMemcpyHostToDevice, c_->stream), "pairs upload");
-  const uint32_t* sa = (const uint32_t*)c_->s_pair_;
-  HIPCHK(launch_pair_f64(X_, ld_, sa, sa + np, (uint32_t)np, (uint32_t)d_, metric,
-                         (double*)c_->s_pout_, c_->stream), "k_pair_f64");
-  HIPCHK(hipMemcpyAsync(out, c_->s_pout_, np * sizeof(double), hipMemcpyDeviceToHost, c_->stream), "pairs download");
-  HIPCHK(hipStreamSynchronize(c_->stream), "pairs");
+  const size_t cap = std::min(np, kPairBlock);
+  char* st = static_cast<char*>(host_stage(&h_stage_, &h_stage_n_, cap * (sizeof(double) + 2 * sizeof(uint32_t))));
+  if (!st) {
+    set_error(SVDB_EDEVICE, "hipHostMalloc failed");
+    return SVDB_EDEVICE;
+  }
+  double* ho = reinterpret_cast<double*>(st);
+  uint32_t* hs = reinterpret_cast<uint32_t*>(ho + cap);
+  auto to_slots = [&](const size_t* x, size_t n, uint32_t* s) {
+    bool bad = false;
+    if (!has_deletes_) {
+      for (size_t i = 0; i < n; i++) {
+        bad |= x[i] >= nalive_;
+        s[i] = (uint32_t)x[i];
+      }
+      return !bad;
+    }
+    for (size_t i = 0; i < n; i++) {
+      if (x[i] >= nalive_) return false;
+      s[i] = select_slot(x[i]);
+    }
+    return true;
+  };
+  for (size_t b0 = 0; b0 < np; b0 += kPairBlock) {
+    const size_t n = std::min(kPairBlock, np - b0);
+    auto run = [&]() -> int {
+      for (size_t c0 = 0, e = 0; c0 < n; c0 += kPairChunk, e++) {
+        const size_t m = std::min(kPairChunk, n - c0);
+        uint32_t* s = hs + 2 * c0;
+        if (!to_slots(a + b0 + c0, m, s) || !to_slots(b + b0 + c0, m, s + m)) return bad_index();
+        HIPCHK(launch_pair_f64(X_, ld_, s, (uint32_t)m, (uint32_t)d_, metric, ho + c0, c_->stream),
+               "k_pair_f64");
+        if (c0 + m == n) break;  // (the last chunk is waited for with the stream)
+        if (pair_ev_.size() <= e) {
+          hipEvent_t ev;
+          HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event");
+          pair_ev_.push_back(ev);
+        }
+        HIPCHK(hipEventRecord(pair_ev_[e], c_->stream), "event");
+      }
+      for (size_t c0 = 0, e = 0; c0 < n; c0 += kPairChunk, e++) {
+        const size_t m = std::min(kPairChunk, n - c0);
+        HIPCHK(c0 + m == n ? hipStreamSynchronize(c_->stream) : hipEventSynchronize(pair_ev_[e]),
+               "pairs");
+        std::memcpy(out + b0 + c0, ho + c0, m * sizeof(double));
+      }
+      return SVDB_OK;
+    };
+    if (const int rc = run()) {
+      (void)hipStreamSynchronize(c_->stream);  // the staging is free again
+      return rc;
+    }
+  }
   return SVDB_OK;
 }
 

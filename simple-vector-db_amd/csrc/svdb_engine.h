@@ -243,8 +243,6 @@ class Engine {
     void* s_ps_ = nullptr;     size_t s_ps_n_ = 0;
     void* s_ids_ = nullptr;    size_t s_ids_n_ = 0;
     void* s_sc_ = nullptr;     size_t s_sc_n_ = 0;
-    void* s_pair_ = nullptr;   size_t s_pair_n_ = 0;
-    void* s_pout_ = nullptr;   size_t s_pout_n_ = 0;
     void* s_qb_ = nullptr;     size_t s_qb_n_ = 0;
     void* s_qp_ = nullptr;     size_t s_qp_n_ = 0;
     void* s_ck_ = nullptr;     size_t s_ck_n_ = 0;
@@ -313,8 +311,9 @@ class Engine {
   static constexpr int kCtx = 3;
   SearchCtx ctx_[kCtx];
   SearchCtx* c_ = &ctx_[0];
-  void* h_stage_ = nullptr;  // pinned: row upload staging
+  void* h_stage_ = nullptr;  // pinned: row upload and pair staging
   size_t h_stage_n_ = 0;
+  std::vector<hipEvent_t> pair_ev_;  // one per chunk of a block of pairs
   void* near_dev_ = nullptr;        // k_nearest1: block results and ticket
   uint64_t* near_host_ = nullptr;   // pinned: its answer (id, seq)
   uint64_t near_seq_ = 0;

@@ -119,8 +119,10 @@ hipError_t launch_nearest1(const Nearest1Args& a, hipStream_t s);
 // floats.  mfma_loop_flop gives the flop of one such launch.
 hipError_t launch_mfma_loop(int kind, uint32_t blocks, int iters, float* out, hipStream_t s);
 double mfma_loop_flop(int kind, uint32_t blocks, int iters);
-hipError_t launch_pair_f64(const double* X, size_t ldx, const uint32_t* sa, const uint32_t* sb,
-                           uint32_t np, uint32_t D, int metric, double* out, hipStream_t s);
+// FP64 metrics of np pairs of rows: slots[i] and slots[np + i] to out[i]; slots
+// and out may lie in pinned host memory.
+hipError_t launch_pair_f64(const double* X, size_t ldx, const uint32_t* slots, uint32_t np,
+                           uint32_t D, int metric, double* out, hipStream_t s);
 // The reference's float metric of one pair of n-element device rows.
 hipError_t launch_pair_ref32(const double* A, const double* B, uint32_t n, int metric, float* out,
                              hipStream_t s);
