@@ -1038,8 +1038,11 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // it: they then skip nearly every row from the first tile on, and take a
   // few hundred rows per query in all.
   // BF16: j = 3·L·f, so that about three times the shortlist passes, and at
-  // least k + 16, so that at least that many do however the rows are placed.
-  // (j = L let about L / f rows pass: 1M × 128, 16 times the shortlist.)
+  // least 12 + k / 8, whose spread between samples is 28 % (k = 10) to 20 %
+  // (k = 100).  (Each insertion costs the scan: j = L let about L / f rows
+  // pass, k + 16 of a 30th of the store 30·k; 1M × 128 served 512 queries at a
+  // time, k up to 100: 6.9 ms at k + 16, 5.16 so, and as many queries
+  // certified, also where clusters of 40 to 20,000 rows were stored in a row.)
   // FP8 keeps j = L: its widening retries look for up to kMaxShort candidates
   // in the lists, and its error band needs them.
   // At least twice j minima: a rank near their number is the largest of them,
@@ -1063,7 +1066,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     const uint32_t w = width(kk);
     return fp8 ? w
                : std::min<uint32_t>(
-                     w, std::max<uint32_t>((uint32_t)std::ceil(3.0 * w * frac), kk + 16));
+                     w, std::max<uint32_t>((uint32_t)std::ceil(3.0 * w * frac), 12 + kk / 8));
   };
   auto enough = [&] { return ns_pre * kLowpLanesPerQuery >= 2 * thr_rank(k); };
   for (;; ns_pre *= 2) {
