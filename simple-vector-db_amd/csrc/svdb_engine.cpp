@@ -192,7 +192,7 @@ Engine::~Engine() {
   for (auto& c : ctx_) {
     if (c.stream) (void)hipStreamSynchronize(c.stream);
     void* cb[] = {c.s_q_, c.s_qn_, c.s_k_, c.s_pk_, c.s_ps_, c.s_ids_, c.s_sc_, c.s_qb_, c.s_qp_, c.s_ck_, c.s_cs_, c.s_sk_, c.s_ss_, c.s_beta_,
-                  c.s_fail_, c.s_err_, c.s_lk_, c.s_ls_, c.s_km_, c.s_fq_, c.s_fid_, c.s_fsc_, c.s_fk_, c.s_sk2_, c.s_ss2_,
+                  c.s_fail_, c.s_lk_, c.s_ls_, c.s_km_, c.s_fq_, c.s_fid_, c.s_fsc_, c.s_fk_, c.s_sk2_, c.s_ss2_,
                   c.s_beta2_, c.s_fail2_, c.s_cidx_, c.s_cq_, c.s_cid_, c.s_csc_};
     for (void* p : cb)
       if (p) (void)hipFree(p);
@@ -979,9 +979,14 @@ uint32_t Engine::lowp_width(int kk, bool fp8, size_t shortlist) {
 }
 
 int Engine::run_lowp(const double* dQ, size_t ldq, uint32_t nq, int metric, int k,
-                     uint64_t* dids, double* dscores, uint32_t ostride, bool fp8) {
+                     uint64_t* dids, double* dscores, uint32_t ostride, bool fp8,
+                     const double* hQ) {
   LowpRange r{metric, 0, nq, k, 0, 0, 0, 0, 0, 0};
-  return run_lowp_ranges(dQ, ldq, &r, 1, k, dids, dscores, ostride, fp8);
+  if (const int rc = lowp_enqueue(dQ, ldq, &r, 1, k, dids, dscores, ostride, fp8, hQ)) {
+    c_->lp.on = false;
+    return rc;
+  }
+  return lowp_complete();
 }
 
 // Low-precision search of nr metric ranges: range i holds R[i].n queries of
@@ -989,12 +994,13 @@ int Engine::run_lowp(const double* dQ, size_t ldq, uint32_t nq, int metric, int 
 // ranges (BF16 rows <= 256 wide only) each take a run of slots starting on a
 // wavefront boundary (padding slots are flagged and never scanned).  The
 // first pass runs one single-metric launch per metric, or one launch of the
-// mixed-metric kernel when all ranges fit one query block; the pre-pass runs
-// per range; the shortlists and the reranks of all ranges share a launch;
-// widening and fallback run per range, each with its own k and shortlist
-// width (k is the largest over ranges).
+// mixed-metric kernel when all ranges fit one query block, and so does the
+// pre-pass; the thresholds, the shortlists and the reranks of all ranges share
+// a launch; widening and fallback run per range, each with its own k and
+// shortlist width (k is the largest over ranges).
 int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int k,
-                         uint64_t* dids, double* dscores, uint32_t ostride, bool fp8) {
+                         uint64_t* dids, double* dscores, uint32_t ostride, bool fp8,
+                         const double* hQ) {
   int rc;
   if (nr < 1 || nr > 3) {
     set_error(SVDB_EINVAL, "one to three query ranges");
@@ -1170,13 +1176,12 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   if ((rc = scratch(&c_->s_beta_, &c_->s_beta_n_, (size_t)nq * sizeof(float)))) return rc;
   // fail counts (one per range) then each range's fail list at nr + soff
   if ((rc = scratch(&c_->s_fail_, &c_->s_fail_n_, ((size_t)nq + nr) * sizeof(uint32_t)))) return rc;
-  if ((rc = scratch(&c_->s_err_, &c_->s_err_n_, (size_t)nq * sizeof(double)))) return rc;
   // (a range's lists sit at soff * k, k the largest over ranges)
   if ((rc = scratch(&c_->s_lk_, &c_->s_lk_n_, (size_t)nq * k * sizeof(uint64_t)))) return rc;
   if ((rc = scratch(&c_->s_ls_, &c_->s_ls_n_, (size_t)nq * k * sizeof(uint32_t)))) return rc;
   if ((rc = scratch(&c_->s_km_, &c_->s_km_n_, (size_t)nq * sizeof(float)))) return rc;
   if (!c_->h_fail_) HIPCHK(hipHostMalloc((void**)&c_->h_fail_, sizeof(uint32_t)), "hipHostMalloc");
-  const size_t io_b = round_up(nr * sizeof(uint32_t), 64) + (size_t)nq * sizeof(double);
+  const size_t io_b = (size_t)nq * sizeof(double);
   if (c_->h_io_n_ < io_b) {
     if (c_->h_io_) (void)hipHostFree(c_->h_io_);
     c_->h_io_ = nullptr;
@@ -1184,16 +1189,15 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     HIPCHK(hipHostMalloc(&c_->h_io_, round_up(io_b, 4096)), "hipHostMalloc");
     c_->h_io_n_ = round_up(io_b, 4096);
   }
-  uint32_t* h_counts = static_cast<uint32_t*>(c_->h_io_);
-  double* h_err = reinterpret_cast<double*>(static_cast<char*>(c_->h_io_) + round_up(nr * sizeof(uint32_t), 64));
   if ((rc = sync_alive())) return rc;
   if ((rc = refresh_degen())) return rc;
 
   // query prep, every range in one launch: a range's slots run to the next
   // range (the last's to nq_pad), the slots past its queries flagged as
-  // padding.  It also clears the error report and the fail counts.
-  QueryPrepArgs pq{dQ, ldq, nq_pad, (uint32_t)d_, dp, fp8 ? sh8_.rho_bits : sh_.rho_bits,
-                   c_->s_qb_, (QParams*)c_->s_qp_, (double*)c_->s_err_, nq,
+  // padding.  It also clears the fail counts, and brings queries the caller has
+  // in host memory to the device.
+  QueryPrepArgs pq{hQ ? hQ : dQ, ldq, nq_pad, (uint32_t)d_, dp, fp8 ? sh8_.rho_bits : sh_.rho_bits,
+                   c_->s_qb_, (QParams*)c_->s_qp_, hQ ? const_cast<double*>(dQ) : nullptr,
                    (uint32_t*)c_->s_fail_, nr, {}, {}, {}, {}};
   for (int i = 0; i < nr; i++) {
     pq.metric[i] = R[i].metric;
@@ -1220,27 +1224,38 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   LowpScanArgs sa{fp8 ? (const uint16_t*)sh8_.X8 : sh_.Xb, dp, nullptr, nullptr, nullptr,
                   nullptr, (const uint16_t*)c_->s_qb_, (const QParams*)c_->s_qp_, nq, 0, 0,
                   nrows_pad, 0, (float*)c_->s_ck_, (uint2*)c_->s_ck_, (uint2*)c_->s_cs_, nullptr, 0};
+  // a scan group's queries and row arrays
+  auto group_args = [&](const ScanGroup& g) {
+    const bool mk = g.metric == kMixed;
+    LowpScanArgs x = sa;
+    x.w0 = mk ? sh_.nx : w0_of(g.metric);
+    x.w1 = mk ? sh_.pen : w1_of(g.metric);
+    x.w2 = mk ? sh_.xn : nullptr;
+    x.w3 = mk ? sh_.inv : nullptr;
+    x.Qb = (const uint16_t*)((const unsigned char*)c_->s_qb_ + (size_t)g.soff * dp * qbytes);
+    x.qp = (const QParams*)c_->s_qp_ + g.soff;
+    x.nq = g.n;
+    return x;
+  };
   if (pre) {
     prof_begin(SVDB_K_PREPASS);
-    for (int i = 0; i < nr; i++) {
-      LowpScanArgs pa = sa;
-      pa.w0 = w0_of(R[i].metric);
-      pa.w1 = w1_of(R[i].metric);
-      pa.w2 = pa.w3 = nullptr;
-      pa.Qb = (const uint16_t*)((const unsigned char*)c_->s_qb_ + (size_t)R[i].soff * dp * qbytes);
-      pa.qp = (const QParams*)c_->s_qp_ + R[i].soff;
-      pa.nq = R[i].n;
+    for (const ScanGroup& g : sgs) {
+      if (g.n == 0) continue;
+      LowpScanArgs pa = group_args(g);
       pa.rows_per_slice = tp * kLowpTile;
       pa.slice_stride = (tiles / ns_pre) * kLowpTile;
       pa.NL = NL_pre;
-      pa.cand_key = (float*)c_->s_ck_ + (size_t)R[i].soff * NL_pre;
-      HIPCHK(scan(pa, R[i].metric, ns_pre, true), "first-pass scan (sample)");
-      // thresholds in c_->s_beta_, read by the main scan before the shortlist
-      // below overwrites them (padding slots' values are never used)
-      HIPCHK(launch_kth_key((const float*)c_->s_ck_ + (size_t)R[i].soff * NL_pre, R[i].n, NL_pre,
-                            thr_rank(R[i].k), (float*)c_->s_beta_ + R[i].soff, c_->stream),
-             "k_kth_key");
+      pa.cand_key = (float*)c_->s_ck_ + (size_t)g.soff * NL_pre;
+      HIPCHK(scan(pa, g.metric, ns_pre, true), "first-pass scan (sample)");
     }
+    // thresholds in c_->s_beta_, read by the main scan before the shortlist
+    // below overwrites them (padding slots' values are never used)
+    KthArgs ka{(const float*)c_->s_ck_, (float*)c_->s_beta_, nq, NL_pre, nr, {}, {}};
+    for (int i = 0; i < nr; i++) {
+      ka.first[i] = R[i].soff;
+      ka.rank[i] = thr_rank(R[i].k);
+    }
+    HIPCHK(launch_kth_key(ka, c_->stream), "k_kth_key");
     prof_end(SVDB_K_PREPASS);
     sa.tau0 = (const float*)c_->s_beta_;
     sa.tau0_stride = 1;
@@ -1249,15 +1264,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   for (const ScanGroup& g : sgs) {
     if (g.n == 0) continue;
     const LowpRange& r = R[g.r0];
-    const bool mk = g.metric == kMixed;
-    LowpScanArgs ma = sa;
-    ma.w0 = mk ? sh_.nx : w0_of(g.metric);
-    ma.w1 = mk ? sh_.pen : w1_of(g.metric);
-    ma.w2 = mk ? sh_.xn : nullptr;
-    ma.w3 = mk ? sh_.inv : nullptr;
-    ma.Qb = (const uint16_t*)((const unsigned char*)c_->s_qb_ + (size_t)g.soff * dp * qbytes);
-    ma.qp = (const QParams*)c_->s_qp_ + g.soff;
-    ma.nq = g.n;
+    LowpScanArgs ma = group_args(g);
     ma.rows_per_slice = ma.slice_stride = r.rps;
     ma.NL = r.NL;
     ma.hdr = (uint2*)c_->s_ck_ + r.coff;
@@ -1293,7 +1300,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
                       w1_of(rg.metric), rg.n, width(rg.k), (uint32_t)rg.k, ostride,
                       dids + (size_t)rg.qoff * ostride, dscores + (size_t)rg.qoff * ostride,
                       (uint32_t*)c_->s_fail_ + ri, const_cast<uint32_t*>(fl),
-                      (double*)c_->s_err_ + rg.soff, nullptr,
+                      (double*)c_->h_io_ + rg.soff, nullptr,
                       (uint64_t*)c_->s_lk_ + (size_t)rg.soff * k,
                       (uint32_t*)c_->s_ls_ + (size_t)rg.soff * k, (float*)c_->s_km_ + rg.soff, 0};
   };
@@ -1306,10 +1313,6 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   prof_begin(SVDB_K_RERANK);
   HIPCHK(launch_rerank_ranges(ras.data(), rms.data(), nr, c_->stream), "k_rerank");
   prof_end(SVDB_K_RERANK);
-  HIPCHK(hipMemcpyAsync(h_counts, c_->s_fail_, nr * sizeof(uint32_t), hipMemcpyDeviceToHost, c_->stream),
-         "copy");
-  HIPCHK(hipMemcpyAsync(h_err, c_->s_err_, (size_t)nq * sizeof(double), hipMemcpyDeviceToHost, c_->stream),
-         "copy");
   // what lowp_complete needs once the counts are back
   SearchCtx::LowpPending& lp = c_->lp;
   lp.on = true;
@@ -1322,9 +1325,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   lp.dscores = dscores;
   lp.ostride = ostride;
   lp.fp8 = fp8;
-  lp.nq = nq;
   lp.shortlist = shortlist;
-  lp.failed = false;
   return SVDB_OK;
 }
 
@@ -1344,7 +1345,6 @@ int Engine::lowp_complete() {
   double* dscores = lp.dscores;
   const uint32_t ostride = lp.ostride;
   const bool fp8 = lp.fp8;
-  const uint32_t nq = lp.nq;
   auto width = [&](int kk) { return lowp_width(kk, fp8, lp.shortlist); };
   auto w0_of = [&](int m) {
     return fp8 ? (m == kL2 ? sh8_.nx : m == kDot ? sh8_.xn : sh8_.inv)
@@ -1366,18 +1366,23 @@ int Engine::lowp_complete() {
                       w1_of(rg.metric), rg.n, width(rg.k), (uint32_t)rg.k, ostride,
                       dids + (size_t)rg.qoff * ostride, dscores + (size_t)rg.qoff * ostride,
                       (uint32_t*)c_->s_fail_ + ri, const_cast<uint32_t*>(fl),
-                      (double*)c_->s_err_ + rg.soff, nullptr,
+                      (double*)c_->h_io_ + rg.soff, nullptr,
                       (uint64_t*)c_->s_lk_ + (size_t)rg.soff * lp.k,
                       (uint32_t*)c_->s_ls_ + (size_t)rg.soff * lp.k, (float*)c_->s_km_ + rg.soff,
                       0};
   };
-  uint32_t* h_counts = static_cast<uint32_t*>(c_->h_io_);
-  double* h_err = reinterpret_cast<double*>(static_cast<char*>(c_->h_io_) +
-                                            round_up(nr * sizeof(uint32_t), 64));
+  // the error report, written by the reranks in host memory (-1: the query is
+  // not certified)
+  const double* h_err = static_cast<const double*>(c_->h_io_);
   HIPCHK(hipStreamSynchronize(c_->stream), "lowp");
   double mx = 0.0;
-  for (uint32_t i = 0; i < nq; i++) mx = std::max(mx, h_err[i]);
-  std::vector<uint32_t> nfail(h_counts, h_counts + nr);
+  std::vector<uint32_t> nfail(nr, 0);
+  for (int ri = 0; ri < nr; ri++)
+    for (uint32_t i = 0; i < R[ri].n; i++) {
+      const double e = h_err[R[ri].soff + i];
+      nfail[ri] += e < 0.0;
+      mx = std::max(mx, e);
+    }
   for (int ri = 0; ri < nr; ri++) {
     const LowpRange& rg = R[ri];
     const int metric = rg.metric;
@@ -1388,8 +1393,6 @@ int Engine::lowp_complete() {
     const uint32_t nf1 = nfail[ri];
     st_.certified += nqr - nf1;
     if (nf1 == 0) continue;
-    c_->lp.failed = true;  // (restored below for the caller's record)
-    lp.failed = true;
     // this range's views: slot-space arrays at soff, query-space at qoff
     const double* rQ = dQ + (size_t)rg.qoff * ldq;
     uint64_t* rids = dids + (size_t)rg.qoff * ostride;
@@ -1475,14 +1478,8 @@ int Engine::lowp_complete() {
       }
     }
     // the error report again, now with the widened queries certified
-    if (nf != nf1) {
-      double* he = reinterpret_cast<double*>(static_cast<char*>(c_->h_io_) +
-                                             round_up(nr * sizeof(uint32_t), 64));
-      HIPCHK(hipMemcpyAsync(he, (double*)c_->s_err_ + rg.soff, nqr * sizeof(double),
-                            hipMemcpyDeviceToHost, c_->stream), "copy");
-      HIPCHK(hipStreamSynchronize(c_->stream), "copy");
-      for (uint32_t i = 0; i < nqr; i++) mx = std::max(mx, he[i]);
-    }
+    if (nf != nf1)
+      for (uint32_t i = 0; i < nqr; i++) mx = std::max(mx, h_err[rg.soff + i]);
     st_.certified += nf1 - nf;
     st_.widened += nf1 - nf;
     if (nf == 0) continue;
@@ -1533,21 +1530,8 @@ int Engine::lowp_complete() {
     st_.fallbacks += nf;
   }
   st_.last_max_rel_err = mx;
-  c_->lp.failed = lp.failed;
   return SVDB_OK;
 }
-
-int Engine::run_lowp_ranges(const double* dQ, size_t ldq, LowpRange* R, int nr, int k,
-                            uint64_t* dids, double* dscores, uint32_t ostride, bool fp8) {
-  int rc = lowp_enqueue(dQ, ldq, R, nr, k, dids, dscores, ostride, fp8);
-  if (rc) {
-    c_->lp.on = false;
-    return rc;
-  }
-  return lowp_complete();
-}
-
-
 
 int Engine::use_lowp(int precision, size_t D, int* rc) {
   *rc = SVDB_OK;
@@ -1947,8 +1931,6 @@ int Engine::search_begin_locked(SearchCtx& c, const double* Q, size_t nq, size_t
     }
     const size_t n = sel.size();
     if ((rc = scratch(&c.s_q_, &c.s_q_n_, n * D * sizeof(double)))) return rc;
-    if ((rc = scratch(&c.s_ids_, &c.s_ids_n_, n * kmax_all * sizeof(uint64_t)))) return rc;
-    if ((rc = scratch(&c.s_sc_, &c.s_sc_n_, n * kmax_all * sizeof(double)))) return rc;
     if (!host_bufs(n, kmax_all)) {
       set_error(SVDB_ENOMEM, "pinned staging unavailable");
       return SVDB_ENOMEM;
@@ -1961,22 +1943,18 @@ int Engine::search_begin_locked(SearchCtx& c, const double* Q, size_t nq, size_t
     c.scores = scores;
     c.pid = pid;
     c.psc = psc;
+    // No copies: the first kernel reads the queries in the pinned staging, and
+    // the reranks (and the retries) write ids, scores and the error report
+    // there.  Five copies took some 4 µs each on the stream (500k × 128, 64
+    // queries: 146 µs a call with them, 130 without).
     for (size_t t = 0; t < n; t++) std::memcpy(pq + t * D, Q + sel[t] * ldq, D * sizeof(double));
-    HIPCHK(hipMemcpyAsync(c.s_q_, pq, n * D * sizeof(double), hipMemcpyHostToDevice, c.stream),
-           "q upload");
-    rc = lowp_enqueue((const double*)c.s_q_, D, R, nr, (int)kmax_all, (uint64_t*)c.s_ids_,
-                      (double*)c.s_sc_, (uint32_t)kmax_all, false);
+    rc = lowp_enqueue((const double*)c.s_q_, D, R, nr, (int)kmax_all, pid, psc,
+                      (uint32_t)kmax_all, false, pq);
     if (rc) {
       c.lp.on = false;
       (void)hipStreamSynchronize(c.stream);
       return rc;
     }
-    // the results of every query the first pass certifies (in practice all
-    // of them): downloaded now, before anyone waits
-    HIPCHK(hipMemcpyAsync(pid, c.s_ids_, n * kmax_all * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                          c.stream), "ids download");
-    HIPCHK(hipMemcpyAsync(psc, c.s_sc_, n * kmax_all * sizeof(double), hipMemcpyDeviceToHost,
-                          c.stream), "scores download");
     c.state = 1;
     return SVDB_OK;
   }
@@ -1989,27 +1967,37 @@ int Engine::search_begin_locked(SearchCtx& c, const double* Q, size_t nq, size_t
       size_t kmax = 0;
       for (size_t t = 0; t < n; t++) kmax = std::max(kmax, k[sel[b0 + t]]);
       if ((rc = scratch(&c.s_q_, &c.s_q_n_, n * D * sizeof(double)))) return rc;
-      if ((rc = scratch(&c.s_k_, &c.s_k_n_, n * sizeof(int)))) return rc;
-      if ((rc = scratch(&c.s_ids_, &c.s_ids_n_, n * kmax * sizeof(uint64_t)))) return rc;
-      if ((rc = scratch(&c.s_sc_, &c.s_sc_n_, n * kmax * sizeof(double)))) return rc;
       const bool pinned = host_bufs(n, kmax);
+      // (a first pass through the pinned staging, as above; rows past 256 wide
+      // are copied to the device, where one load's way over the bus would
+      // repeat for every 256 columns)
+      const bool direct = lowp && pinned, upload = !direct || D > 256;
+      if (!direct) {
+        if ((rc = scratch(&c.s_k_, &c.s_k_n_, n * sizeof(int)))) return rc;
+        if ((rc = scratch(&c.s_ids_, &c.s_ids_n_, n * kmax * sizeof(uint64_t)))) return rc;
+        if ((rc = scratch(&c.s_sc_, &c.s_sc_n_, n * kmax * sizeof(double)))) return rc;
+      }
+      uint64_t* oid = direct ? pid : (uint64_t*)c.s_ids_;
+      double* osc = direct ? psc : (double*)c.s_sc_;
       for (size_t t = 0; t < n; t++) {
         const size_t i = sel[b0 + t];
         std::memcpy(pq + t * D, Q + i * ldq, D * sizeof(double));
         pk[t] = (int)k[i];
       }
       auto enqueue = [&]() -> int {
-        HIPCHK(hipMemcpyAsync(c.s_q_, pq, n * D * sizeof(double), hipMemcpyHostToDevice,
-                              c.stream), "q upload");
-        HIPCHK(hipMemcpyAsync(c.s_k_, pk, n * sizeof(int), hipMemcpyHostToDevice, c.stream),
-               "k upload");
+        if (upload)
+          HIPCHK(hipMemcpyAsync(c.s_q_, pq, n * D * sizeof(double), hipMemcpyHostToDevice,
+                                c.stream), "q upload");
+        if (!lowp)
+          HIPCHK(hipMemcpyAsync(c.s_k_, pk, n * sizeof(int), hipMemcpyHostToDevice, c.stream),
+                 "k upload");
         const int r = lowp ? run_lowp((const double*)c.s_q_, D, (uint32_t)n, m, (int)kmax,
-                                      (uint64_t*)c.s_ids_, (double*)c.s_sc_, (uint32_t)kmax,
-                                      which == 2)
+                                      oid, osc, (uint32_t)kmax, which == 2,
+                                      upload ? nullptr : pq)
                            : run_exact((const double*)c.s_q_, D, (uint32_t)n, (uint32_t)D,
-                                       (const int*)c.s_k_, m, (int)kmax, (uint64_t*)c.s_ids_,
-                                       (double*)c.s_sc_, (uint32_t)kmax);
-        if (r) return r;
+                                       (const int*)c.s_k_, m, (int)kmax, oid, osc,
+                                       (uint32_t)kmax);
+        if (r || direct) return r;
         HIPCHK(hipMemcpyAsync(pid, c.s_ids_, n * kmax * sizeof(uint64_t),
                               hipMemcpyDeviceToHost, c.stream), "ids download");
         HIPCHK(hipMemcpyAsync(psc, c.s_sc_, n * kmax * sizeof(double), hipMemcpyDeviceToHost,
@@ -2056,13 +2044,6 @@ int Engine::search_complete(SearchCtx& c) {
   int rc = lowp_complete();
   if (rc) return c.rc = rc;
   const size_t n = c.sel.size(), kk = c.kmax;
-  if (c.lp.failed) {
-    // retries rewrote some queries' results on the device
-    HIPCHK(hipMemcpyAsync(c.pid, c.s_ids_, n * kk * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                          c.stream), "ids download");
-    HIPCHK(hipMemcpyAsync(c.psc, c.s_sc_, n * kk * sizeof(double), hipMemcpyDeviceToHost,
-                          c.stream), "scores download");
-  }
   HIPCHK(hipStreamSynchronize(c.stream), "search");
   prof_collect();
   for (size_t t = 0; t < n; t++) {

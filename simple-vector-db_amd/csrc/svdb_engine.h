@@ -164,18 +164,19 @@ class Engine {
     int metric;
     uint32_t qoff, n;  // query rows qoff .. qoff+n-1
     int k;             // neighbours wanted (0: the call's k)
-    uint32_t soff;     // first slot (set by run_lowp_ranges)
+    uint32_t soff;     // first slot (set by lowp_enqueue)
     // first-pass row slicing of this range's scan and where its candidate
-    // lists start (set by run_lowp_ranges)
+    // lists start (set by lowp_enqueue)
     uint32_t ns, rps, NL;
     uint32_t pass;         // rows its threshold lets into the lists, about (0: no threshold)
     size_t coff;
   };
   static uint32_t lowp_width(int kk, bool fp8, size_t shortlist);
+  // hQ: the queries in pinned host memory, from where the first kernel brings
+  // them to dQ (else they are in dQ already).  dids and dscores may be pinned
+  // host memory.
   int run_lowp(const double* dQ, size_t ldq, uint32_t nq, int metric, int k, uint64_t* dids,
-               double* dscores, uint32_t ostride, bool fp8);
-  int run_lowp_ranges(const double* dQ, size_t ldq, LowpRange* R, int nr, int k, uint64_t* dids,
-                      double* dscores, uint32_t ostride, bool fp8);
+               double* dscores, uint32_t ostride, bool fp8, const double* hQ = nullptr);
   // 0: FP64 scan, 1: BF16 first pass, 2: FP8 first pass
   int use_lowp(int precision, size_t D, int* rc);
   int alloc_shadow(size_t cap);
@@ -251,7 +252,6 @@ class Engine {
     void* s_ss_ = nullptr;     size_t s_ss_n_ = 0;
     void* s_beta_ = nullptr;   size_t s_beta_n_ = 0;
     void* s_fail_ = nullptr;   size_t s_fail_n_ = 0;
-    void* s_err_ = nullptr;    size_t s_err_n_ = 0;
     void* s_lk_ = nullptr;     size_t s_lk_n_ = 0;    // uncertified queries' lists: keys
     void* s_ls_ = nullptr;     size_t s_ls_n_ = 0;    //   slots
     void* s_km_ = nullptr;     size_t s_km_n_ = 0;    //   shortlists' largest key
@@ -268,7 +268,7 @@ class Engine {
     void* s_cid_ = nullptr;    size_t s_cid_n_ = 0;   //   their ids
     void* s_csc_ = nullptr;    size_t s_csc_n_ = 0;   //   and scores
     uint32_t* h_fail_ = nullptr;  // pinned: fail count
-    void* h_io_ = nullptr;        // pinned: per-range fail counts + first-pass errors
+    void* h_io_ = nullptr;        // pinned: the first pass's error report
     size_t h_io_n_ = 0;
     void* h_stage_ = nullptr;     // pinned: search staging
     size_t h_stage_n_ = 0;
@@ -284,9 +284,7 @@ class Engine {
       double* dscores = nullptr;
       uint32_t ostride = 0;
       bool fp8 = false;
-      uint32_t nq = 0;  // slots
       size_t shortlist = 0;
-      bool failed = false;  // some query went through a retry (set by lowp_complete)
     } lp;
     // an asynchronous search (search_begin): 0 idle, 1 enqueued, 2 completed
     int state = 0;
@@ -318,7 +316,7 @@ class Engine {
   uint64_t* near_host_ = nullptr;   // pinned: its answer (id, seq)
   uint64_t near_seq_ = 0;
   int lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int k, uint64_t* dids,
-                   double* dscores, uint32_t ostride, bool fp8);
+                   double* dscores, uint32_t ostride, bool fp8, const double* hQ = nullptr);
   int lowp_complete();
   int search_begin_locked(SearchCtx& c, const double* Q, size_t nq, size_t ldq, size_t D,
                           const size_t* k, const int* metric, int precision, size_t ostride,

@@ -137,7 +137,8 @@ struct RerankArgs {
   double* scores;
   uint32_t* fail_count;     // queries not certified
   uint32_t* fail_list;      // their indices
-  double* max_rel_err;      // [nq] first-pass score error of the returned scores
+  double* max_rel_err;      // [nq] first-pass score error of the returned scores (first
+                            // stage: -1 for a query not certified); host memory
   const uint32_t* qidx;     // optional: shortlist row i is query qidx[i]
   // Optional carried state, indexed by query q: a stage's top k (FP64
   // ordering keys lk[q*k ..], slots ls[q*k ..]) and kmax[q], the largest
@@ -172,8 +173,7 @@ struct QueryPrepArgs {
   const uint32_t* rho_bits;
   void* Qb;              // [nslots][dp] BF16 or e4m3 query rows
   QParams* qp;           // [nslots]
-  double* err;           // [nerr] first-pass error report, zeroed here
-  uint32_t nerr;
+  double* Qd;            // optional: Q's rows are copied here (same stride)
   uint32_t* fail_count;  // [nr] zeroed here
   int nr;
   int metric[3];
@@ -184,9 +184,17 @@ hipError_t launch_query_prep(const QueryPrepArgs& a, hipStream_t s);
 hipError_t launch_scan_bf16(const LowpScanArgs& a, int metric, uint32_t nslices, bool minonly,
                             hipStream_t s);
 // thr[q] = the L-th smallest of the n keys key[q*n .. q*n+n) (+inf when
-// fewer than L are finite).  One wavefront per query.
-hipError_t launch_kth_key(const float* key, uint32_t nq, uint32_t n, uint32_t L, float* thr,
-                          hipStream_t s);
+// fewer than L are finite), L = rank[i] for the queries of range i (those
+// from first[i] to first[i + 1], the last to nq).  One wavefront per query.
+constexpr int kKthRanges = 3;
+struct KthArgs {
+  const float* key;
+  float* thr;
+  uint32_t nq, n;
+  int nr;
+  uint32_t first[kKthRanges], rank[kKthRanges];
+};
+hipError_t launch_kth_key(const KthArgs& a, hipStream_t s);
 // ---- wide rows (svdb_wide.hip): BF16 at padded widths 512 and 768 ----
 bool bf16_wide_dp_supported(size_t dp);
 hipError_t launch_scan_bf16_wide(const LowpScanArgs& a, int metric, uint32_t nslices,

@@ -32,12 +32,13 @@ __device__ __forceinline__ PrepSlot prep_slot(const QueryPrepArgs& a, uint32_t s
   return i < a.n[r] ? PrepSlot{r, a.qoff[r] + i} : PrepSlot{-1, 0};
 }
 
-// Stages row q (d columns, zeros up to `cols`) and returns its canonical
+// Stages row q (d columns, zeros up to `cols`; copied to qd unless that is
+// null) and returns its canonical
 // Σ fma(v, v, ·) (the zeros beyond d leave a chain's bits as they are),
 // max |v| and whether every element is finite, the same in every lane.
-__device__ __forceinline__ double prep_stage(const double* __restrict__ q, uint32_t d,
-                                             uint32_t cols, double* row, int lane,
-                                             double& maxabs, bool& finite) {
+__device__ __forceinline__ double prep_stage(const double* __restrict__ q,
+                                             double* __restrict__ qd, uint32_t d, uint32_t cols,
+                                             double* row, int lane, double& maxabs, bool& finite) {
   double mx = 0.0;
   bool fin = true;
   for (uint32_t c0 = 0; c0 < cols; c0 += 256) {
@@ -51,6 +52,7 @@ __device__ __forceinline__ double prep_stage(const double* __restrict__ q, uint3
     for (int j = 0; j < 4; j++) {
       const uint32_t c = c0 + j * 64 + lane;
       if (c < cols) row[c] = v[j];
+      if (qd && c < d) qd[c] = v[j];
       fin = fin && isfinite(v[j]);
       mx = fmax(mx, fabs(v[j]));
     }

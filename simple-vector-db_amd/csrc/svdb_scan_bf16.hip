@@ -388,15 +388,9 @@ __global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
 template <int METRIC, int KS, int QF>
 static hipError_t scan_bf16_t(const LowpScanArgs& a, uint32_t nslices, bool minonly,
                               hipStream_t s) {
-  // the mixed scan has no pre-pass form: the engine runs the pre-pass per
-  // metric range with the single-metric kernels
-  if constexpr (METRIC == kMixed) {
-    if (minonly) return hipErrorInvalidValue;
-  }
   auto fn = a.tau0 ? k_scan_bf16<METRIC, KS, QF, kFormAppend>
                    : k_scan_bf16<METRIC, KS, QF, kFormSorted>;
-  if constexpr (METRIC != kMixed)
-    if (minonly) fn = k_scan_bf16<METRIC, KS, QF, kFormMin>;
+  if (minonly) fn = k_scan_bf16<METRIC, KS, QF, kFormMin>;
   constexpr size_t shm = 0;  // both tile buffers are static LDS
   const uint32_t qpb = kLowpWaves * QF * 16;
   // nslices is a multiple of 8 (one set of slices per XCD); 1-D grid.

@@ -203,7 +203,6 @@ __global__ __launch_bounds__(64 * kPrepWaves) void k_query_prep8(QueryPrepArgs a
   const uint32_t d = a.d, cols = (d + 15) & ~15u;
   uint32_t* q8 = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(a.Qb) + (size_t)i * a.dp);
   QParams* qp = a.qp;
-  if (lane == 0 && i < a.nerr) a.err[i] = 0.0;
   QParams p{};
   p.metric = metric;
   if (ps.range < 0) {
@@ -215,7 +214,9 @@ __global__ __launch_bounds__(64 * kPrepWaves) void k_query_prep8(QueryPrepArgs a
   double* row = prep_rows8 + (threadIdx.x >> 6) * cols;
   double maxabs;
   bool finite;
-  const double nq2 = prep_stage(a.Q + (size_t)ps.row * a.ldq, d, cols, row, lane, maxabs, finite);
+  const double nq2 = prep_stage(a.Q + (size_t)ps.row * a.ldq,
+                                a.Qd ? a.Qd + (size_t)ps.row * a.ldq : nullptr, d, cols, row,
+                                lane, maxabs, finite);
   const double sc = metric == kL2 ? -2.0 : -1.0;
   const double qn = sqrt(nq2);
   const double lim = 1152921504606846976.0;  // 2^60
