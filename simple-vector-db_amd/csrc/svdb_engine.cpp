@@ -600,7 +600,7 @@ int Engine::append(const double* rows, size_t n, size_t lds, size_t dim, uint32_
              "row upload");
       HIPCHK(hipStreamSynchronize(stream_), "row upload");
     }
-    HIPCHK(launch_row_norms(X_, ld_, nullptr, (uint32_t)s0, (uint32_t)n, (uint32_t)d_, nx2_, xn_,
+    HIPCHK(launch_row_norms(X_, ld_, (uint32_t)s0, (uint32_t)n, (uint32_t)d_, nx2_, xn_,
                             stream_), "k_row_norms");
     if ((rc = shadow_rows((uint32_t)s0, (uint32_t)n, nullptr))) return rc;
   }
@@ -637,7 +637,7 @@ int Engine::overwrite(size_t logical, const double* row, size_t dim) {
   degen_dirty_ = lowp_ || lowp8_;
   HIPCHK(hipMemcpyAsync(X_ + (size_t)s * ld_, row, d_ * sizeof(double), hipMemcpyHostToDevice,
                         stream_), "row upload");
-  HIPCHK(launch_row_norms(X_, ld_, nullptr, s, 1, (uint32_t)d_, nx2_, xn_, stream_), "k_row_norms");
+  HIPCHK(launch_row_norms(X_, ld_, s, 1, (uint32_t)d_, nx2_, xn_, stream_), "k_row_norms");
   int rc = shadow_rows(s, 1, nullptr);
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(stream_), "overwrite");
@@ -724,7 +724,7 @@ int Engine::compact() {
   if (hipMemcpyAsync(didx, keep.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, stream_) !=
           hipSuccess ||
       launch_gather_rows(X_, ld_, didx, n, (uint32_t)ld_, X, ld_, stream_) != hipSuccess ||
-      launch_row_norms(X, ld_, nullptr, 0, n, (uint32_t)d_, nx2, xn, stream_) != hipSuccess ||
+      launch_row_norms(X, ld_, 0, n, (uint32_t)d_, nx2, xn, stream_) != hipSuccess ||
       hipStreamSynchronize(stream_) != hipSuccess)
     fail("row gather");
   dev_free(didx, ib);

@@ -108,35 +108,12 @@ struct WList {
 
 // ------------------------------------------------------------ store writes
 
-// One thread per row: the sequential fma chain of the squared norm of a row
-// already copied into the master (padding columns are zero).  Rows are the
-// slots first..first+n-1, or slots[0..n) when a slot list is given.
-__global__ void k_row_norms(const double* __restrict__ X, size_t ldx,
-                            const uint32_t* __restrict__ slots, uint32_t first, uint32_t n,
-                            uint32_t d, double* __restrict__ nx2, double* __restrict__ xn) {
-  uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  uint32_t slot = slots ? slots[r] : first + r;
-  const double* x = X + (size_t)slot * ldx;
-  double acc = 0.0;
-  for (uint32_t i = 0; i < d; i++) acc = fma(x[i], x[i], acc);
-  nx2[slot] = acc;
-  xn[slot] = sqrt(acc);
-}
-
-hipError_t launch_row_norms(const double* X, size_t ldx, const uint32_t* slots, uint32_t first,
-                            uint32_t n, uint32_t d, double* nx2, double* xn, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_row_norms, dim3((n + 255) / 256), dim3(256), 0, s, X, ldx, slots, first, n,
-                     d, nx2, xn);
-  return hipGetLastError();
-}
-
-// One wavefront per query: coalesced loads into LDS, 512 columns at a time,
-// then the chain over broadcast reads, 16 columns per step (a thread per query
-// had a load latency per column on the chain: 77 queries of 100 columns 14 µs,
-// now 3).
-__global__ __launch_bounds__(256) void k_query_norms(const double* __restrict__ Q, size_t ldq,
+// ‖·‖ and its square (the sequential fma chain) of n rows of D columns, stored
+// rows or queries.  One wavefront per row: coalesced loads into LDS, 512
+// columns at a time, then the chain over broadcast reads, 16 columns per step.
+// A thread per row had a load latency per column on the chain: 77 rows of 100
+// columns 14 µs, now 3; 500k of 128 columns 770 µs, now 260.
+__global__ __launch_bounds__(256) void k_row_norms(const double* __restrict__ Q, size_t ldq,
                                                      uint32_t nq, uint32_t D,
                                                      double* __restrict__ qn,
                                                      double* __restrict__ qq) {
@@ -174,8 +151,13 @@ __global__ __launch_bounds__(256) void k_query_norms(const double* __restrict__ 
 hipError_t launch_query_norms(const double* Q, size_t ldq, uint32_t nq, uint32_t D, double* qn,
                               double* qq, hipStream_t s) {
   if (nq == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_query_norms, dim3((nq + 3) / 4), dim3(256), 0, s, Q, ldq, nq, D, qn, qq);
+  hipLaunchKernelGGL(k_row_norms, dim3((nq + 3) / 4), dim3(256), 0, s, Q, ldq, nq, D, qn, qq);
   return hipGetLastError();
+}
+
+hipError_t launch_row_norms(const double* X, size_t ldx, uint32_t first, uint32_t n, uint32_t d,
+                            double* nx2, double* xn, hipStream_t s) {
+  return launch_query_norms(X + (size_t)first * ldx, ldx, n, d, xn + first, nx2 + first, s);
 }
 
 // Plain device copy, 16 bytes per lane, grid-stride (also the known-traffic
