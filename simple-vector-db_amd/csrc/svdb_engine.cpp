@@ -1082,7 +1082,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   }
   const bool pre = prepass_ && tiles >= 4 * ns_pre && enough();
   const uint32_t NL_pre = ns_pre * kLowpLanesPerQuery;
-  // Row slices for a scan of grp query blocks wanting kk neighbours: at
+  // Row slices for a scan of n queries wanting kk neighbours: at
   // least 8, more when there are few query blocks, each at least 4 tiles
   // long.  One block per CU fits at a time, so the grid is kept at or just
   // under two rounds of the 256 CUs (a few blocks past a round cost a whole
@@ -1092,7 +1092,13 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // 512 lists per query and for FP8 2,048, which keep the lists' own bound
   // (the smallest 8th entry) clear of the k-th neighbour and of the retries'
   // 4,096th candidate.
-  auto slicing = [&](uint32_t grp, int kk, LowpRange& r) {
+  auto slicing = [&](uint32_t n, int kk, LowpRange& r) {
+    const uint32_t sq = fp8 ? qpb : (uint32_t)lowp_scan_queries(dp, n);
+    const uint32_t grp = (n + sq - 1) / sq;
+    // (blocks of less than the most queries run two to a CU at padded widths
+    // <= 128; up to 256 such queries may have the slices to fill them)
+    const uint32_t round = sq < qpb && dp <= 128 ? 512 : 256;
+    const uint32_t nsmax = round == 512 && n <= 256 ? 512 : 240;
     uint32_t ns = std::max<uint32_t>(8, (512 / grp) & ~7u);
     // rows below the threshold: a lane's smallest of m rows lies below it with
     // probability 1 - (1 - p)^m = j / (number of lanes), p the share of rows
@@ -1102,8 +1108,8 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     if (pre) ns = std::max<uint32_t>(ns, r.pass / (kLowpLC / 2 * kLowpLanesPerQuery));
     else if (fp8) ns = std::max<uint32_t>(ns, 512);
     else if (kk > 32) ns = std::max<uint32_t>(ns, 128);
-    // (a query's lists stay within 128 KiB: 960 lists of 17 words)
-    ns = std::min<uint32_t>(ns, pre ? 240 : 512);
+    // (a query's lists stay within 128 KiB, 960 lists of 17 words, or 272 KiB)
+    ns = std::min<uint32_t>(ns, pre ? nsmax : 512);
     ns = std::max<uint32_t>(1, std::min<uint32_t>(ns, std::max<uint32_t>(1, tiles / 4)));
     // With a threshold more slices cost little, and fill the last round: a
     // round lasts as long as a slice and about 8 tiles' time of starting up
@@ -1112,9 +1118,9 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     // blocks, 8 slices 9.0 ms, 64 4.7).
     if (pre) {
       auto cost = [&](uint32_t n) {
-        return (double)((grp * n + 255) / 256) * (tiles / (double)n + 8);
+        return (double)((grp * n + round - 1) / round) * (tiles / (double)n + 8);
       };
-      for (uint32_t n = (ns & ~7u) + 8; n <= std::min<uint32_t>(240, tiles / 16); n += 8)
+      for (uint32_t n = (ns & ~7u) + 8; n <= std::min<uint32_t>(nsmax, tiles / 16); n += 8)
         if (cost(n) < cost(ns)) ns = n;
     }
     r.rps = (uint32_t)((tiles + ns - 1) / ns) * kLowpTile;
@@ -1150,7 +1156,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     int kg = 0;
     for (int i = g.r0; i < g.r1; i++) kg = std::max(kg, R[i].k);
     LowpRange sl{};
-    slicing((g.n + qpb - 1) / qpb, kg, sl);
+    slicing(g.n, kg, sl);
     for (int i = g.r0; i < g.r1; i++) {
       R[i].ns = sl.ns;
       R[i].rps = sl.rps;

@@ -153,8 +153,10 @@ struct RerankArgs {
   int carry;
 };
 
-// Queries per block of the scan for a padded row length dp.
+// The most queries per block of the scan for a padded row length dp (slots are
+// padded to it), and those of a launch over nq queries.
 int lowp_queries_per_block(size_t dp);
+int lowp_scan_queries(size_t dp, uint32_t nq);
 
 hipError_t launch_shadow_init(const Shadow& sh, uint32_t first, uint32_t n, hipStream_t s);
 hipError_t launch_quantize_rows(const Shadow& sh, const double* X, size_t ldx, const double* nx2,

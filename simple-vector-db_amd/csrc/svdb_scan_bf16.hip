@@ -76,8 +76,9 @@ __device__ __forceinline__ void issue_tile(const LowpScanArgs& a, unsigned char*
 // METRIC kMixed: each wavefront's queries share one metric (QParams.metric
 // of its first slot; the engine aligns metric ranges to wavefronts), read at
 // run time; the tile then carries all four per-row arrays.
+// QF, a wavefront's 16-query fragments, from lowp_scan_queries.
 template <int METRIC, int KS, int QF, int FORM>
-__global__ __launch_bounds__(512) void k_scan_bf16(LowpScanArgs a) {
+__global__ __launch_bounds__(512, (KS <= 2 ? QF <= 2 : KS == 4 && QF == 1) ? 4 : 2) void k_scan_bf16(LowpScanArgs a) {
   constexpr bool MIXED = METRIC == kMixed;
   constexpr bool MINONLY = FORM == kFormMin, SORTED = FORM == kFormSorted;
   constexpr int NAUX = MIXED ? 4 : (METRIC == kCos ? 2 : 1);
@@ -403,9 +404,15 @@ static hipError_t scan_bf16_t(const LowpScanArgs& a, uint32_t nslices, bool mino
 template <int METRIC>
 static hipError_t scan_bf16_m(const LowpScanArgs& a, uint32_t nslices, bool minonly,
                               hipStream_t s) {
+  if (lowp_scan_queries(a.dp, a.nq) == kLowpWaves * 16) switch (a.dp / 32) {
+    case 1: return scan_bf16_t<METRIC, 1, 1>(a, nslices, minonly, s);
+    case 2: return scan_bf16_t<METRIC, 2, 1>(a, nslices, minonly, s);
+    case 4: return scan_bf16_t<METRIC, 4, 1>(a, nslices, minonly, s);
+    case 8: return scan_bf16_t<METRIC, 8, 1>(a, nslices, minonly, s);
+  }
   switch (a.dp / 32) {
-    case 1: return scan_bf16_t<METRIC, 1, 4>(a, nslices, minonly, s);
-    case 2: return scan_bf16_t<METRIC, 2, 4>(a, nslices, minonly, s);
+    case 1: return scan_bf16_t<METRIC, 1, 2>(a, nslices, minonly, s);
+    case 2: return scan_bf16_t<METRIC, 2, 2>(a, nslices, minonly, s);
     case 4: return scan_bf16_t<METRIC, 4, 4>(a, nslices, minonly, s);
     case 8: return scan_bf16_t<METRIC, 8, 2>(a, nslices, minonly, s);
   }
@@ -416,6 +423,24 @@ int lowp_queries_per_block(size_t dp) {
   if (dp > 768) return 4 * 16;           // k_scan_wide, 4 wavefronts of one fragment
   if (dp > 256) return kLowpWaves * 16;  // k_scan_wide, one fragment per wavefront
   return dp / 32 == 8 ? kLowpWaves * 2 * 16 : kLowpQPB;
+}
+
+// Few queries: one fragment per wavefront.  Its share of a tile's MFMAs and tests
+// is then a quarter of four fragments', which no longer fitted beside the
+// tile's load, and its registers let two blocks share a CU at padded widths
+// <= 128, twice the rows in flight (scans of 500k × 128, 64 cosine queries: 58
+// µs with four, 26 with one; 1M × 128, dot: 16 queries 107 and 41, 200 queries
+// 126 with two, 77 with one).
+// Many: as many fragments as the registers hold at padded width 128 and 256
+// (each tile then read from LDS by fewer wavefronts per query), two below, where
+// a tile's MFMAs are so few that a second block per CU is worth more (2M × 32,
+// 16,384 queries: 3.55 ms with four, 3.05 with two; 1M × 128, 8,192 queries:
+// 1.98 and 2.05, and the whole call at 2M × 128, 16,384: 7.4 and 8.5).
+int lowp_scan_queries(size_t dp, uint32_t nq) {
+  const int most = lowp_queries_per_block(dp);
+  if (dp > 256) return most;
+  if (nq <= (dp == 256 ? 128u : 256u)) return kLowpWaves * 16;
+  return dp <= 64 ? kLowpWaves * 2 * 16 : most;
 }
 
 hipError_t launch_scan_bf16(const LowpScanArgs& a, int metric, uint32_t nslices, bool minonly,

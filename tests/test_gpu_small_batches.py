@@ -120,3 +120,28 @@ def test_slices_past_two_rounds(d, nq, k):
         assert np.array_equal(ids, rid), f"{d} {nq} {metric}: ids differ"
         assert np.array_equal(sc.view(np.uint64), rsc.view(np.uint64)), f"{d} {nq} {metric}"
     db.close()
+
+
+@pytest.mark.parametrize("d", [30, 64, 128, 200])
+def test_query_counts_at_the_fragments_edges(d):
+    """Query counts at which the first-pass scan changes the queries of a block
+    and of a wavefront, single-metric and mixed."""
+    rng = np.random.default_rng(d)
+    n = 20_011
+    X = rng.standard_normal((n, d))
+    X[7000:7000 + n // 4] = X[0] + 0.1 * rng.standard_normal((n // 4, d))
+    Q = np.vstack([X[0] + 0.1 * rng.standard_normal((100, d)), rng.standard_normal((157, d))])
+    Q = Q[rng.permutation(257)]
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    want = {m: O.topk(X, Q, 10, m) for m in ("l2", "cos", "dot")}
+    for nq in (16, 17, 128, 129, 256, 257):
+        for m in ("l2", "cos", "dot"):
+            ids, sc = db.search(Q[:nq], 10, m, "bf16")
+            assert np.array_equal(ids, want[m][0][:nq]), f"{d} {nq} {m}"
+            assert np.array_equal(sc, want[m][1][:nq]), f"{d} {nq} {m}"
+        ms = [("l2", "cos", "dot")[i % 3] for i in range(nq)]
+        ids, sc = db.search(Q[:nq], 10, ms, "bf16")
+        for i, m in enumerate(ms):
+            assert np.array_equal(ids[i], want[m][0][i]) and np.array_equal(sc[i], want[m][1][i]), f"{d} {nq} mixed {i}"
+    db.close()
