@@ -1083,8 +1083,9 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   const bool pre = prepass_ && tiles >= 4 * ns_pre && enough();
   const uint32_t NL_pre = ns_pre * kLowpLanesPerQuery;
   // Row slices for a scan of n queries wanting kk neighbours: at
-  // least 8, more when there are few query blocks, each at least 4 tiles
-  // long.  One block per CU fits at a time, so the grid is kept at or just
+  // least 8, more when there are few query blocks, without a threshold each at
+  // least 4 tiles long (with one a slice of a single tile is as good: 60k ×
+  // 1,536, 32 queries, scan 66 µs in 96 slices, 38 in 240).  One block per CU fits at a time, so the grid is kept at or just
   // under two rounds of the 256 CUs (a few blocks past a round cost a whole
   // round).  With a threshold, enough that the rows it lets pass fill a list
   // to half on average (a full list's bound becomes its largest key, which
@@ -1110,7 +1111,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     else if (kk > 32) ns = std::max<uint32_t>(ns, 128);
     // (a query's lists stay within 128 KiB, 960 lists of 17 words, or 272 KiB)
     ns = std::min<uint32_t>(ns, pre ? nsmax : 512);
-    ns = std::max<uint32_t>(1, std::min<uint32_t>(ns, std::max<uint32_t>(1, tiles / 4)));
+    ns = std::max<uint32_t>(1, std::min<uint32_t>(ns, std::max<uint32_t>(1, pre ? tiles : tiles / 4)));
     // With a threshold more slices cost little, and fill the last round: a
     // round lasts as long as a slice and about 8 tiles' time of starting up
     // (scans of 1M × 128, 11,969 queries: 24 blocks of queries, 16 slices and
@@ -1120,7 +1121,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
       auto cost = [&](uint32_t n) {
         return (double)((grp * n + round - 1) / round) * (tiles / (double)n + 8);
       };
-      for (uint32_t n = (ns & ~7u) + 8; n <= std::min<uint32_t>(nsmax, tiles / 16); n += 8)
+      for (uint32_t n = (ns & ~7u) + 8; n <= std::min<uint32_t>(nsmax, tiles); n += 8)
         if (cost(n) < cost(ns)) ns = n;
     }
     r.rps = (uint32_t)((tiles + ns - 1) / ns) * kLowpTile;
