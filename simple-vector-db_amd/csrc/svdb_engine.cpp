@@ -1043,12 +1043,14 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // lie below it (f: the sampled fraction).  The main scan's lists start from
   // it: they then skip nearly every row from the first tile on, and take a
   // few hundred rows per query in all.
-  // BF16: j = 3·L·f, so that about three times the shortlist passes, and at
-  // least 12 + k / 8, whose spread between samples is 28 % (k = 10) to 20 %
-  // (k = 100).  (Each insertion costs the scan: j = L let about L / f rows
-  // pass, k + 16 of a 30th of the store 30·k; 1M × 128 served 512 queries at a
-  // time, k up to 100: 6.9 ms at k + 16, 5.16 so, and as many queries
-  // certified, also where clusters of 40 to 20,000 rows were stored in a row.)
+  // BF16: L·f and two and a half times its spread between samples, so that
+  // hardly any query has fewer than L rows pass, and at least 12 + k / 16, where
+  // the spread is some 25 %.  (Each row that passes costs the scan an insertion:
+  // j = L let about L / f rows pass, k + 16 of a 30th of the store 30·k.  1M ×
+  // 128 served 64 requests a tick, k up to 100: 6.9 ms at k + 16, 5.16 at 3·L·f
+  // and 12 + k / 8, and 4.29 → 4.15 from there to this rule; 2,000 queries, k =
+  // 100: 734 → 692 µs.  As many queries certified each time, also where clusters
+  // of 40 to 20,000 rows were stored in a row.)
   // FP8 keeps j = L: its widening retries look for up to kMaxShort candidates
   // in the lists, and its error band needs them.
   // At least twice j minima: a rank near their number is the largest of them,
@@ -1070,9 +1072,10 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   double frac;
   auto thr_rank = [&](int kk) {
     const uint32_t w = width(kk);
-    return fp8 ? w
-               : std::min<uint32_t>(
-                     w, std::max<uint32_t>((uint32_t)std::ceil(3.0 * w * frac), 12 + kk / 8));
+    if (fp8) return w;
+    const double e = w * frac;
+    return std::min<uint32_t>(w, (uint32_t)std::max(std::ceil(e + 2.5 * std::sqrt(e) + 3.0),
+                                                    12.0 + kk / 16));
   };
   auto enough = [&] { return ns_pre * kLowpLanesPerQuery >= 2 * thr_rank(k); };
   for (;; ns_pre *= 2) {
