@@ -1083,7 +1083,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     frac = (double)ns_pre * tp / std::max<uint32_t>(1, tiles);
     if (enough() || ns_pre >= kPrepassSlices || tiles < 8 * ns_pre) break;
   }
-  const bool pre = prepass_ && tiles >= 4 * ns_pre && enough();
+  bool pre = prepass_ && tiles >= 4 * ns_pre && enough();
   const uint32_t NL_pre = ns_pre * kLowpLanesPerQuery;
   // Row slices for a scan of n queries wanting kk neighbours: at
   // least 8, more when there are few query blocks, without a threshold each at
@@ -1096,7 +1096,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // 512 lists per query and for FP8 2,048, which keep the lists' own bound
   // (the smallest 8th entry) clear of the k-th neighbour and of the retries'
   // 4,096th candidate.
-  auto slicing = [&](uint32_t n, int kk, LowpRange& r) {
+  auto slicing = [&](uint32_t n, int kk, uint32_t cap, LowpRange& r) {
     const uint32_t sq = fp8 ? qpb : (uint32_t)lowp_scan_queries(dp, n);
     const uint32_t grp = (n + sq - 1) / sq;
     // (blocks of less than the most queries run two to a CU at padded widths
@@ -1127,6 +1127,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
       for (uint32_t n = (ns & ~7u) + 8; n <= std::min<uint32_t>(nsmax, tiles); n += 8)
         if (cost(n) < cost(ns)) ns = n;
     }
+    ns = std::min(ns, cap);
     r.rps = (uint32_t)((tiles + ns - 1) / ns) * kLowpTile;
     ns = (nrows_pad + r.rps - 1) / r.rps;
     // one set of slices per XCD: a multiple of 8 (trailing slices may be empty)
@@ -1153,34 +1154,30 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
       sgs.push_back({i, i + 1, mixed_scan ? kMixed : R[i].metric, R[i].soff, 0});
   }
   size_t nlists = 0;  // candidate lists, all groups
-  for (auto& g : sgs) {
-    const LowpRange& last = R[g.r1 - 1];
-    g.n = last.soff + last.n - g.soff;
-    const uint32_t send = g.r1 < nr ? R[g.r1].soff : nq;
-    int kg = 0;
-    for (int i = g.r0; i < g.r1; i++) kg = std::max(kg, R[i].k);
-    LowpRange sl{};
-    slicing(g.n, kg, sl);
-    for (int i = g.r0; i < g.r1; i++) {
-      R[i].ns = sl.ns;
-      R[i].rps = sl.rps;
-      R[i].NL = sl.NL;
-      R[i].pass = sl.pass;
-      R[i].coff = nlists + (size_t)(R[i].soff - g.soff) * sl.NL;
+  auto plan = [&](uint32_t cap) {
+    nlists = 0;
+    for (auto& g : sgs) {
+      const LowpRange& last = R[g.r1 - 1];
+      g.n = last.soff + last.n - g.soff;
+      const uint32_t send = g.r1 < nr ? R[g.r1].soff : nq;
+      int kg = 0;
+      for (int i = g.r0; i < g.r1; i++) kg = std::max(kg, R[i].k);
+      LowpRange sl{};
+      slicing(g.n, kg, cap, sl);
+      for (int i = g.r0; i < g.r1; i++) {
+        R[i].ns = sl.ns;
+        R[i].rps = sl.rps;
+        R[i].NL = sl.NL;
+        R[i].pass = sl.pass;
+        R[i].coff = nlists + (size_t)(R[i].soff - g.soff) * sl.NL;
+      }
+      nlists += (size_t)(send - g.soff) * sl.NL;
     }
-    nlists += (size_t)(send - g.soff) * sl.NL;
-  }
+  };
   // query rows: nq_pad slots plus one block, since a launch over one range
   // (at slot offset soff) reads whole blocks of rows from soff on
   if ((rc = scratch(&c_->s_qb_, &c_->s_qb_n_, ((size_t)nq_pad + qpb) * dp * qbytes))) return rc;
   if ((rc = scratch(&c_->s_qp_, &c_->s_qp_n_, (size_t)nq_pad * sizeof(QParams)))) return rc;
-  // list headers (before them, in the same place, the pre-pass's keys) and
-  // entries
-  if ((rc = scratch(&c_->s_ck_, &c_->s_ck_n_,
-                    std::max(nlists * sizeof(uint2),
-                             pre ? (size_t)nq * NL_pre * sizeof(float) : (size_t)0))))
-    return rc;
-  if ((rc = scratch(&c_->s_cs_, &c_->s_cs_n_, nlists * kLowpLC * sizeof(uint2)))) return rc;
   if ((rc = scratch(&c_->s_sk_, &c_->s_sk_n_, (size_t)nq * L * sizeof(float)))) return rc;
   if ((rc = scratch(&c_->s_ss_, &c_->s_ss_n_, (size_t)nq * L * sizeof(uint32_t)))) return rc;
   if ((rc = scratch(&c_->s_beta_, &c_->s_beta_n_, (size_t)nq * sizeof(float)))) return rc;
@@ -1190,6 +1187,26 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   if ((rc = scratch(&c_->s_lk_, &c_->s_lk_n_, (size_t)nq * k * sizeof(uint64_t)))) return rc;
   if ((rc = scratch(&c_->s_ls_, &c_->s_ls_n_, (size_t)nq * k * sizeof(uint32_t)))) return rc;
   if ((rc = scratch(&c_->s_km_, &c_->s_km_n_, (size_t)nq * sizeof(float)))) return rc;
+  // list headers (before them, in the same place, the pre-pass's keys) and
+  // entries, in what the device-memory budget leaves: half the slices, down to
+  // 8, while it is too little, then no threshold (both only cost certificates)
+  for (uint32_t cap = 512;; cap = cap > 8 ? cap / 2 : 512) {
+    plan(cap);
+    rc = scratch(&c_->s_ck_, &c_->s_ck_n_,
+                 std::max(nlists * sizeof(uint2),
+                          pre ? (size_t)nq * NL_pre * sizeof(float) : (size_t)0));
+    if (!rc) rc = scratch(&c_->s_cs_, &c_->s_cs_n_, nlists * kLowpLC * sizeof(uint2));
+    if (!rc) break;
+    if (rc != SVDB_ENOMEM || (cap <= 8 && !pre)) return rc;
+    (void)hipGetLastError();
+    if (cap <= 8) pre = false;
+    // (the headers' buffer grew first; its room may be what is missing)
+    HIPCHK(hipStreamSynchronize(c_->stream), "sync");
+    scratch_gen_++;
+    dev_free(c_->s_ck_, c_->s_ck_n_);
+    c_->s_ck_ = nullptr;
+    c_->s_ck_n_ = 0;
+  }
   if (!c_->h_fail_) HIPCHK(hipHostMalloc((void**)&c_->h_fail_, sizeof(uint32_t)), "hipHostMalloc");
   const size_t io_b = (size_t)nq * sizeof(double);
   if (c_->h_io_n_ < io_b) {

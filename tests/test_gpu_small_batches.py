@@ -145,3 +145,31 @@ def test_query_counts_at_the_fragments_edges(d):
         for i, m in enumerate(ms):
             assert np.array_equal(ids[i], want[m][0][i]) and np.array_equal(sc[i], want[m][1][i]), f"{d} {nq} mixed {i}"
     db.close()
+
+
+@pytest.mark.parametrize("nq", [40, 3000])
+def test_candidate_lists_within_a_budget(nq):
+    """A device-memory budget that leaves no room for the scan's usual lists:
+    fewer slices, the same answers; without any room the search is refused,
+    and answered again once the budget is lifted."""
+    rng = np.random.default_rng(nq)
+    X = rng.standard_normal((40_007, 64))
+    Q = rng.standard_normal((nq, 64))
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    want = O.topk(X, Q, 10, "l2")
+    lists = nq * 8 * 4 * 17 * 8  # 8 slices' lists
+    rest = nq * (64 * 8 + 64 * 2 + 64 * 8 + 10 * 12 + 256) + (2 << 20)
+    db.set_budget(db.stats()["device_bytes"] + lists + rest)
+    ids, sc = db.search(Q, 10, "l2", "bf16")
+    assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
+    db.close()
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    db.set_budget(db.stats()["device_bytes"] + 4096)
+    with pytest.raises(Exception):
+        db.search(Q, 10, "l2", "bf16")
+    db.set_budget(0)
+    ids, sc = db.search(Q, 10, "l2", "bf16")
+    assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
+    db.close()
