@@ -292,7 +292,15 @@ k_scan_f64_mfma(ScanF64Args a) {
   // query values: the first and second chunk's (QRES), or this stage's and
   // the next one's
   double qa[KS], qb[KS];
+  // (whole stages without a test per value, which the compiler turns into a
+  // branch each)
   auto load_q = [&](double (&v)[KS], uint32_t col0) __attribute__((always_inline)) {
+    if (!QRES && col0 + SC <= a.D) {
+      const double* __restrict__ q = qp + col0 + g;
+#pragma unroll
+      for (int s = 0; s < KS; s++) v[s] = q[4 * s];
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < KS; s++) {
       const uint32_t c = col0 + 4 * s + g;
@@ -652,11 +660,17 @@ hipError_t launch_scan_f64_mfma(const ScanF64Args& a, int metric, int kmax, hipS
   const uint32_t want = ((uint32_t)kmax + 7) / 8;
   uint32_t S = std::max<uint32_t>(a.st.nrows / 1024,
                                   std::min<uint32_t>((want + 7) / 8 * 8, a.st.nrows / 256));
+  // 1/16 of the rows up to 128 columns; wider, where an insertion costs less
+  // beside the products, as much less (300k × 768, 1,024 queries: dot 11.5 ms
+  // with 1/16 and a test per query value, 9.95 so; a share falling with the
+  // square of the width: Euclidean 12.5 → 18.7).
+  const uint32_t c = (a.D + 127) / 128, share = a.st.nrows / (16 * c);
+  if (c > 1) S = std::min(S, std::max((want + 7) / 8 * 8, share / 64));
   S = std::min<uint32_t>({S, kMinsPerLane * 4, a.P * a.kstride / 8}) / 8 * 8;
   if (S && 16 * S >= 2 * (uint32_t)kmax) {
     m.P = S;
     m.slice_stride = a.st.nrows / S / 64 * 64;
-    m.rows_per_slice = std::max<uint32_t>(64, a.st.nrows / 16 / S / 64 * 64);
+    m.rows_per_slice = std::max<uint32_t>(64, share / S / 64 * 64);
     if ((e = scan_f64_mfma_m<true>(m, metric, s)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_bound_f64, dim3((a.nq + 3) / 4), dim3(256), 0, s,
                        reinterpret_cast<const uint32_t*>(a.part_key), 16 * S, a.nq, a.k, a.gtk);
