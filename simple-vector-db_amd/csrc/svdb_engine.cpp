@@ -1091,8 +1091,11 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // 1,536, 32 queries, scan 66 µs in 96 slices, 38 in 240).  One block per CU fits at a time, so the grid is kept at or just
   // under two rounds of the 256 CUs (a few blocks past a round cost a whole
   // round).  With a threshold, enough that the rows it lets pass fill a list
-  // to half on average (a full list's bound becomes its largest key, which
-  // may then lie below the shortlist's); without one, past k = 32 at least
+  // to half on average, for FP8, whose retries certify by the threshold itself,
+  // to a quarter (a full list's bound becomes its largest key, which may then
+  // lie below the shortlist's; 5M × 768 FP8, 4,096 cosine queries, k = 100: the
+  // retries certify 832 with lists half full, 1,679 so, 63.0 → 54.8 ms);
+  // without one, past k = 32 at least
   // 512 lists per query and for FP8 2,048, which keep the lists' own bound
   // (the smallest 8th entry) clear of the k-th neighbour and of the retries'
   // 4,096th candidate.
@@ -1109,7 +1112,8 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     const double m = tp * (double)kLowpTile / kLowpLanesPerQuery;
     r.pass = pre ? (uint32_t)(nrows_pad * -std::expm1(std::log1p(-std::min(0.99, (double)thr_rank(kk) / NL_pre)) / m))
                  : 0;
-    if (pre) ns = std::max<uint32_t>(ns, r.pass / (kLowpLC / 2 * kLowpLanesPerQuery));
+    if (pre)
+      ns = std::max<uint32_t>(ns, r.pass / (kLowpLC / (fp8 ? 4 : 2) * kLowpLanesPerQuery));
     else if (fp8) ns = std::max<uint32_t>(ns, 512);
     else if (kk > 32) ns = std::max<uint32_t>(ns, 128);
     // (a query's lists stay within 128 KiB, 960 lists of 17 words, or 272 KiB)
