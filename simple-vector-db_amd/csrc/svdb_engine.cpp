@@ -946,7 +946,7 @@ int Engine::run_exact_with(const double* dQ, size_t ldq, uint32_t nq, uint32_t D
   if ((rc = sync_alive())) return rc;
   if (metric == kCos || (metric == kL2 && p.mfma))
     HIPCHK(launch_query_norms(dQ, ldq, nq, D, qn, metric == kL2 ? qq : nullptr, c_->stream),
-           "k_query_norms");
+           "k_row_norms");
   if (p.P) {
     if (!p.mfma)
       HIPCHK(launch_fill_i32(reinterpret_cast<int*>(gtk), 2 * nq, -1, c_->stream), "k_fill_i32");
