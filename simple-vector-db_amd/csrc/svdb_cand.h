@@ -26,15 +26,32 @@ namespace svdb {
 // starting threshold (stored as they come).
 enum ScanForm { kFormMin = 0, kFormSorted = 1, kFormAppend = 2 };
 
-// An MFMA's result must not be read by another unit for some wait states after
-// it issued, and the compiler, which inserts them, does not see a read behind a
+// Wait states from an MFMA to another unit's use of its result: passes + 4,
+// v_mfma_f32_16x16x32_bf16 taking 4 passes and FP8's
+// v_mfma_scale_f32_16x16x128_f8f6f4 8.
+constexpr int kBf16States = 8, kFp8States = 12;
+
+// The compiler, which inserts those states, does not always see a read behind a
 // branch that the scans nearly always fall through (the rare insertion): at
 // 1,536 columns accumulators were copied four states after their last MFMA,
 // three too early, and rows were lost.  The scans therefore read a subtile's
 // accumulators behind the next subtile's first MFMAs, which fences hold in
-// front, and let the last subtile's settle here, once per tile.
-__device__ __forceinline__ void settle_mfma(float __attribute__((ext_vector_type(4))) & acc) {
-  asm volatile("s_nop 7" : "+v"(acc));
+// front, and let the last subtile's settle here, once per tile; where those
+// MFMAs are too few for the form's states (FP8 with one fragment) the rest is
+// waited for here too.  What the compiler makes of it is followed through every
+// branch of the built kernels by tests/test_mfma_waits_cpu.py.
+template <int STATES, int QF>
+__device__ __forceinline__ void settle_mfma(float __attribute__((ext_vector_type(4))) (&acc)[QF]) {
+  static_assert(STATES >= 1 && STATES <= 16, "one s_nop");
+  static_assert(QF == 1 || QF == 2 || QF == 4, "every accumulator is named");
+  if constexpr (QF == 1)
+    asm volatile("s_nop %1" : "+v"(acc[0]) : "n"(STATES - 1));
+  else if constexpr (QF == 2)
+    asm volatile("s_nop %2" : "+v"(acc[0]), "+v"(acc[1]) : "n"(STATES - 1));
+  else
+    asm volatile("s_nop %4"
+                 : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])
+                 : "n"(STATES - 1));
 }
 
 __device__ __forceinline__ size_t cand_list(const LowpScanArgs& a, uint32_t q, uint32_t list) {

@@ -37,8 +37,11 @@ __global__ __launch_bounds__(256) void k_mfma_loop(float* __restrict__ out, int 
     for (int i = 0; i < iters; i++)
 #pragma unroll
       for (int t = 0; t < 4; t++) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[t], 0, 0, 0);
+    // (every element: a register the compiler took for free would be written
+    // to while its MFMA is in flight)
 #pragma unroll
-    for (int t = 0; t < 4; t++) s += (float)(acc[t][0] + acc[t][3]);
+    for (int t = 0; t < 4; t++)
+      s += (float)((acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3]));
   } else if constexpr (KIND == 1) {
     f32x4_t acc[4];
 #pragma unroll

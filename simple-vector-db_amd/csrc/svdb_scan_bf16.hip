@@ -310,7 +310,7 @@ __global__ __launch_bounds__(512, (KS <= 2 ? QF <= 2 : KS == 4 && QF == 1) ? 4 :
           }
 #pragma unroll
           for (int f = 0; f < QF; f++) pacc[f] = acc[f];
-          if (sub == kLowpTile / 16 - 1) settle_mfma(pacc[QF - 1]);
+          if (sub == kLowpTile / 16 - 1) settle_mfma<kBf16States>(pacc);
           pw = w;
           ppen = pen;
           prow = trow + rl;
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(512, (KS <= 2 ? QF <= 2 : KS == 4 && QF == 1) ? 4 :
           }
 #pragma unroll
           for (int f = 0; f < QF; f++) pacc[f] = acc[f];
-          if (sub == kLowpTile / 16 - 1) settle_mfma(pacc[QF - 1]);
+          if (sub == kLowpTile / 16 - 1) settle_mfma<kBf16States>(pacc);
           pw = w;
           ppen = pen;
           prow = trow + rl;

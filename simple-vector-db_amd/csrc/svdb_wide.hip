@@ -344,6 +344,7 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
   constexpr int LP = kLowpLP;
   constexpr bool COS = METRIC == kCos;
   constexpr bool MINONLY = FORM == kFormMin, SORTED = FORM == kFormSorted;
+  constexpr int STATES = BF ? kBf16States : kFp8States;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -544,6 +545,9 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
                                                                         0, 127, 0, 127);
             }
           }
+          // (one FP8 MFMA lies between; the chain on its result waits longer)
+          if constexpr (!BF && QF == 1)
+            if (ks == 1) settle_mfma<STATES - 1>(pacc);
 #pragma unroll
           for (int f = 0; f < QF; f++)
             if (f + 1 == ks || (ks == KS - 1 && f + 1 > ks)) need |= need_of(pacc, f, pw0, pw1);
@@ -562,7 +566,7 @@ __global__ __launch_bounds__(64 * NW) void k_scan_wide(LowpScanArgs a) {
         const int rl = sub * 16 + rg * 4;
 #pragma unroll
         for (int f = 0; f < QF; f++) pacc[f] = acc[f];
-        if (sub == NSUB - 1) settle_mfma(pacc[QF - 1]);
+        if (sub == NSUB - 1) settle_mfma<STATES>(pacc);
         pw0 = *reinterpret_cast<const float4*>(aux + rl);
         pw1 = *reinterpret_cast<const float4*>(aux + G::TR + rl);
         prow = trow + rl;

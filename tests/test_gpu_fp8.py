@@ -271,3 +271,24 @@ def test_fp8_retries_with_exact_ties():
             say(f"  widened {s1['widened'] - s0['widened']}, second pass "
                 f"{s1['second_pass'] - s0['second_pass']}, fp64 {s1['fallbacks'] - s0['fallbacks']}")
     db.close()
+
+
+@pytest.mark.parametrize("d", [600, 769, 1000, 1024, 1400])
+def test_fp8_lists_without_a_threshold(d):
+    """A store too small for the sample's threshold, its rows stored farthest
+    first, so that every subtile of the scan brings rows into the lists."""
+    rng = np.random.default_rng(d)
+    n, nq = 1500, 33
+    c = rng.standard_normal(d)
+    w = np.linspace(1.0, 0.05, n)[:, None]
+    X = (1.0 - w) * c + w * rng.standard_normal((n, d))
+    X /= np.linalg.norm(X, axis=1, keepdims=True)
+    Q = c + 0.1 * rng.standard_normal((nq, d))
+    db = store(X)
+    for metric in ("cos", "l2", "dot"):
+        for k in (10, 100):
+            say(f"fp8 without a threshold {d} {metric} k={k}")
+            ids, sc = db.search(Q, k, metric, precision="fp8")
+            rid, rsc = O.topk(X, Q, k, metric)
+            assert_same(ids, sc, rid, rsc, f"fp8 {d} {metric} k={k}")
+    db.close()
