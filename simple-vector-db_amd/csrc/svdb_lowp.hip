@@ -5,6 +5,7 @@
 
 #include <math.h>
 
+#include "svdb_bins.h"
 #include "svdb_prep.h"
 
 namespace svdb {
@@ -477,8 +478,7 @@ __device__ __forceinline__ void shortlist_body(const ShortlistArgs& a, uint32_t 
       // the L-th smallest key is the sm.rank-th of those in [l, h]
       const uint32_t l = sm.lo, h = sm.hi;
       if (l == h) break;
-      const uint32_t w = h - l;
-      const int shift = max(0, 24 - __clz((int)w));
+      const int shift = bin_shift(h - l);
       for (int b = tid; b < 256; b += T) sm.hist[b] = 0;
       __syncthreads();
       each([&](uint32_t k, uint32_t) {
@@ -507,7 +507,7 @@ __device__ __forceinline__ void shortlist_body(const ShortlistArgs& a, uint32_t 
             }
           sm.rank = rank - cum;
           sm.lo = l + (bin << shift);
-          sm.hi = min(h, l + (bin << shift) + ((1u << shift) - 1u));
+          sm.hi = bin_last(l, h, bin, shift);
         }
       }
       __syncthreads();

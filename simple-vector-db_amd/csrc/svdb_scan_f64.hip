@@ -55,6 +55,7 @@
 
 #include <algorithm>
 
+#include "svdb_bins.h"
 #include "svdb_kernels.h"
 #include "svdb_rank.h"
 
@@ -811,7 +812,7 @@ __global__ __launch_bounds__(T) void k_select_f64(MergeArgs a, const uint32_t* _
     for (;;) {
       const uint64_t l = sm.lo, h = sm.hi;
       if (l == h || sm.le <= kCountMax) break;
-      const int shift = max(0, 56 - __clzll((long long)(h - l)));
+      const int shift = bin_shift(h - l);
       for (int b = tid; b < 256; b += T) sm.hist[b] = 0;
       __syncthreads();
       each([&](uint64_t k, uint32_t s) {
@@ -841,11 +842,10 @@ __global__ __launch_bounds__(T) void k_select_f64(MergeArgs a, const uint32_t* _
                 bin++;
               }
             }
-          const uint64_t off = (uint64_t)bin << shift, top = off | ((1ull << shift) - 1ull);
           sm.le = sm.le - total + cum + here;
           sm.rank = r - cum;
-          sm.lo = l + off;
-          sm.hi = top >= h - l ? h : l + top;
+          sm.lo = l + ((uint64_t)bin << shift);
+          sm.hi = bin_last(l, h, bin, shift);
         }
       }
       __syncthreads();

@@ -292,3 +292,25 @@ def test_fp8_lists_without_a_threshold(d):
             rid, rsc = O.topk(X, Q, k, metric)
             assert_same(ids, sc, rid, rsc, f"fp8 {d} {metric} k={k}")
     db.close()
+
+
+def test_fp8_keys_at_the_top_of_the_float_range():
+    """Tiny queries over large rows: the ordering keys, divided by the query's
+    scale, lie between 2^127 and 2^128 but for those of a few rows as small as
+    the queries, which are negative, so the shortlist's range of keys spans
+    both ends."""
+    rng = np.random.default_rng(61)
+    n, d, nq = 1500, 300, 9
+    X = rng.standard_normal((n, d))
+    X *= 2.0 ** 40.25 / np.linalg.norm(X, axis=1, keepdims=True)
+    X *= rng.uniform(0.95, 1.05, (n, 1))
+    Q = 2.0 ** -40 * rng.uniform(-1, 1, (nq, d))
+    Q[:, 0] = 2.0 ** -40
+    X[700:703] = Q[:3]
+    db = store(X)
+    for k in (1, 10, 60):
+        say(f"fp8 largest keys k={k}")
+        ids, sc = db.search(Q, k, "l2", precision="fp8")
+        rid, rsc = O.topk(X, Q, k, "l2")
+        assert_same(ids, sc, rid, rsc, f"fp8 largest keys k={k}")
+    db.close()
