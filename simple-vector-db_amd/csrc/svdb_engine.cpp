@@ -1,6 +1,8 @@
 // svdb_engine.cpp — device store, search pipeline and pair metrics.
 #include "svdb_engine.h"
 
+#include "svdb_f64_lists.h"
+
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -215,15 +217,21 @@ Engine::~Engine() {
   (void)hipStreamDestroy(stream_);
 }
 
-int Engine::dev_alloc(void** p, size_t bytes) {
+// quiet: the caller makes do with less, so a lack of memory is no error yet
+int Engine::dev_alloc(void** p, size_t bytes, bool quiet) {
   if (dev_bytes_ + bytes > budget_) {
-    set_error(SVDB_ENOMEM, "device-memory budget exceeded (" + std::to_string(dev_bytes_ + bytes) +
-                               " > " + std::to_string(budget_) + " bytes)");
+    if (!quiet)
+      set_error(SVDB_ENOMEM, "device-memory budget exceeded (" +
+                                 std::to_string(dev_bytes_ + bytes) + " > " +
+                                 std::to_string(budget_) + " bytes)");
     return SVDB_ENOMEM;
   }
   if (hipMalloc(p, std::max<size_t>(bytes, 256)) != hipSuccess) {
     *p = nullptr;
-    set_error(SVDB_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
+    if (quiet)
+      (void)hipGetLastError();
+    else
+      set_error(SVDB_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
     return SVDB_ENOMEM;
   }
   dev_bytes_ += bytes;
@@ -238,18 +246,44 @@ void Engine::dev_free(void* p, size_t bytes) {
 
 // Grow-only device scratch of the current search context: a buffer being
 // replaced may still be read by that context's queued kernels.
-int Engine::scratch(void** p, size_t* have, size_t need) {
+int Engine::scratch(void** p, size_t* have, size_t need, bool quiet) {
   if (need <= *have && *p) return SVDB_OK;
   HIPCHK(hipStreamSynchronize(c_->stream), "sync");
   scratch_gen_++;  // captured launch sequences that used the old buffer are stale
   dev_free(*p, *have);
   *p = nullptr;
   *have = 0;
-  size_t n = round_up(std::max<size_t>(need, 4096), 4096);
-  int rc = dev_alloc(p, n);
+  size_t n = scratch_size(need);
+  int rc = dev_alloc(p, n, quiet);
   if (rc) return rc;
   *have = n;
   return SVDB_OK;
+}
+
+// The scratch buffers of one plan, all of them or an error.  quiet: a plan past
+// the budget leaves everything as it was (a smaller one may do with the buffers
+// that are there), one past the device's memory gives its buffers back.
+int Engine::scratch_set(std::initializer_list<ScratchNeed> set, bool quiet) {
+  size_t more = 0;  // (what the buffers to be replaced hold is room)
+  for (const ScratchNeed& b : set)
+    if (b.need > *b.have || !*b.p) more += scratch_size(b.need) - *b.have;
+  if (more == 0) return SVDB_OK;
+  if (quiet && dev_bytes_ + more > budget_) return SVDB_ENOMEM;
+  HIPCHK(hipStreamSynchronize(c_->stream), "sync");
+  scratch_gen_++;
+  auto drop = [](Engine* e, const ScratchNeed& b) {
+    e->dev_free(*b.p, *b.have);
+    *b.p = nullptr;
+    *b.have = 0;
+  };
+  for (const ScratchNeed& b : set)
+    if (b.need > *b.have) drop(this, b);
+  int rc = SVDB_OK;
+  for (const ScratchNeed& b : set)
+    if (!rc) rc = scratch(b.p, b.have, b.need, quiet);
+  if (rc && quiet)
+    for (const ScratchNeed& b : set) drop(this, b);
+  return rc;
 }
 
 // Pinned host staging shared by row uploads and searches (both run under
@@ -883,11 +917,12 @@ uint32_t Engine::exact_slices(uint32_t nq, int kmax, size_t max_entries) const {
 }
 
 // The partial lists of an exact scan within max_entries: on the matrix cores
-// from scan_f64_lists, on the VALU nslices · kWavesPerBlock sorted lists of
-// kmax entries.  ok = false when exact_slices refuses the size (in either
-// form, so that what is accepted does not depend on the path).
+// from scan_f64_lists, which takes at most max_lists of them, on the VALU
+// nslices · kWavesPerBlock sorted lists of kmax entries.  ok = false when
+// exact_slices refuses the size (in either form, so that what is accepted does
+// not depend on the path) or the lists do not fit.
 Engine::ExactPlan Engine::exact_plan(int metric, uint32_t nq, uint32_t D, int kmax,
-                                     size_t max_entries) const {
+                                     size_t max_entries, size_t max_lists) const {
   ExactPlan p{};
   p.nslices = exact_slices(nq, kmax, max_entries);
   p.ok = nphys_ == 0 || p.nslices != 0;
@@ -896,9 +931,12 @@ Engine::ExactPlan Engine::exact_plan(int metric, uint32_t nq, uint32_t D, int km
   p.mfma = scan_f64_uses_mfma(metric, D, sv);
   if (p.mfma) {
     // (64 entries are left for the arrays' alignment)
-    const F64Lists l = scan_f64_lists((uint32_t)nphys_, nq, kmax, max_entries - 64);
+    const size_t room = std::min(max_entries, max_lists);
+    const F64Lists l =
+        scan_f64_lists((uint32_t)nphys_, nq, kmax, D, room > 64 ? room - 64 : 0);
     p.P = l.P;
     p.stride = l.cap;
+    p.ok = p.ok && l.entries + 64 <= room;
   } else {
     p.P = p.nslices * kWavesPerBlock;
     p.stride = (uint32_t)kmax;
@@ -912,12 +950,23 @@ int Engine::run_exact(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, con
   int rc;
   if (nq == 0) return SVDB_OK;
   // partial lists stay under 2^25 entries (~400 MB)
-  const ExactPlan p = exact_plan(metric, nq, D, kmax,
-                                 std::max<size_t>((size_t)1 << 25, (size_t)nq * 32 * kmax));
-  const size_t n = std::max<size_t>(p.entries, 1);
-  if ((rc = scratch(&c_->s_pk_, &c_->s_pk_n_, n * sizeof(uint64_t)))) return rc;
-  if ((rc = scratch(&c_->s_ps_, &c_->s_ps_n_, n * sizeof(uint32_t)))) return rc;
-  if ((rc = scratch(&c_->s_qn_, &c_->s_qn_n_, exact_aux_bytes(nq, p)))) return rc;
+  const size_t most = std::max<size_t>((size_t)1 << 25, (size_t)nq * 32 * kmax);
+  ExactPlan p = exact_plan(metric, nq, D, kmax, most, most);
+  // on the matrix cores fewer and shorter lists where there is no room for
+  // these, down to the fewest
+  for (size_t room = most;;) {
+    room = std::min(room, p.entries) / 2;
+    ExactPlan less = p;
+    if (p.mfma) less = exact_plan(metric, nq, D, kmax, most, room);
+    const bool last = less.entries >= p.entries;
+    const size_t n = std::max<size_t>(p.entries, 1);
+    rc = scratch_set({{&c_->s_pk_, &c_->s_pk_n_, n * sizeof(uint64_t)},
+                      {&c_->s_ps_, &c_->s_ps_n_, n * sizeof(uint32_t)},
+                      {&c_->s_qn_, &c_->s_qn_n_, exact_aux_bytes(nq, p)}}, !last);
+    if (!rc) break;
+    if (rc != SVDB_ENOMEM || last) return rc;
+    p = less;
+  }
   return run_exact_with(dQ, ldq, nq, D, dk, metric, kmax, dids, dscores, ostride, p,
                         (uint64_t*)c_->s_pk_, (uint32_t*)c_->s_ps_, (double*)c_->s_qn_);
 }
@@ -1667,7 +1716,7 @@ int Engine::search_device_noalloc(const double* dQ, size_t nq, size_t ldq, size_
     return SVDB_EINVAL;
   }
   const size_t entries = (bytes - kb - qb - 256) / (sizeof(uint64_t) + sizeof(uint32_t));
-  const ExactPlan p = exact_plan(metric, (uint32_t)nq, (uint32_t)d_, (int)k, entries);
+  const ExactPlan p = exact_plan(metric, (uint32_t)nq, (uint32_t)d_, (int)k, entries, entries);
   if (!p.ok) {
     set_error_static(SVDB_EINVAL, "queries x k too large for the allocation-free scratch");
     return SVDB_EINVAL;

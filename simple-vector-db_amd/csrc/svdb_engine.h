@@ -21,7 +21,9 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <functional>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -141,9 +143,18 @@ class Engine {
   int refresh_degen();
   int compact();
   static constexpr size_t kCompactMin = 256;  // fewest tombstones worth a compaction
-  int dev_alloc(void** p, size_t bytes);
+  int dev_alloc(void** p, size_t bytes, bool quiet = false);
   void dev_free(void* p, size_t bytes);
-  int scratch(void** p, size_t* have, size_t need);
+  static size_t scratch_size(size_t need) {
+    return (std::max<size_t>(need, 4096) + 4095) / 4096 * 4096;
+  }
+  int scratch(void** p, size_t* have, size_t need, bool quiet = false);
+  struct ScratchNeed {
+    void** p;
+    size_t* have;
+    size_t need;
+  };
+  int scratch_set(std::initializer_list<ScratchNeed> set, bool quiet);
   // pinned staging, grow-only; nullptr past its cap
   void* host_stage(void** buf, size_t* have, size_t bytes);
   int run_exact(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, const int* dk, int metric,
@@ -154,7 +165,8 @@ class Engine {
     uint32_t P, stride;  // partial lists per query, entries per list
     size_t entries;      // nq * P * stride
   };
-  ExactPlan exact_plan(int metric, uint32_t nq, uint32_t D, int kmax, size_t max_entries) const;
+  ExactPlan exact_plan(int metric, uint32_t nq, uint32_t D, int kmax, size_t max_entries,
+                       size_t max_lists) const;
   static size_t exact_aux_bytes(uint32_t nq, const ExactPlan& p);
   int run_exact_with(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, const int* dk,
                      int metric, int kmax, uint64_t* dids, double* dscores, uint32_t ostride,

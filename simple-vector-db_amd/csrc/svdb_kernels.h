@@ -83,13 +83,7 @@ hipError_t launch_merge(const MergeArgs& a, int kmax, hipStream_t s);
 // ---- the FP64 scan on the matrix cores (svdb_scan_f64.hip) ----
 // Whether it serves this metric, width and row layout: every column compared.
 bool scan_f64_uses_mfma(int metric, uint32_t D, const StoreView& st);
-// Its partial lists per query and entries per list (P · cap · nq entries, at
-// most max_entries; P = 0 for an empty store).
-struct F64Lists {
-  uint32_t P, cap;
-};
-F64Lists scan_f64_lists(uint32_t nrows, uint32_t nq, int kmax, size_t max_entries);
-// a.P and a.kstride from scan_f64_lists; a.gtk, a.part_cnt set (gtk written).
+// a.P and a.kstride from scan_f64_lists (svdb_f64_lists.h); a.gtk, a.part_cnt set (gtk written).
 hipError_t launch_scan_f64_mfma(const ScanF64Args& a, int metric, int kmax, hipStream_t s);
 // The k best of a query's unsorted lists (m.kstride entries apart,
 // cnt[q][list] of them) with keys at most gtk[q].

@@ -11,7 +11,7 @@
 // matrix form: the dot product gives a = (xx + qq) − 2·dot (xx, qq the
 // canonical squared norms), within E = c·(‖x‖ + ‖q‖)² + e of the canonical key
 // (l2_bound), and only a pair whose lower bound a − E could still be among its
-// query's nearest computes the canonical key (exact_l2); every other pair is
+// query's nearest computes the canonical key (exact_chain); every other pair is
 // provably out.
 //
 // Block: 4 wavefronts, 16 queries each (64 per block), sharing the rows of
@@ -43,8 +43,8 @@
 // Results: each (query, slice) has an unsorted list in global memory.  A row
 // enters when its key is at most the query's global bound gtk — the smallest
 // k-th key any of its lists has reached, atomic min — and ranks before the
-// list's own k-th.  A list that could not take another row step is cut to its
-// k best (compact), which gives it that k-th and lowers gtk.  A test per
+// list's own k-th.  A list that cannot take a row is cut to its k best
+// (compact), which gives it that k-th and lowers gtk, and the row is tried again.  A test per
 // (query, row) is one comparison of doubles; all else happens in branches that
 // a row step seldom takes.  (Sorted lists spread over a wavefront's registers
 // had taken 48 of them at k <= 64 and 96 above, and every insertion a chain of
@@ -56,6 +56,7 @@
 #include <algorithm>
 
 #include "svdb_bins.h"
+#include "svdb_f64_lists.h"
 #include "svdb_kernels.h"
 #include "svdb_rank.h"
 
@@ -63,14 +64,19 @@ namespace svdb {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
-constexpr int kF64StageRows = 64;
-constexpr int kF64MaxCap = 320;  // entries of a list
 
 __device__ __forceinline__ uint64_t uni64(uint64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
   return ((uint64_t)hi << 32) | lo;
 }
+
+// Hides a lane's value at the end of a loop over whole wavefronts: where the
+// compiler sees what a lane that has nothing left does in the next turn, it may
+// send it there by a way of its own, and the cross-lane steps on the way are
+// then taken without it (such lanes had held the counts by which full lists are
+// found: they were not cut).
+__device__ __forceinline__ void whole_wave(uint32_t& v) { asm volatile("" : "+v"(v)); }
 
 // Byte offset in a stage of SC columns of 16-byte unit u (columns 2u, 2u+1)
 // of row r.
@@ -99,10 +105,11 @@ __device__ __forceinline__ void f64_issue_stage(const StoreView& st, unsigned ch
   }
 }
 
-// The canonical Euclidean key of row x and query q over D columns
-// (x 16-byte aligned, zero past D): Σ_i fma(t, t, s), t = x_i − q_i.
-__device__ __forceinline__ double exact_l2(const double* __restrict__ x,
-                                          const double* __restrict__ q, uint32_t D) {
+// The canonical chain of row x and query q over D columns (x 16-byte aligned,
+// zero past D): Euclidean Σ_i fma(t, t, s), t = x_i − q_i, else Σ_i fma(q_i, x_i, s).
+template <bool L2>
+__device__ __forceinline__ double exact_chain(const double* __restrict__ x,
+                                              const double* __restrict__ q, uint32_t D) {
   double s = 0.0;
   for (uint32_t c = 0; c < D; c += 8) {
     double xv[8], qv[8];
@@ -117,7 +124,7 @@ __device__ __forceinline__ double exact_l2(const double* __restrict__ x,
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       const double t = xv[i] - qv[i];
-      s = fma(t, t, s);
+      s = L2 ? fma(t, t, s) : fma(qv[i], xv[i], s);
     }
   }
   return s;
@@ -152,18 +159,40 @@ struct F64Wave {
   uint32_t own_slot[kScanTQ];
   uint64_t own_key[kScanTQ];
   uint64_t gk[kScanTQ];
-  uint32_t queue[128];  // Euclidean: pairs awaiting their key
+  uint32_t queue[128];  // pairs awaiting their key
 };
 
-// Cuts a list of n entries to its k best by (key, slot), one wavefront.  The
-// k-th key is found by bisecting the key's bits with counts over the
-// wavefront, the slot among equal keys likewise; what remains is packed.
+// Cuts a list of n entries to its k best by (key, slot), one wavefront.  Up to 64
+// entries find their places by comparing with each other (28 entries: 0.5 µs);
+// of more, the k-th key is found by bisecting the key's bits with counts over the
+// wavefront, the slot among equal keys likewise, and what remains is packed (3 µs).
 __device__ __attribute__((noinline)) void f64_compact(uint64_t* key, uint32_t* slot, uint32_t n,
                                                       uint32_t k, uint64_t* own_key,
                                                       uint32_t* own_slot, uint64_t* gtk) {
   constexpr int R = kF64MaxCap / 64;
   const int lane = threadIdx.x & 63;
   __threadfence_block();  // entries other lanes have stored
+  if (n <= 64) {
+    const bool in = (uint32_t)lane < n;
+    const uint64_t kl = in ? key[lane] : ~0ull;
+    const uint32_t sl = in ? slot[lane] : ~0u;
+    uint32_t place = 0;
+    for (uint32_t t = 0; t < n; t++) {
+      const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)kl, t);
+      const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(kl >> 32), t);
+      place += lex_lt(((uint64_t)hi << 32) | lo, __builtin_amdgcn_readlane(sl, t), kl, sl);
+    }
+    if (in && place < k) {
+      key[place] = kl;
+      slot[place] = sl;
+    }
+    if (in && place == k - 1) {
+      *own_key = kl;
+      *own_slot = sl;
+      __hip_atomic_fetch_min(gtk, kl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return;
+  }
   uint64_t kv[R];
   uint32_t sv[R];
   uint64_t kmin = ~0ull, kmax = 0;
@@ -218,6 +247,111 @@ __device__ __attribute__((noinline)) void f64_compact(uint64_t* key, uint32_t* s
     *own_slot = slo;
     __hip_atomic_fetch_min(gtk, K, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+// A wavefront's way into its lists.
+template <int METRIC>
+struct F64Lane {
+  const ScanF64Args& a;
+  F64Wave& ws;
+  size_t list0, list_q;  // query qw's list; from one query's to the next's
+  uint32_t qw, r_begin;
+  int lane;
+
+  // Row `row` with rank key `kk` enters query j's list if it is to (lanes with
+  // c set); true where the list is full, to be tried again once it is cut.
+  __device__ __forceinline__ bool append(bool c, uint64_t kk, uint32_t row, int j) {
+    if (!(c && kk <= ws.gk[j] && lex_lt(kk, row, ws.own_key[j], ws.own_slot[j]))) return false;
+    const uint32_t pos = atomicAdd(&ws.cnt[j], 1u);
+    if (pos >= a.kstride) return true;
+    const size_t o = list0 + (size_t)j * list_q + pos;
+    a.part_key[o] = kk;
+    a.part_slot[o] = row;
+    return false;
+  }
+
+  // Lists that could not take a row are cut.
+  __device__ __forceinline__ void cut_lists() {
+    const uint32_t n = lane < kScanTQ ? __hip_atomic_load(&ws.cnt[lane], __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_WORKGROUP)
+                                      : 0u;
+    uint64_t m = __ballot(n > a.kstride);
+    while (m) {
+      const int j = __ffsll((long long)m) - 1;
+      m &= m - 1;
+      const uint32_t kj = (uint32_t)a.k[qw + j];
+      const size_t o = list0 + (size_t)j * list_q;
+      f64_compact(a.part_key + o, a.part_slot + o, a.kstride, kj, &ws.own_key[j],
+                  &ws.own_slot[j], a.gtk + qw + j);
+      if (lane == 0) ws.cnt[j] = kj;
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+
+  // n queued pairs, one per lane, get their canonical keys and enter their lists.
+  __device__ __forceinline__ void run_batch(uint32_t n) {
+    uint32_t v = (uint32_t)lane < n;
+    const uint32_t e = v ? ws.queue[lane] : 0u;
+    const uint32_t row = r_begin + (e >> 4);
+    const int j = (int)(e & 15u);
+    uint64_t kk = ~0ull;
+    if (v) {
+      const uint32_t q = qw + (uint32_t)j;
+      double s = exact_chain<METRIC == kL2>(a.st.X + (size_t)row * a.st.ldx,
+                                            a.Q + (size_t)q * a.ldq, a.D);
+      if (METRIC == kDot) s = -s;
+      if (METRIC == kCos) s = -(s / (a.qn[q] * a.st.xn[row]));
+      kk = rank_bits(s);
+    }
+    for (;;) {
+      v = append(v != 0, kk, row, j);
+      if (__builtin_expect(__ballot(v) == 0, 1)) break;
+      cut_lists();
+      whole_wave(v);
+    }
+  }
+
+  // The pairs of the row step at base in `hits` (bit 4t + r) join the queue, qcount
+  // long; full batches of 64 are run.
+  __device__ __forceinline__ void queue_pairs(uint32_t hits, uint32_t base, uint32_t& qcount) {
+    const int g = lane >> 4, jr = lane & 15;
+    uint64_t any;
+    while ((any = __ballot(hits != 0)) != 0) {
+      if (hits) {
+        const int b = __ffs((int)hits) - 1;
+        hits &= hits - 1;
+        const uint32_t row = base + 16 * (b >> 2) + jr;
+        ws.queue[qcount + __popcll(any & ((1ull << lane) - 1ull))] =
+            ((row - r_begin) << 4) | (uint32_t)(g + 4 * (b & 3));
+      }
+      qcount += __popcll(any);
+      __builtin_amdgcn_wave_barrier();
+      if (qcount >= 64) {
+        run_batch(64);
+        qcount -= 64;
+        const uint32_t rest = (uint32_t)lane < qcount ? ws.queue[64 + lane] : 0u;
+        __builtin_amdgcn_wave_barrier();
+        if ((uint32_t)lane < qcount) ws.queue[lane] = rest;
+        __builtin_amdgcn_wave_barrier();
+      }
+      whole_wave(hits);
+    }
+  }
+};
+
+// The pairs of a row step whose lists were full: their keys are computed again
+// (in line, with the keys kept, the accumulators would be live across the cuts
+// and the loop over the rows would spill).
+template <int METRIC>
+__device__ __attribute__((noinline)) void f64_again(const ScanF64Args* a, F64Wave* ws,
+                                                    size_t list0, uint32_t qw, uint32_t r_begin,
+                                                    uint32_t again, uint32_t base) {
+  F64Lane<METRIC> in{*a, *ws, list0, (size_t)a->P * a->kstride, qw, r_begin,
+                     (int)(threadIdx.x & 63)};
+  uint32_t n = 0;
+  in.cut_lists();
+  in.queue_pairs(again, base, n);
+  if (n) in.run_batch(n);
 }
 
 // MINS: the sample; mins[(query · slices + slice) · 16 + lane % 16] gets the
@@ -309,50 +443,8 @@ k_scan_f64_mfma(ScanF64Args a) {
     }
   };
 
-  // Row `row` with rank key `kk` enters query j's list if it is to (lanes with
-  // c set; at most 64 rows a query before the next cut_lists).
-  auto append = [&](bool c, uint64_t kk, uint32_t row, int j) __attribute__((always_inline)) {
-    if (c && kk <= ws.gk[j] && lex_lt(kk, row, ws.own_key[j], ws.own_slot[j])) {
-      const uint32_t pos = atomicAdd(&ws.cnt[j], 1u);
-      const size_t o = list0 + (size_t)j * list_q + pos;
-      a.part_key[o] = kk;
-      a.part_slot[o] = row;
-    }
-  };
-  // Lists without room for another 64 rows are cut.
-  auto cut_lists = [&]() __attribute__((always_inline)) {
-    const uint32_t n = lane < kScanTQ ? __hip_atomic_load(&ws.cnt[lane], __ATOMIC_RELAXED,
-                                                          __HIP_MEMORY_SCOPE_WORKGROUP)
-                                      : 0u;
-    uint64_t m = __ballot(n + 64 > a.kstride);
-    while (m) {
-      const int j = __ffsll((long long)m) - 1;
-      m &= m - 1;
-      const uint32_t nj = __builtin_amdgcn_readlane(n, j);
-      const uint32_t kj = (uint32_t)a.k[qw + j];
-      if (nj <= kj) continue;  // (a slice shorter than its lists)
-      const size_t o = list0 + (size_t)j * list_q;
-      f64_compact(a.part_key + o, a.part_slot + o, nj, kj, &ws.own_key[j], &ws.own_slot[j],
-                  a.gtk + qw + j);
-      if (lane == 0) ws.cnt[j] = kj;
-    }
-    __builtin_amdgcn_wave_barrier();
-  };
-
-  // Euclidean: n queued pairs, one per lane, get their canonical keys.
-  uint32_t qcount = 0;
-  auto run_batch = [&](uint32_t n) __attribute__((always_inline)) {
-    const bool v = (uint32_t)lane < n;
-    const uint32_t e = v ? ws.queue[lane] : 0u;
-    const uint32_t row = r_begin + (e >> 4);
-    const int j = (int)(e & 15u);
-    uint64_t kk = ~0ull;
-    if (v)
-      kk = rank_bits(exact_l2(a.st.X + (size_t)row * a.st.ldx,
-                              a.Q + (size_t)(qw + (uint32_t)j) * a.ldq, a.D));
-    append(v, kk, row, j);
-    cut_lists();
-  };
+  F64Lane<METRIC> in{a, ws, list0, list_q, qw, r_begin, lane};
+  uint32_t qcount = 0;  // Euclidean: queued pairs
 
   // The per-row values of the row step at base into rowv / alivew[par]:
   // wave 0 the norms, wave 1 the squared norms (4-byte direct-to-LDS loads,
@@ -434,28 +526,9 @@ k_scan_f64_mfma(ScanF64Args a) {
     }
     if (__builtin_expect(__ballot(hits != 0) == 0, 1)) return;
     if constexpr (METRIC == kL2) {
-      // pairs join the wavefront's queue, full batches of 64 get their keys
-      uint64_t any;
-      while ((any = __ballot(hits != 0)) != 0) {
-        if (hits) {
-          const int b = __ffs((int)hits) - 1;
-          hits &= hits - 1;
-          const uint32_t row = base + 16 * (b >> 2) + jr;
-          ws.queue[qcount + __popcll(any & ((1ull << lane) - 1ull))] =
-              ((row - r_begin) << 4) | (uint32_t)(g + 4 * (b & 3));
-        }
-        qcount += __popcll(any);
-        __builtin_amdgcn_wave_barrier();
-        if (qcount >= 64) {
-          run_batch(64);
-          qcount -= 64;
-          const uint32_t rest = (uint32_t)lane < qcount ? ws.queue[64 + lane] : 0u;
-          __builtin_amdgcn_wave_barrier();
-          if ((uint32_t)lane < qcount) ws.queue[lane] = rest;
-          __builtin_amdgcn_wave_barrier();
-        }
-      }
+      in.queue_pairs(hits, base, qcount);
     } else {
+      uint32_t again = 0;
 #pragma unroll
       for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -464,9 +537,14 @@ k_scan_f64_mfma(ScanF64Args a) {
           if (__ballot(c) == 0) continue;
           const double xn = METRIC == kCos ? rowv[par][0][16 * t + jr] : 0.0;
           const double sc = METRIC == kCos ? -(acc[t][r] / (qn4[r] * xn)) : -acc[t][r];
-          append(c, rank_bits(sc), base + 16 * t + jr, g + 4 * r);
+          if (in.append(c, rank_bits(sc), base + 16 * t + jr, g + 4 * r))
+            again |= 1u << (4 * t + r);
         }
-      cut_lists();
+      if (__builtin_expect(__ballot(again != 0) != 0, 0))
+        // (the arguments where the kernel got them: a pointer to `a` would have
+        // every wavefront copy it to its stack)
+        f64_again<METRIC>((const ScanF64Args*)__builtin_amdgcn_kernarg_segment_ptr(), &ws, list0,
+                          qw, r_begin, again, base);
     }
   };
 
@@ -553,7 +631,7 @@ k_scan_f64_mfma(ScanF64Args a) {
             mins[r] < INFINITY ? (uint32_t)(rank_bits(mins[r]) >> 32) : ~0u;
     return;
   }
-  if (METRIC == kL2 && qcount) run_batch(qcount);
+  if (METRIC == kL2 && qcount) in.run_batch(qcount);
   __builtin_amdgcn_wave_barrier();
   if (lane < kScanTQ && qw + lane < a.nq)
     a.part_cnt[(size_t)(qw + lane) * a.P + slice] = ws.cnt[lane];
@@ -565,30 +643,6 @@ k_scan_f64_mfma(ScanF64Args a) {
 bool scan_f64_uses_mfma(int metric, uint32_t D, const StoreView& st) {
   return D > 0 && st.ldx % 8 == 0 && D <= st.ldx && D + 8 > st.ldx &&
          ((uintptr_t)st.X & 15) == 0 && st.nx2 != nullptr && metric >= 0;
-}
-
-// Slices for about 512 blocks (two per CU, one round: the fewer and longer a
-// query's lists, the sooner their bounds are tight), at least 64 rows each (a
-// one-query call over 10,000 rows: 8 slices of 1,250 rows took 193 µs per
-// call, 64 slices 88 µs).  A list takes k and up to three row steps on top
-// (two cuts of a list then lie at least 128 rows that entered apart), or its
-// whole slice if that is less.
-F64Lists scan_f64_lists(uint32_t nrows, uint32_t nq, int kmax, size_t max_entries) {
-  if (nrows == 0 || nq == 0) return F64Lists{0, 0};
-  const uint32_t QB = kScanTQ * kWavesPerBlock;
-  const uint32_t groups = (nq + QB - 1) / QB;
-  uint32_t P = (512 + groups - 1) / groups;
-  P = std::min<uint32_t>(P, (nrows + 63) / 64);
-  if (P >= 8) P = P / 8 * 8;
-  // (a queued pair holds the row's place in its slice in 28 bits)
-  const uint32_t minP = (nrows >> 27) + 1;
-  P = std::max(P, minP);
-  uint32_t cap = std::min<uint32_t>(kF64MaxCap, ((uint32_t)kmax + 192 + 63) / 64 * 64);
-  auto entries = [&](uint32_t p, uint32_t c) { return (size_t)nq * p * (c + 1); };
-  while (entries(P, cap) > max_entries && P > minP) P = std::max(minP, P > 8 ? P / 16 * 8 : P / 2);
-  while (entries(P, cap) > max_entries && cap > (uint32_t)kmax + 64) cap--;
-  const uint32_t rows = ((nrows + P - 1) / P + 63) / 64 * 64;
-  return F64Lists{P, std::max<uint32_t>(std::min(cap, rows + 64), (uint32_t)kmax + 64)};
 }
 
 // gtk[q] = a rank key at or above the k-th of the n sample minima of query q
@@ -650,28 +704,19 @@ static hipError_t scan_f64_mfma_m(const ScanF64Args& a, int metric, hipStream_t 
 hipError_t launch_scan_f64_mfma(const ScanF64Args& a, int metric, int kmax, hipStream_t s) {
   if (a.nq == 0 || a.P == 0) return hipSuccess;
   if (!scan_f64_uses_mfma(metric, a.D, a.st) || !a.gtk || !a.part_cnt ||
-      a.kstride > (uint32_t)kF64MaxCap || a.kstride < (uint32_t)kmax + 64 ||
-      (metric == kL2 && !a.qq))
+      a.kstride > kF64MaxCap || (metric == kL2 && !a.qq))
     return hipErrorInvalidValue;
+  const uint32_t rows = f64_slice_rows(a.st.nrows, a.P);
+  if (a.kstride <= (uint32_t)kmax && a.kstride < rows) return hipErrorInvalidValue;
   ScanF64Args m = a;
   hipError_t e;
-  // The sample: up to 64 runs of row steps, 16 minima each, at least twice k
-  // of them (on small stores up to a quarter of the rows for that); the minima
-  // lie where the lists will.
-  const uint32_t want = ((uint32_t)kmax + 7) / 8;
-  uint32_t S = std::max<uint32_t>(a.st.nrows / 1024,
-                                  std::min<uint32_t>((want + 7) / 8 * 8, a.st.nrows / 256));
-  // 1/16 of the rows up to 128 columns; wider, where an insertion costs less
-  // beside the products, as much less (300k × 768, 1,024 queries: dot 11.5 ms
-  // with 1/16 and a test per query value, 9.95 so; a share falling with the
-  // square of the width: Euclidean 12.5 → 18.7).
-  const uint32_t c = (a.D + 127) / 128, share = a.st.nrows / (16 * c);
-  if (c > 1) S = std::min(S, std::max((want + 7) / 8 * 8, share / 64));
-  S = std::min<uint32_t>({S, kMinsPerLane * 4, a.P * a.kstride / 8}) / 8 * 8;
-  if (S && 16 * S >= 2 * (uint32_t)kmax) {
+  // The sample; the minima lie where the lists will.
+  const uint32_t S =
+      f64_sample_runs(a.st.nrows, kmax, a.D, (size_t)a.P * a.kstride / 8);
+  if (S) {
     m.P = S;
     m.slice_stride = a.st.nrows / S / 64 * 64;
-    m.rows_per_slice = std::max<uint32_t>(64, share / S / 64 * 64);
+    m.rows_per_slice = std::max<uint32_t>(64, a.st.nrows / f64_share(a.D) / S / 64 * 64);
     if ((e = scan_f64_mfma_m<true>(m, metric, s)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_bound_f64, dim3((a.nq + 3) / 4), dim3(256), 0, s,
                        reinterpret_cast<const uint32_t*>(a.part_key), 16 * S, a.nq, a.k, a.gtk);
@@ -681,7 +726,7 @@ hipError_t launch_scan_f64_mfma(const ScanF64Args& a, int metric, int kmax, hipS
     if (e != hipSuccess) return e;
   }
   m.P = a.P;
-  m.rows_per_slice = m.slice_stride = ((a.st.nrows + a.P - 1) / a.P + 63) / 64 * 64;
+  m.rows_per_slice = m.slice_stride = rows;
   return scan_f64_mfma_m<false>(m, metric, s);
 }
 

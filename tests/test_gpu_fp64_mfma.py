@@ -200,3 +200,23 @@ def test_sampled_bounds_and_ties(n, nq, k):
         say(f"ties {n} rows {nq} queries k={k} {metric}")
         check(db, X, Q, k, metric, what="ties")
     db.close()
+
+
+@pytest.mark.parametrize("nq,k", [(64, 1), (3, 128), (1000, 10), (500, 2)])
+def test_lists_within_a_budget(nq, k):
+    """A device-memory budget that holds a slice's k best per wavefront and query,
+    one slice per 1,024 rows: the scan makes do with it."""
+    rng = np.random.default_rng(nq)
+    n, d = 50_000, 32
+    X = rng.standard_normal((n, d))
+    Q = rng.standard_normal((nq, d))
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    lists = nq * 4 * min(n // 1024, max(8, 8192 * 16 // nq)) * k
+    need = [lists * 8, lists * 4, nq * 24, nq * d * 8, nq * 4, nq * k * 8, nq * k * 8]
+    db.set_budget(db.stats()["device_bytes"] + sum((b + 4095) // 4096 * 4096 for b in need))
+    say(f"budget {nq} queries k={k}")
+    for metric in ("l2", "cos", "dot"):
+        check(db, X, Q, k, metric, what="budget")
+    assert svdb.lib().svdb_last_error() == b"" or b"budget" not in svdb.lib().svdb_last_error()
+    db.close()
