@@ -3,7 +3,8 @@
 // A list belongs to one lane of a scan and one of its queries: up to
 // kLowpLC (ordering key, slot) entries in global memory, in no order, and a
 // header {entries, bound}: every row the list covers and does not hold is
-// keyed at or above the bound.  With a starting threshold most subtiles bring
+// keyed at or above the bound.  (Lists from nothing, in registers: see
+// cand_store_sorted.)  With a starting threshold most subtiles bring
 // a lane nothing and a query's lists together take a few hundred rows of a
 // million, so an entry is one 8-byte store at the lane's own count — no list
 // in registers (eight sorted entries per fragment had taken 64 of a wavefront's
@@ -127,19 +128,15 @@ __device__ __forceinline__ void cand_append4(uint2* ent, CandPending& p, uint32_
   } while (__ballot(fminf(fminf(k4[0], k4[1]), fminf(k4[2], k4[3])) < tau));
 }
 
-// A sorted register list (unused entries: slot ~0) to its place.
+// A sorted register list to its place: kLowpLP entries, unused ones with slot ~0
+// behind the others and keyed with the bound, which is the last entry's key.
 __device__ __forceinline__ void cand_store_sorted(const LowpScanArgs& a, size_t list,
                                                   const float (&lk)[kLowpLP],
                                                   const uint32_t (&ls)[kLowpLP]) {
-  uint2* e = a.ent + list * kLowpLC;
-  uint32_t n = 0;
+  uint4* e = reinterpret_cast<uint4*>(a.ent + list * kLowpLP);
 #pragma unroll
-  for (int j = 0; j < kLowpLP; j++)
-    if (ls[j] != ~0u) {
-      e[j] = make_uint2(__float_as_uint(lk[j]), ls[j]);
-      n++;
-    }
-  a.hdr[list] = make_uint2(n, __float_as_uint(lk[kLowpLP - 1]));
+  for (int j = 0; j < kLowpLP; j += 2)
+    e[j / 2] = make_uint4(__float_as_uint(lk[j]), ls[j], __float_as_uint(lk[j + 1]), ls[j + 1]);
 }
 
 }  // namespace svdb

@@ -219,23 +219,51 @@ Engine::~Engine() {
 
 // quiet: the caller makes do with less, so a lack of memory is no error yet
 int Engine::dev_alloc(void** p, size_t bytes, bool quiet) {
-  if (dev_bytes_ + bytes > budget_) {
-    if (!quiet)
-      set_error(SVDB_ENOMEM, "device-memory budget exceeded (" +
-                                 std::to_string(dev_bytes_ + bytes) + " > " +
-                                 std::to_string(budget_) + " bytes)");
-    return SVDB_ENOMEM;
+  quiet |= quiet_;
+  do {
+    if (dev_bytes_ + bytes <= budget_) {
+      if (hipMalloc(p, std::max<size_t>(bytes, 256)) == hipSuccess) {
+        dev_bytes_ += bytes;
+        return SVDB_OK;
+      }
+      *p = nullptr;
+      if (quiet) (void)hipGetLastError();
+    }
+  } while (release_lists());
+  if (quiet) return SVDB_ENOMEM;
+  if (dev_bytes_ + bytes > budget_)
+    set_error(SVDB_ENOMEM, "device-memory budget exceeded (" + std::to_string(dev_bytes_ + bytes) +
+                               " > " + std::to_string(budget_) + " bytes)");
+  else
+    set_error(SVDB_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
+  return SVDB_ENOMEM;
+}
+
+// Gives back the lists that earlier searches left behind, the part of a
+// context's scratch that goes with the store rather than with the call; false if
+// there were none.
+bool Engine::release_lists() {
+  bool any = false;
+  for (auto& c : ctx_) {
+    auto drop = [&](void*& p, size_t& n) {
+      if (!p) return;
+      (void)hipStreamSynchronize(c.stream);
+      scratch_gen_++;
+      dev_free(p, n);
+      p = nullptr;
+      n = 0;
+      any = true;
+    };
+    if (!c.cand_live) {
+      drop(c.s_ck_, c.s_ck_n_);
+      drop(c.s_cs_, c.s_cs_n_);
+    }
+    if (!c.part_live) {
+      drop(c.s_pk_, c.s_pk_n_);
+      drop(c.s_ps_, c.s_ps_n_);
+    }
   }
-  if (hipMalloc(p, std::max<size_t>(bytes, 256)) != hipSuccess) {
-    *p = nullptr;
-    if (quiet)
-      (void)hipGetLastError();
-    else
-      set_error(SVDB_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
-    return SVDB_ENOMEM;
-  }
-  dev_bytes_ += bytes;
-  return SVDB_OK;
+  return any;
 }
 
 void Engine::dev_free(void* p, size_t bytes) {
@@ -285,6 +313,13 @@ int Engine::scratch_set(std::initializer_list<ScratchNeed> set, bool quiet) {
     for (const ScratchNeed& b : set) drop(this, b);
   return rc;
 }
+
+// Holds a context's flag while its lists are in use.
+struct Live {
+  bool& on;
+  explicit Live(bool& b) : on(b) { on = true; }
+  ~Live() { on = false; }
+};
 
 // Pinned host staging shared by row uploads and searches (both run under
 // mu_ and synchronise the stream before returning, so the buffer is free on
@@ -952,6 +987,7 @@ int Engine::run_exact(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, con
   // partial lists stay under 2^25 entries (~400 MB)
   const size_t most = std::max<size_t>((size_t)1 << 25, (size_t)nq * 32 * kmax);
   ExactPlan p = exact_plan(metric, nq, D, kmax, most, most);
+  Live live(c_->part_live);
   // on the matrix cores fewer and shorter lists where there is no room for
   // these, down to the fewest
   for (size_t room = most;;) {
@@ -1031,10 +1067,7 @@ int Engine::run_lowp(const double* dQ, size_t ldq, uint32_t nq, int metric, int 
                      uint64_t* dids, double* dscores, uint32_t ostride, bool fp8,
                      const double* hQ) {
   LowpRange r{metric, 0, nq, k, 0, 0, 0, 0, 0, 0};
-  if (const int rc = lowp_enqueue(dQ, ldq, &r, 1, k, dids, dscores, ostride, fp8, hQ)) {
-    c_->lp.on = false;
-    return rc;
-  }
+  if (const int rc = lowp_enqueue(dQ, ldq, &r, 1, k, dids, dscores, ostride, fp8, hQ)) return rc;
   return lowp_complete();
 }
 
@@ -1049,8 +1082,10 @@ int Engine::run_lowp(const double* dQ, size_t ldq, uint32_t nq, int metric, int 
 // shortlist width (k is the largest over ranges).
 int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int k,
                          uint64_t* dids, double* dscores, uint32_t ostride, bool fp8,
-                         const double* hQ) {
+                         const double* hQ, bool frugal) {
   int rc;
+  c_->lp.on = false;
+  c_->cand_live = false;
   if (nr < 1 || nr > 3) {
     set_error(SVDB_EINVAL, "one to three query ranges");
     return SVDB_EINVAL;
@@ -1132,7 +1167,7 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     frac = (double)ns_pre * tp / std::max<uint32_t>(1, tiles);
     if (enough() || ns_pre >= kPrepassSlices || tiles < 8 * ns_pre) break;
   }
-  bool pre = prepass_ && tiles >= 4 * ns_pre && enough();
+  bool pre = prepass_ && !frugal && tiles >= 4 * ns_pre && enough();
   const uint32_t NL_pre = ns_pre * kLowpLanesPerQuery;
   // Row slices for a scan of n queries wanting kk neighbours: at
   // least 8, more when there are few query blocks, without a threshold each at
@@ -1241,25 +1276,33 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   if ((rc = scratch(&c_->s_ls_, &c_->s_ls_n_, (size_t)nq * k * sizeof(uint32_t)))) return rc;
   if ((rc = scratch(&c_->s_km_, &c_->s_km_n_, (size_t)nq * sizeof(float)))) return rc;
   // list headers (before them, in the same place, the pre-pass's keys) and
-  // entries, in what the device-memory budget leaves: half the slices, down to
-  // 8, while it is too little, then no threshold (both only cost certificates)
+  // entries, in what the device memory leaves: half the slices, down to 8,
+  // while it is too little, then no threshold (both only cost certificates).
+  // Without one a list is its kLowpLP sorted entries and nothing else.
+  c_->cand_live = true;
   for (uint32_t cap = 512;; cap = cap > 8 ? cap / 2 : 512) {
     plan(cap);
-    rc = scratch(&c_->s_ck_, &c_->s_ck_n_,
-                 std::max(nlists * sizeof(uint2),
-                          pre ? (size_t)nq * NL_pre * sizeof(float) : (size_t)0));
-    if (!rc) rc = scratch(&c_->s_cs_, &c_->s_cs_n_, nlists * kLowpLC * sizeof(uint2));
+    const bool last = cap <= 8 && !pre;
+    rc = pre ? scratch_set({{&c_->s_ck_, &c_->s_ck_n_,
+                             std::max(nlists * sizeof(uint2), (size_t)nq * NL_pre * sizeof(float))},
+                            {&c_->s_cs_, &c_->s_cs_n_, nlists * kLowpLC * sizeof(uint2)}}, true)
+             : scratch_set({{&c_->s_cs_, &c_->s_cs_n_, nlists * kLowpLP * sizeof(uint2)}}, !last);
     if (!rc) break;
-    if (rc != SVDB_ENOMEM || (cap <= 8 && !pre)) return rc;
-    (void)hipGetLastError();
-    if (cap <= 8) pre = false;
-    // (the headers' buffer grew first; its room may be what is missing)
-    HIPCHK(hipStreamSynchronize(c_->stream), "sync");
-    scratch_gen_++;
-    dev_free(c_->s_ck_, c_->s_ck_n_);
-    c_->s_ck_ = nullptr;
-    c_->s_ck_n_ = 0;
+    if (rc != SVDB_ENOMEM || last) {
+      c_->cand_live = false;
+      return rc;
+    }
+    if (cap <= 8) {
+      pre = false;
+      HIPCHK(hipStreamSynchronize(c_->stream), "sync");
+      scratch_gen_++;
+      dev_free(c_->s_ck_, c_->s_ck_n_);
+      c_->s_ck_ = nullptr;
+      c_->s_ck_n_ = 0;
+    }
   }
+  const bool sorted = !pre;
+  const size_t LC = sorted ? kLowpLP : kLowpLC;  // entries of a list
   if (!c_->h_fail_) HIPCHK(hipHostMalloc((void**)&c_->h_fail_, sizeof(uint32_t)), "hipHostMalloc");
   const size_t io_b = (size_t)nq * sizeof(double);
   if (c_->h_io_n_ < io_b) {
@@ -1347,8 +1390,8 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
     LowpScanArgs ma = group_args(g);
     ma.rows_per_slice = ma.slice_stride = r.rps;
     ma.NL = r.NL;
-    ma.hdr = (uint2*)c_->s_ck_ + r.coff;
-    ma.ent = (uint2*)c_->s_cs_ + r.coff * kLowpLC;
+    ma.hdr = sorted ? nullptr : (uint2*)c_->s_ck_ + r.coff;
+    ma.ent = (uint2*)c_->s_cs_ + r.coff * LC;
     if (ma.tau0) ma.tau0 += g.soff;
     HIPCHK(scan(ma, g.metric, r.ns, false), "first-pass scan");
   }
@@ -1358,8 +1401,8 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // every range's shortlist, in as few launches as the kernels allow
   std::vector<ShortlistArgs> sls(nr);
   for (int i = 0; i < nr; i++)
-    sls[i] = ShortlistArgs{(const uint2*)c_->s_ck_ + R[i].coff,
-                           (const uint2*)c_->s_cs_ + R[i].coff * kLowpLC, R[i].n, R[i].NL, width(R[i].k),
+    sls[i] = ShortlistArgs{sorted ? nullptr : (const uint2*)c_->s_ck_ + R[i].coff,
+                           (const uint2*)c_->s_cs_ + R[i].coff * LC, R[i].n, R[i].NL, width(R[i].k),
                            (uint32_t*)c_->s_ss_ + (size_t)R[i].soff * L,
                            (float*)c_->s_sk_ + (size_t)R[i].soff * L, (float*)c_->s_beta_ + R[i].soff};
   prof_begin(SVDB_K_SHORTLIST);
@@ -1406,13 +1449,35 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   lp.ostride = ostride;
   lp.fp8 = fp8;
   lp.shortlist = shortlist;
+  lp.sorted = sorted;
+  lp.frugal = frugal;
   return SVDB_OK;
+}
+
+// Completes lowp_enqueue's search.  Where the retries find no device memory, the
+// candidate lists had taken too much of it: the search is done again with the
+// fewest and shortest.
+int Engine::lowp_complete() {
+  const SearchCtx::LowpPending lp = c_->lp;  // (a nested pass reuses c_->lp)
+  const EngineStats st = st_;
+  const bool quiet = quiet_;
+  quiet_ |= !lp.frugal;
+  int rc = lowp_retries();
+  quiet_ = quiet;
+  c_->cand_live = false;
+  if (rc != SVDB_ENOMEM || lp.frugal) return rc;
+  st_ = st;
+  (void)release_lists();
+  LowpRange R[3] = {lp.R[0], lp.R[1], lp.R[2]};
+  rc = lowp_enqueue(lp.dQ, lp.ldq, R, lp.nr, lp.k, lp.dids, lp.dscores, lp.ostride, lp.fp8, nullptr,
+                    true);
+  return rc ? rc : lowp_complete();
 }
 
 // Waits for lowp_enqueue's work and answers what the first pass could not
 // certify: the widening retries, the FP8 queries' BF16 second pass, and the
 // FP64 rescan.
-int Engine::lowp_complete() {
+int Engine::lowp_retries() {
   int rc;
   SearchCtx::LowpPending lp = c_->lp;  // a nested pass below reuses c_->lp
   c_->lp.on = false;
@@ -1477,8 +1542,8 @@ int Engine::lowp_complete() {
     const double* rQ = dQ + (size_t)rg.qoff * ldq;
     uint64_t* rids = dids + (size_t)rg.qoff * ostride;
     double* rsc = dscores + (size_t)rg.qoff * ostride;
-    const uint2* rhdr = (const uint2*)c_->s_ck_ + rg.coff;
-    const uint2* rent = (const uint2*)c_->s_cs_ + rg.coff * kLowpLC;
+    const uint2* rhdr = lp.sorted ? nullptr : (const uint2*)c_->s_ck_ + rg.coff;
+    const uint2* rent = (const uint2*)c_->s_cs_ + rg.coff * (lp.sorted ? kLowpLP : kLowpLC);
     const RerankArgs ra = rerank_args(ri);
     uint32_t* fail_list = ra.fail_list;  // may be redirected to a widening retry's list
     uint32_t nf = nf1;
@@ -1507,7 +1572,7 @@ int Engine::lowp_complete() {
     for (int wi = 0; wi < 2; wi++) {
       const uint32_t Lw = wi == 0 ? 1024u : (uint32_t)kMaxShort;
       if (nf == 0 || Lw <= L) continue;
-      if (rg.pass ? 2 * rg.pass < 3 * Lprev : (size_t)NL * kLowpLP < 2 * (size_t)Lw) continue;
+      if (!lp.sorted ? 2 * rg.pass < 3 * Lprev : (size_t)NL * kLowpLP < 2 * (size_t)Lw) continue;
       if (second_pass_cheaper(nf, Lw)) break;
       Lprev = Lw;
       // A retry that has lately certified almost none of its queries for
@@ -2031,7 +2096,6 @@ int Engine::search_begin_locked(SearchCtx& c, const double* Q, size_t nq, size_t
     rc = lowp_enqueue((const double*)c.s_q_, D, R, nr, (int)kmax_all, pid, psc,
                       (uint32_t)kmax_all, false, pq);
     if (rc) {
-      c.lp.on = false;
       (void)hipStreamSynchronize(c.stream);
       return rc;
     }

@@ -155,6 +155,7 @@ class Engine {
     size_t need;
   };
   int scratch_set(std::initializer_list<ScratchNeed> set, bool quiet);
+  bool release_lists();
   // pinned staging, grow-only; nullptr past its cap
   void* host_stage(void** buf, size_t* have, size_t bytes);
   int run_exact(const double* dQ, size_t ldq, uint32_t nq, uint32_t D, const int* dk, int metric,
@@ -226,7 +227,7 @@ class Engine {
   bool lowp_ = false;
   bool lowp_wanted_ = true;
   bool prepass_ = true;  // sample pre-pass before the first-pass scan (SVDB_PREPASS=0: off)
-  static constexpr uint32_t kPrepassSlices = 256;  // 64 on stores of under 16*256 tiles
+  static constexpr uint32_t kPrepassSlices = 256;  // at most; 16 or 64 on smaller stores
   static constexpr uint32_t kPrepassMaxTiles = 8;
   Shadow sh_;
   bool lowp8_ = false;  // FP8 shadow present (built on request)
@@ -234,6 +235,7 @@ class Engine {
 
   size_t dev_bytes_ = 0;
   size_t budget_ = SIZE_MAX;
+  bool quiet_ = false;  // a lack of device memory is no error yet (lowp_complete)
   size_t shortlist_ = 64;
 
   struct ProfSlot {
@@ -297,7 +299,12 @@ class Engine {
       uint32_t ostride = 0;
       bool fp8 = false;
       size_t shortlist = 0;
+      bool sorted = false;  // lists without a starting threshold
+      bool frugal = false;  // ... for lack of device memory
     } lp;
+    // the candidate lists (s_ck_, s_cs_), the partial lists (s_pk_, s_ps_) are
+    // in use beyond the launches already enqueued
+    bool cand_live = false, part_live = false;
     // an asynchronous search (search_begin): 0 idle, 1 enqueued, 2 completed
     int state = 0;
     int rc = 0;
@@ -328,8 +335,10 @@ class Engine {
   uint64_t* near_host_ = nullptr;   // pinned: its answer (id, seq)
   uint64_t near_seq_ = 0;
   int lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int k, uint64_t* dids,
-                   double* dscores, uint32_t ostride, bool fp8, const double* hQ = nullptr);
+                   double* dscores, uint32_t ostride, bool fp8, const double* hQ = nullptr,
+                   bool frugal = false);
   int lowp_complete();
+  int lowp_retries();
   int search_begin_locked(SearchCtx& c, const double* Q, size_t nq, size_t ldq, size_t D,
                           const size_t* k, const int* metric, int precision, size_t ostride,
                           size_t* ids, double* scores);

@@ -99,8 +99,11 @@ struct LowpScanArgs {
   uint32_t nrows_pad;       // rows readable in Xb / aux (multiple of kLowpTile)
   uint32_t NL;              // lists per query = slices * 4
   float* cand_key;          // [nq][NL] sample pre-pass: each list's smallest key
-  uint2* hdr;               // [nq][NL] {entries, fp32 bound on the rows left out}
-  uint2* ent;               // [nq][NL][kLowpLC] {fp32 ordering key, slot}
+  // Candidate lists (svdb_cand.h): with a threshold [nq][NL] headers {entries, fp32
+  // bound on the rows left out} and [nq][NL][kLowpLC] entries {fp32 ordering key,
+  // slot}; without one [nq][NL][kLowpLP] entries alone.
+  uint2* hdr;
+  uint2* ent;
   // Optional per-query starting threshold: query q's lists only take keys
   // below tau0[q * tau0_stride], the ordering key of an actual row (so that a
   // list which leaves nothing else out has it as its bound).
@@ -109,7 +112,7 @@ struct LowpScanArgs {
 };
 
 struct ShortlistArgs {
-  const uint2* hdr;
+  const uint2* hdr;         // null: sorted lists (LowpScanArgs)
   const uint2* ent;
   uint32_t nq, NL, L;
   uint32_t* short_slot;     // [nq][L]  (UINT32_MAX when fewer)

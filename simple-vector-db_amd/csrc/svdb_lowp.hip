@@ -383,8 +383,10 @@ __device__ __forceinline__ void shortlist_body(const ShortlistArgs& a, uint32_t 
                                                SelShared<T, CAP>& sm) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t q = a.qidx ? a.qidx[i] : i;  // candidate lists of query q -> output row i
-  const uint2* __restrict__ hdr = a.hdr + (size_t)q * a.NL;
-  const uint2* __restrict__ ent = a.ent + (size_t)q * a.NL * kLowpLC;
+  const bool sorted = !a.hdr;
+  const uint2* __restrict__ hdr = a.hdr + (sorted ? 0 : (size_t)q * a.NL);
+  const uint32_t LC = sorted ? kLowpLP : kLowpLC;
+  const uint2* __restrict__ ent = a.ent + (size_t)q * a.NL * LC;
   if (tid == 0) {
     sm.n = 0;
     sm.lt = 0;
@@ -395,20 +397,33 @@ __device__ __forceinline__ void shortlist_body(const ShortlistArgs& a, uint32_t 
   float bmin = INFINITY;
   uint32_t lo = ~0u, hi = 0u;
   for (uint32_t l = tid; l < a.NL; l += T) {
+    if (sorted) {
+      uint32_t m = 0;
+#pragma unroll
+      for (int e = 0; e < kLowpLP; e += 2) {
+        const uint4 v = *reinterpret_cast<const uint4*>(ent + (size_t)l * kLowpLP + e);
+        m += (v.y != ~0u) + (v.w != ~0u);
+        if (e == kLowpLP - 2) bmin = fminf(bmin, __uint_as_float(v.z));
+      }
+      sm.cnt[l] = (uint8_t)m;
+      continue;
+    }
     const uint2 h = hdr[l];
     sm.cnt[l] = (uint8_t)h.x;
     bmin = fminf(bmin, __uint_as_float(h.y));
   }
   __syncthreads();
   constexpr int U = 4;
-  const uint32_t quads = a.NL * (kLowpLC / 4);
+  const int qs = sorted ? 1 : 2;  // log2 of a list's groups of four entries
+  static_assert(kLowpLP == 8 && kLowpLC == 16, "qs");
+  const uint32_t quads = a.NL << qs;
   for (uint32_t t0 = 0; t0 < quads; t0 += U * T) {
     uint32_t m[U], sum = 0;
     uint4 v[U][2];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const uint32_t t = t0 + u * T + tid, e0 = (t & 3) * 4;
-      const uint32_t c = t < quads ? sm.cnt[t >> 2] : 0u;
+      const uint32_t t = t0 + u * T + tid, e0 = (t & ((1u << qs) - 1)) * 4;
+      const uint32_t c = t < quads ? sm.cnt[t >> qs] : 0u;
       m[u] = c > e0 ? min(4u, c - e0) : 0u;
       sum += m[u];
       if (m[u]) {
@@ -467,7 +482,7 @@ __device__ __forceinline__ void shortlist_body(const ShortlistArgs& a, uint32_t 
     for (uint32_t l = tid; l < a.NL; l += T) {
       const uint32_t m = sm.cnt[l];
       for (uint32_t e = 0; e < m; e++) {
-        const uint2 v = ent[(size_t)l * kLowpLC + e];
+        const uint2 v = ent[(size_t)l * LC + e];
         f(rank_bits32(__uint_as_float(v.x)), v.y);
       }
     }

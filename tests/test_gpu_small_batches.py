@@ -173,3 +173,88 @@ def test_candidate_lists_within_a_budget(nq):
     ids, sc = db.search(Q, 10, "l2", "bf16")
     assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
     db.close()
+
+
+def pages(*sizes):
+    return sum((max(int(b), 1) + 4095) // 4096 * 4096 for b in sizes)
+
+
+def first_pass_scratch(nq, k, dp, qpb, lists, L):
+    """Device scratch of a first pass whose lists hold 8 entries of 8 bytes, for
+    queries and results in device memory."""
+    pad = (nq + qpb - 1) // qpb * qpb
+    return pages((pad + qpb) * dp * 2, pad * 48, lists * 32, lists * 32, nq * L * 4, nq * L * 4,
+                 nq * 4, (nq + 3) * 4, nq * 8, nq * k * 8, nq * k * 4, nq * 4, nq * 4)
+
+
+@pytest.mark.parametrize("n,d,nq,k", [(4000, 64, 3000, 5), (4000, 250, 2000, 1),
+                                      (30_000, 60, 700, 10), (30_000, 128, 400, 100)])
+def test_lists_of_eight_entries_fit(n, d, nq, k):
+    """A device-memory budget that holds 8 slices' lists of eight entries, with
+    nothing besides, on stores with and without a sample's threshold."""
+    rng = np.random.default_rng(n + nq)
+    X = rng.standard_normal((n, d))
+    Q = rng.standard_normal((nq, d))
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    dQ = svdb.DeviceArray.from_host(Q)
+    ids = svdb.DeviceArray((nq, k), np.uint64)
+    sc = svdb.DeviceArray((nq, k), np.float64)
+    dp = 64 if d <= 64 else 128 if d <= 128 else 256
+    L = 64 if k <= 32 else 256
+    lists = nq * 4 * (128 if k > 32 else 8)
+    db.set_budget(db.stats()["device_bytes"] +
+                  first_pass_scratch(nq, k, dp, 512 if dp < 256 else 256, lists, L))
+    error = svdb.lib().svdb_last_error()
+    db.search_device(dQ.ptr, nq, d, k, "dot", "bf16", ids.ptr, sc.ptr)
+    rid, rsc = O.topk(X, Q, k, "dot")
+    assert np.array_equal(ids.to_host(), rid) and np.array_equal(sc.to_host(), rsc)
+    assert svdb.lib().svdb_last_error() == error  # the smaller plan's is no error
+    for a in (dQ, ids, sc):
+        a.free()
+    db.close()
+
+
+@pytest.mark.parametrize("n,nq", [(4000, 300), (40_007, 300), (40_007, 3000)])
+def test_fallback_within_a_budget(n, nq):
+    """A zero query, which only the FP64 scan can answer, in a batch under a budget
+    that holds lists of eight entries, the retries' buffers and that scan's: the
+    lists must not take what those need."""
+    rng = np.random.default_rng(n + nq)
+    d, k = 64, 10
+    X = rng.standard_normal((n, d))
+    Q = rng.standard_normal((nq, d))
+    Q[nq // 2] = 0.0
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    tiles = (n + 127) // 128
+    slices = min(512 // ((nq + 511) // 512) // 8 * 8, max(8, (tiles // 4 + 7) // 8 * 8))
+    retries = pages(1024 * 4, 1024 * 4, 4, 16, 4096 * 4, 4096 * 4)
+    exact = pages(d * 8, k * 8, k * 8, 4, 4 * max(8, n // 1024) * k * 8, 4 * max(8, n // 1024) * k * 4, 24)
+    db.set_budget(db.stats()["device_bytes"] + pages(nq * d * 8, nq * k * 8, nq * k * 8) +
+                  first_pass_scratch(nq, k, 64, 512, nq * 4 * slices, 64) + retries + exact)
+    error = svdb.lib().svdb_last_error()
+    for metric in ("l2", "dot"):
+        check(db, X, Q, k, metric, "bf16")
+        assert db.stats()["fallbacks"] > 0
+        assert svdb.lib().svdb_last_error() == error  # the smaller plan's is no error
+    db.close()
+
+
+def test_lists_make_room_for_rows():
+    """What searches leave behind in device memory does not stand in the way of
+    rows or of another kind of search."""
+    rng = np.random.default_rng(5)
+    X = rng.standard_normal((20_000, 32))
+    Q = rng.standard_normal((4000, 32))
+    db = svdb.Database(kd_dimension=1)
+    db.bulk_insert(X)
+    db.search(Q, 10, "l2", "bf16")
+    db.search(Q, 10, "l2", "fp64")
+    db.set_budget(db.stats()["device_bytes"] + (1 << 20))
+    db.bulk_insert(rng.standard_normal((15_000, 32)))  # the store doubles
+    db.set_budget(0)
+    ids, sc = db.search(Q[:50], 10, "l2", "bf16")
+    rid, rsc = db.search(Q[:50], 10, "l2", "fp64")
+    assert np.array_equal(ids, rid) and np.array_equal(sc, rsc)
+    db.close()
