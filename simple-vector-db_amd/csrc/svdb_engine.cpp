@@ -1283,7 +1283,10 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   for (uint32_t cap = 512;; cap = cap > 8 ? cap / 2 : 512) {
     plan(cap);
     const bool last = cap <= 8 && !pre;
-    rc = pre ? scratch_set({{&c_->s_ck_, &c_->s_ck_n_,
+    rc = !last && nlists * (pre ? sizeof(uint2) * (1 + kLowpLC) : sizeof(uint2) * kLowpLP) >
+                      c_->list_room
+             ? SVDB_ENOMEM
+         : pre ? scratch_set({{&c_->s_ck_, &c_->s_ck_n_,
                              std::max(nlists * sizeof(uint2), (size_t)nq * NL_pre * sizeof(float))},
                             {&c_->s_cs_, &c_->s_cs_n_, nlists * kLowpLC * sizeof(uint2)}}, true)
              : scratch_set({{&c_->s_cs_, &c_->s_cs_n_, nlists * kLowpLP * sizeof(uint2)}}, !last);
@@ -1873,13 +1876,14 @@ int Engine::search_host(const double* Q, size_t nq, size_t ldq, size_t D, const 
 
 int Engine::search_begin(int slot, const double* Q, size_t nq, size_t ldq, size_t D,
                          const size_t* k, const int* metric, int precision, size_t ostride,
-                         size_t* ids, double* scores) {
+                         size_t* ids, double* scores, size_t list_room) {
   std::lock_guard<std::mutex> g(mu_);
   if (slot < 1 || slot >= kCtx || ctx_[slot].state != 0) {
     set_error(SVDB_EINVAL, "search slot busy or out of range");
     return SVDB_EINVAL;
   }
   SearchCtx& c = ctx_[slot];
+  c.list_room = list_room;
   int rc = search_begin_locked(c, Q, nq, ldq, D, k, metric, precision, ostride, ids, scores);
   if (rc != SVDB_OK) c.state = 0;
   c_ = &ctx_[0];

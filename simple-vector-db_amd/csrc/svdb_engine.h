@@ -107,10 +107,12 @@ class Engine {
   // search on context `slot` (1 or 2) and returns; end completes it (waits,
   // runs any retries) and writes ids / scores, which must stay valid from
   // begin to end.  Two searches may be in flight at once; a store mutation
-  // completes them first.
+  // completes them first.  list_room: bytes that the first pass's candidate
+  // lists may take; kListBytes a query always do.
+  static constexpr size_t kListBytes = (size_t)128 << 10;
   int search_begin(int slot, const double* Q, size_t nq, size_t ldq, size_t D, const size_t* k,
                    const int* metric, int precision, size_t ostride, size_t* ids,
-                   double* scores);
+                   double* scores, size_t list_room);
   int search_end(int slot);
   // Device queries and outputs; one k and metric.
   int search_device(const double* dQ, size_t nq, size_t ldq, size_t D, size_t k, int metric,
@@ -305,6 +307,7 @@ class Engine {
     // the candidate lists (s_ck_, s_cs_), the partial lists (s_pk_, s_ps_) are
     // in use beyond the launches already enqueued
     bool cand_live = false, part_live = false;
+    size_t list_room = SIZE_MAX;  // bytes for the candidate lists (search_begin)
     // an asynchronous search (search_begin): 0 idle, 1 enqueued, 2 completed
     int state = 0;
     int rc = 0;

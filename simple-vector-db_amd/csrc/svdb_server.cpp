@@ -151,9 +151,9 @@ class Server {
 
   size_t query_bytes(size_t nq, size_t k) const {
     // FP64 query + BF16 query + parameters + results + first-pass candidate
-    // lists (at most 512 slices × 4 lists × 8 entries of 8 bytes)
+    // lists (which take more than that only where the tick's budget has room)
     const size_t d = eng_->dim() ? eng_->dim() : 1;
-    return nq * (d * 8 + d * 2 + 64 + k * 16 + 512 * 4 * 8 * 8);
+    return nq * (d * 8 + d * 2 + 64 + k * 16 + Engine::kListBytes);
   }
 
   const svdb_server_config& cfg() const { return cfg_; }
@@ -355,7 +355,8 @@ class Server {
         f->sc.resize(t->nq * t->kmax);
         f->rc = eng_->search_begin(f->slot, t->q.data(), t->nq, d, d, t->k.data(),
                                    t->metric.data(), cfg_.precision, t->kmax, f->ids.data(),
-                                   f->sc.data());
+                                   f->sc.data(),
+                                   cfg_.budget_bytes - t->bytes + t->nq * Engine::kListBytes);
       } catch (const std::bad_alloc&) {
         f->rc = SVDB_ENOMEM;
       } catch (...) {

@@ -295,3 +295,27 @@ def test_serving_mix_on_the_fp64_scan_store():
             model = np.delete(model, p[1], axis=0)
     assert checked >= 100
     assert stats["certified"] > 0
+
+
+@pytest.mark.parametrize("nq", [64, 100])
+def test_a_tick_stays_within_its_memory(nq):
+    """A budget that just admits a request: the device memory its search takes is
+    within a tenth of it."""
+    d, k = 32, 10
+    rng = np.random.default_rng(nq)
+    rows = rng.standard_normal((200_000, d))
+    db = svdb.Database(kd_dimension=3)
+    db.bulk_insert(rows)
+    budget = nq * (d * 8 + d * 2 + 64 + k * 16 + (128 << 10))
+    srv = svdb.Server(db, budget_bytes=budget)
+    with pytest.raises(svdb.SvdbError):
+        srv.submit_search(rows[:nq + 1], k, "l2")  # one query more than fits
+    b0 = db.stats()["device_bytes"]
+    Q = rng.standard_normal((nq, d))
+    for metric in ("l2", "cos", "dot"):
+        rc, ids, sc, _ = srv.wait(srv.submit_search(Q, k, metric))
+        rid, rsc = O.topk(rows, Q, k, metric)
+        assert rc == 0 and np.array_equal(ids, rid) and np.array_equal(sc, rsc)
+    assert db.stats()["device_bytes"] - b0 <= 1.1 * budget
+    srv.stop()
+    db.close()
