@@ -386,11 +386,19 @@ __global__ __launch_bounds__(512, (KS <= 2 ? QF <= 2 : KS == 4 && QF == 1) ? 4 :
   }
 }
 
+// Sorted lists of 256-wide rows: one fragment per wavefront for any number of
+// queries.  Two fragments' query rows and lists are more than the registers hold
+// beside the MFMAs (cosine spilled 27): 20k rows, k = 100, scans of 300 queries
+// cosine 148 → 63 µs, Euclidean 124 → 64, of 4,000 265 → 214 and 215 → 211.  The
+// mixed scan's are the same with either (250 queries 191).
+constexpr bool sorted_takes_one(int metric, int ks) { return ks == 8 && metric != kMixed; }
+
 template <int METRIC, int KS, int QF>
 static hipError_t scan_bf16_t(const LowpScanArgs& a, uint32_t nslices, bool minonly,
                               hipStream_t s) {
-  auto fn = a.tau0 ? k_scan_bf16<METRIC, KS, QF, kFormAppend>
-                   : k_scan_bf16<METRIC, KS, QF, kFormSorted>;
+  auto fn = k_scan_bf16<METRIC, KS, QF, kFormAppend>;
+  if constexpr (!sorted_takes_one(METRIC, KS) || QF == 1)
+    if (!a.tau0) fn = k_scan_bf16<METRIC, KS, QF, kFormSorted>;
   if (minonly) fn = k_scan_bf16<METRIC, KS, QF, kFormMin>;
   constexpr size_t shm = 0;  // both tile buffers are static LDS
   const uint32_t qpb = kLowpWaves * QF * 16;
@@ -404,12 +412,15 @@ static hipError_t scan_bf16_t(const LowpScanArgs& a, uint32_t nslices, bool mino
 template <int METRIC>
 static hipError_t scan_bf16_m(const LowpScanArgs& a, uint32_t nslices, bool minonly,
                               hipStream_t s) {
-  if (lowp_scan_queries(a.dp, a.nq) == kLowpWaves * 16) switch (a.dp / 32) {
-    case 1: return scan_bf16_t<METRIC, 1, 1>(a, nslices, minonly, s);
-    case 2: return scan_bf16_t<METRIC, 2, 1>(a, nslices, minonly, s);
-    case 4: return scan_bf16_t<METRIC, 4, 1>(a, nslices, minonly, s);
-    case 8: return scan_bf16_t<METRIC, 8, 1>(a, nslices, minonly, s);
-  }
+  const bool sorted = !minonly && !a.tau0;
+  if (lowp_scan_queries(a.dp, a.nq) == kLowpWaves * 16 ||
+      (sorted && sorted_takes_one(METRIC, (int)a.dp / 32)))
+    switch (a.dp / 32) {
+      case 1: return scan_bf16_t<METRIC, 1, 1>(a, nslices, minonly, s);
+      case 2: return scan_bf16_t<METRIC, 2, 1>(a, nslices, minonly, s);
+      case 4: return scan_bf16_t<METRIC, 4, 1>(a, nslices, minonly, s);
+      case 8: return scan_bf16_t<METRIC, 8, 1>(a, nslices, minonly, s);
+    }
   switch (a.dp / 32) {
     case 1: return scan_bf16_t<METRIC, 1, 2>(a, nslices, minonly, s);
     case 2: return scan_bf16_t<METRIC, 2, 2>(a, nslices, minonly, s);
