@@ -133,10 +133,13 @@ __device__ __forceinline__ void cand_append4(uint2* ent, CandPending& p, uint32_
 __device__ __forceinline__ void cand_store_sorted(const LowpScanArgs& a, size_t list,
                                                   const float (&lk)[kLowpLP],
                                                   const uint32_t (&ls)[kLowpLP]) {
-  uint4* e = reinterpret_cast<uint4*>(a.ent + list * kLowpLP);
+  // (a branch an entry: with plain stores the compiler keeps the lists elsewhere
+  // during the scan; FP8, 31k × 768, 1,848 cosine queries: 432 µs, 409 so)
+  uint2* e = a.ent + list * kLowpLP;
 #pragma unroll
-  for (int j = 0; j < kLowpLP; j += 2)
-    e[j / 2] = make_uint4(__float_as_uint(lk[j]), ls[j], __float_as_uint(lk[j + 1]), ls[j + 1]);
+  for (int j = 0; j < kLowpLP; j++)
+    if (ls[j] != ~0u) e[j] = make_uint2(__float_as_uint(lk[j]), ls[j]);
+    else e[j] = make_uint2(__float_as_uint(lk[kLowpLP - 1]), ~0u);
 }
 
 }  // namespace svdb
