@@ -1172,9 +1172,9 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // Row slices for a scan of n queries wanting kk neighbours: at
   // least 8, more when there are few query blocks, without a threshold each at
   // least 4 tiles long (with one a slice of a single tile is as good: 60k ×
-  // 1,536, 32 queries, scan 66 µs in 96 slices, 38 in 240).  One block per CU fits at a time, so the grid is kept at or just
-  // under two rounds of the 256 CUs (a few blocks past a round cost a whole
-  // round).  With a threshold, enough that the rows it lets pass fill a list
+  // 1,536, 32 queries, scan 66 µs in 96 slices, 38 in 240).  One block per CU
+  // fits at a time, so the grid is kept at or just under two rounds of the 256
+  // CUs (a few blocks past a round cost a whole round).  With a threshold, enough that the rows it lets pass fill a list
   // to half on average, for FP8, whose retries certify by the threshold itself,
   // to a quarter (a full list's bound becomes its largest key, which may then
   // lie below the shortlist's; 5M × 768 FP8, 4,096 cosine queries, k = 100: the
@@ -1200,7 +1200,8 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
       ns = std::max<uint32_t>(ns, r.pass / (kLowpLC / (fp8 ? 4 : 2) * kLowpLanesPerQuery));
     else if (fp8) ns = std::max<uint32_t>(ns, 512);
     else if (kk > 32) ns = std::max<uint32_t>(ns, 128);
-    // (a query's lists stay within 128 KiB, 960 lists of 17 words, or 272 KiB)
+    // (a query's lists stay within 272 KiB: 2,048 of 136 bytes with a threshold,
+    // 960 of those in large batches; without one 2,048 of 64 bytes)
     ns = std::min<uint32_t>(ns, pre ? nsmax : 512);
     ns = std::max<uint32_t>(1, std::min<uint32_t>(ns, std::max<uint32_t>(1, pre ? tiles : tiles / 4)));
     // With a threshold more slices cost little, and fill the last round: a

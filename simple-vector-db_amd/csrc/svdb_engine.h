@@ -229,7 +229,7 @@ class Engine {
   bool lowp_ = false;
   bool lowp_wanted_ = true;
   bool prepass_ = true;  // sample pre-pass before the first-pass scan (SVDB_PREPASS=0: off)
-  static constexpr uint32_t kPrepassSlices = 256;  // at most; 16 or 64 on smaller stores
+  static constexpr uint32_t kPrepassSlices = 256;  // at most; from 16 up on smaller stores
   static constexpr uint32_t kPrepassMaxTiles = 8;
   Shadow sh_;
   bool lowp8_ = false;  // FP8 shadow present (built on request)

@@ -26,7 +26,6 @@ inline uint32_t f64_slice_rows(uint32_t nrows, uint32_t P) {
 constexpr uint32_t kF64Share = 16;
 inline uint32_t f64_share(uint32_t D) { return kF64Share * ((D + 127) / 128); }
 
-
 // The sample's runs of row steps, 16 minima each, or 0 where there would be less
 // than twice k of them: one run per 1,024 rows up to 64, on small stores up to a
 // quarter of the rows for enough minima.

@@ -215,7 +215,7 @@ hipError_t launch_quantize_rows8(const Shadow8& sh, const double* X, size_t ldx,
                                  uint32_t n, uint32_t d, hipStream_t s);
 hipError_t launch_kill_rows8(const Shadow8& sh, const uint32_t* slots, uint32_t n, hipStream_t s);
 // Q8: e4m3 queries [nq_pad][dp]; QParams as for BF16 with P / scale carrying
-// the query's power-of-two scale (see svdb_fp8.hip).
+// the query's power-of-two scale (see svdb_wide.hip).
 hipError_t launch_query_prep8(const QueryPrepArgs& a, hipStream_t s);
 // a.Xb / a.Qb point at e4m3 bytes; a.w0 / a.w1: L2 (nx, sx), dot (xn, sx),
 // cosine (inv, pen).

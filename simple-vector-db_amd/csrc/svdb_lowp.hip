@@ -7,6 +7,7 @@
 
 #include "svdb_bins.h"
 #include "svdb_prep.h"
+#include "svdb_rank.h"
 
 namespace svdb {
 
@@ -29,32 +30,10 @@ __device__ __forceinline__ double bf16_val(uint16_t b) {
   return (double)__uint_as_float((uint32_t)b << 16);
 }
 
-__device__ __forceinline__ uint64_t rank_bits64(double v) {
-  v = v + 0.0;
-  uint64_t u = (uint64_t)__double_as_longlong(v);
-  if (v != v) u = 0x7FF8000000000000ull;
-  return (u >> 63) ? ~u : (u | 0x8000000000000000ull);
-}
-
-__device__ __forceinline__ double rank_val64(uint64_t u) {
-  uint64_t b = (u >> 63) ? (u & 0x7FFFFFFFFFFFFFFFull) : ~u;
-  return __longlong_as_double((long long)b);
-}
-
 __device__ __forceinline__ uint32_t rank_bits32(float v) {
   uint32_t u = __float_as_uint(v + 0.0f);
   if (v != v) u = 0x7FC00000u;
   return (u >> 31) ? ~u : (u | 0x80000000u);
-}
-
-__device__ __forceinline__ bool lt2(uint64_t ka, uint32_t sa, uint64_t kb, uint32_t sb) {
-  return (ka < kb) | ((ka == kb) & (sa < sb));
-}
-
-__device__ __forceinline__ uint64_t uni64(uint64_t v) {
-  uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-  uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return ((uint64_t)hi << 32) | lo;
 }
 
 __device__ __forceinline__ uint32_t uni32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -87,7 +66,7 @@ struct WL {
   __device__ __forceinline__ void insert(uint64_t K, uint32_t S, int kk, int lane) {
     int pos = 0;
 #pragma unroll
-    for (int p = 0; p < KPL; p++) pos += __popcll(__ballot(lt2(k[p], s[p], K, S)));
+    for (int p = 0; p < KPL; p++) pos += __popcll(__ballot(lex_lt(k[p], s[p], K, S)));
     if (pos >= kk) return;
     uint64_t pk[KPL];
     uint32_t ps[KPL];
@@ -817,9 +796,9 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a, uint32_t blk, d
       double v = acc;
       if (METRIC == kDot) v = -acc;
       else if (METRIC == kCos) v = -(acc / (qp.qn * a.st.xn[slot]));
-      K = rank_bits64(v);
+      K = rank_bits(v);
     }
-    uint64_t m = __ballot(valid && lt2(K, slot, tk, ts));
+    uint64_t m = __ballot(valid && lex_lt(K, slot, tk, ts));
     while (m) {
       int src = __ffsll((long long)m) - 1;
       m &= m - 1;
@@ -830,7 +809,7 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a, uint32_t blk, d
       L.insert(uni64(__shfl(K, src)), S, kk, lane);
       // lanes that no longer beat the (moved) k-th entry drop out
       L.at(kk - 1, tk, ts);
-      m &= __ballot(lt2(K, slot, tk, ts));
+      m &= __ballot(lex_lt(K, slot, tk, ts));
     }
     L.at(kk - 1, tk, ts);
   };
@@ -855,7 +834,7 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a, uint32_t blk, d
       // Prune threshold: the list's k-th value once full (+inf: fetch every
       // candidate).  A row whose lower bound exceeds it cannot be in the
       // top k.  (A NaN bound compares false and keeps its row.)
-      const double thr = (prune && ts != ~0u) ? rank_val64(tk) : INFINITY;
+      const double thr = (prune && ts != ~0u) ? rank_value(tk) : INFINITY;
       if (valid && j < a.L && thr < INFINITY && lower(key) > thr) valid = false;
       // a degenerate row that is also shortlisted must not enter twice
       if (valid && j >= a.L) {
@@ -882,7 +861,7 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a, uint32_t blk, d
   // certification
   // more degenerate rows than the list holds: nothing can be certified
   bool cert = false;
-  const double tau = ts == ~0u ? INFINITY : rank_val64(tk);
+  const double tau = ts == ~0u ? INFINITY : rank_value(tk);
   if (!qp.flags && *a.degen_count <= (uint32_t)kDegenCap) cert = tau < lower(a.beta[i]);
   if (!cert) {
     if (a.lk) {
@@ -936,7 +915,7 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a, uint32_t blk, d
       double sc = __longlong_as_double(0x7FF8000000000000ll);
       const uint32_t slot = L.s[p];
       if (slot != ~0u) {
-        const double v = rank_val64(L.k[p]);
+        const double v = rank_value(L.k[p]);
         if (v == v) sc = METRIC == kL2 ? sqrt(v) : (v == 0.0 ? 0.0 : -v);
         id = a.st.has_deletes
                  ? (uint64_t)a.st.rank_base[slot >> 6] +
@@ -1075,7 +1054,7 @@ __device__ __forceinline__ void rr_score(const RerankArgs& a, const QParams& qp,
     double r = acc;
     if (metric == kDot) r = -acc;
     else if (metric == kCos) r = -(acc / (qp.qn * a.st.xn[sm.oslot[c]]));
-    sm.k64[c] = rank_bits64(r);
+    sm.k64[c] = rank_bits(r);
   }
 }
 
@@ -1167,7 +1146,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const uint64_t K = sm.k64[j];
     const uint32_t S = sm.oslot[j];
     uint32_t r = 0;
-    for (uint32_t t = 0; t < m; t++) r += lt2(sm.k64[t], sm.oslot[t], K, S);
+    for (uint32_t t = 0; t < m; t++) r += lex_lt(sm.k64[t], sm.oslot[t], K, S);
     return r;
   };
   score(0, m1);
@@ -1179,7 +1158,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     __syncthreads();
     // A row whose lower bound exceeds the k-th value cannot be in the top k
     // (a flagged query's keys carry no bound; a NaN bound keeps its row).
-    const double thr = !qp.flags && sm.tau != ~0ull ? rank_val64(sm.tau) : INFINITY;
+    const double thr = !qp.flags && sm.tau != ~0ull ? rank_value(sm.tau) : INFINITY;
     int mine = 0;
     for (uint32_t j = m1 + tid; j < n; j += 256) mine = !(lower(sm.okey[j]) > thr) ? (int)j + 1 : mine;
     if (mine) atomicMax(&sm.n2, mine);
@@ -1202,7 +1181,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
   // certification (more degenerate rows than the list holds: nothing can be
   // certified)
-  const double tau = sm.tau == ~0ull ? INFINITY : rank_val64(sm.tau);
+  const double tau = sm.tau == ~0ull ? INFINITY : rank_value(sm.tau);
   const bool cert =
       !qp.flags && ndeg_all <= (uint32_t)kDegenCap && tau < lower(a.beta[q]);
   if (!cert) {
@@ -1231,7 +1210,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   for (int p = 0; p < 2; p++) {
     if (rk[p] >= kk) continue;
     const uint32_t j = tid + 256 * p, slot = sm.oslot[j];
-    const double v = rank_val64(sm.k64[j]);
+    const double v = rank_value(sm.k64[j]);
     double sc = __longlong_as_double(0x7FF8000000000000ll);
     if (v == v) sc = metric == kL2 ? sqrt(v) : (v == 0.0 ? 0.0 : -v);
     const uint64_t id =

@@ -3,7 +3,7 @@
 // For callers that must not allocate (code under HIP graph capture, tight
 // serving loops, harnesses that forbid hipMalloc): the FP64 exact top-k of
 // svdb_search_device with every intermediate — k per query, query norms and
-// the partial top-k lists of the row slices — in `scratch`, a file-scope
+// the row slices' lists and their counts — in `scratch`, a file-scope
 // device array of kNoAllocScratchBytes that each GPU holds for the life of
 // the process.  The caller passes queries and outputs in device memory.
 //
@@ -11,9 +11,9 @@
 // the device address is taken once per device with hipGetSymbolAddress
 // (with that device current) and only that address is used.  Calls are
 // serialised by a process-wide lock (they share the array); the array keeps
-// the last call's contents, and nothing in it has to start at zero (every
-// partial-list entry the merge reads is written by the scan of the same
-// call).
+// the last call's contents, and nothing in it has to start at zero (the
+// counts and every entry the selection reads are written by the scan of the
+// same call).
 #include <hip/hip_runtime.h>
 
 #include <mutex>

@@ -1,4 +1,4 @@
-// svdb_rank.h — FP64 rank keys and slots (internal, device code).
+// svdb_rank.h — FP64 rank keys, their order, and slots (internal, device code).
 #pragma once
 
 #include "svdb_kernels.h"
@@ -21,6 +21,13 @@ __device__ __forceinline__ double rank_value(uint64_t u) {
 
 __device__ __forceinline__ bool lex_lt(uint64_t ka, uint32_t sa, uint64_t kb, uint32_t sb) {
   return (ka < kb) | ((ka == kb) & (sa < sb));
+}
+
+// A wavefront's common value, in scalar registers.
+__device__ __forceinline__ uint64_t uni64(uint64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return ((uint64_t)hi << 32) | lo;
 }
 
 __device__ __forceinline__ bool slot_alive(const uint64_t* alive, uint32_t r) {

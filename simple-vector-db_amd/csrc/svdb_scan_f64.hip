@@ -44,13 +44,13 @@
 // enters when its key is at most the query's global bound gtk — the smallest
 // k-th key any of its lists has reached, atomic min — and ranks before the
 // list's own k-th.  A list that cannot take a row is cut to its k best
-// (compact), which gives it that k-th and lowers gtk, and the row is tried again.  A test per
-// (query, row) is one comparison of doubles; all else happens in branches that
-// a row step seldom takes.  (Sorted lists spread over a wavefront's registers
+// (f64_compact), which gives it that k-th and lowers gtk, and the row is tried
+// again.  A test per (query, row) is one comparison of doubles; all else happens
+// in branches that a row step seldom takes.  (Sorted lists spread over a wavefront's registers
 // had taken 48 of them at k <= 64 and 96 above, and every insertion a chain of
-// lane shuffles.  500k × 128, 1,024 queries, dot, k = 10: 3.54 → 2.58 ms for the
-// call, 37 → 51 TF/s; 300k × 100, 77 queries, Euclidean, k = 100, on the VALU
-// before: 3.74 → 0.35 ms; 1M × 128, 16 queries, dot, k = 100: 3.59 → 0.36 ms.)
+// lane shuffles.  500k × 128, 1,024 queries, dot, k = 10: 3.54 → 2.53 ms for the
+// call, 37 → 52 TF/s; 300k × 100, 77 queries, Euclidean, k = 100, on the VALU
+// before: 3.74 → 0.32 ms; 1M × 128, 16 queries, dot, k = 100: 3.59 → 0.36 ms.)
 #include <math.h>
 
 #include <algorithm>
@@ -65,12 +65,6 @@ namespace svdb {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
-
-__device__ __forceinline__ uint64_t uni64(uint64_t v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return ((uint64_t)hi << 32) | lo;
-}
 
 // Hides a lane's value at the end of a loop over whole wavefronts: where the
 // compiler sees what a lane that has nothing left does in the next turn, it may
