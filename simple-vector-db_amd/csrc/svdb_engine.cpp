@@ -1174,15 +1174,15 @@ int Engine::lowp_enqueue(const double* dQ, size_t ldq, LowpRange* R, int nr, int
   // least 4 tiles long (with one a slice of a single tile is as good: 60k ×
   // 1,536, 32 queries, scan 66 µs in 96 slices, 38 in 240).  One block per CU
   // fits at a time, so the grid is kept at or just under two rounds of the 256
-  // CUs (a few blocks past a round cost a whole round).  With a threshold, enough that the rows it lets pass fill a list
-  // to half on average, for FP8, whose retries certify by the threshold itself,
-  // to a quarter (a full list's bound becomes its largest key, which may then
-  // lie below the shortlist's; 5M × 768 FP8, 4,096 cosine queries, k = 100: the
-  // retries certify 832 with lists half full, 1,679 so, 63.0 → 54.8 ms);
-  // without one, past k = 32 at least
-  // 512 lists per query and for FP8 2,048, which keep the lists' own bound
-  // (the smallest 8th entry) clear of the k-th neighbour and of the retries'
-  // 4,096th candidate.
+  // CUs (a few blocks past a round cost a whole round).  With a threshold,
+  // enough that the rows it lets pass fill a list to half on average, for
+  // FP8, whose retries certify by the threshold itself, to a quarter (a full
+  // list's bound becomes its largest key, which may then lie below the
+  // shortlist's; 5M × 768 FP8, 4,096 cosine queries, k = 100: the retries
+  // certify 832 with lists half full, 1,679 so, 63.0 → 54.8 ms); without one,
+  // past k = 32 at least 512 lists per query and for FP8 2,048, which keep
+  // the lists' own bound (the smallest 8th entry) clear of the k-th neighbour
+  // and of the retries' 4,096th candidate.
   auto slicing = [&](uint32_t n, int kk, uint32_t cap, LowpRange& r) {
     const uint32_t sq = fp8 ? qpb : (uint32_t)lowp_scan_queries(dp, n);
     const uint32_t grp = (n + sq - 1) / sq;
